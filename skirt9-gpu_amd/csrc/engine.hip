@@ -18,6 +18,7 @@
 #include <memory>
 #include <mutex>
 #include <string>
+#include <unordered_map>
 #include <vector>
 
 #include "../../include/skirt_mi355x.h"
@@ -35,16 +36,18 @@ namespace skg
     template<int GT> __global__ void trace_count(GridView g, const double* __restrict__ rays, int64_t n, int64_t* counts)
     {
         int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
-        stage_top(g);
+        stage_planes<GT>(g);
         if (t >= n) return;
-        const double* r = rays + 6 * t;
+        const double* ray = rays + 6 * t;
         Gen<GT> gen;
-        gen.start(r[0], r[1], r[2], r[3], r[4], r[5]);
+        gen.start(ray[0], ray[1], ray[2], ray[3], ray[4], ray[5]);
         int m;
         double ds, nd;
         int64_t c = 0, cs = 0;
-        while (gen.next(g, m, ds, nd))
+        for (int r = 0; r == 0 || r == 1;)
         {
+            r = gen.advance(g, m, ds, nd);
+            if (r <= 0) continue;
             ++c;
             if (ds > 0.) ++cs;
         }
@@ -57,16 +60,18 @@ namespace skg
                                 double* dso)
     {
         int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
-        stage_top(g);
+        stage_planes<GT>(g);
         if (t >= n) return;
-        const double* r = rays + 6 * t;
+        const double* ray = rays + 6 * t;
         Gen<GT> gen;
-        gen.start(r[0], r[1], r[2], r[3], r[4], r[5]);
+        gen.start(ray[0], ray[1], ray[2], ray[3], ray[4], ray[5]);
         int m;
         double ds, nd;
         int64_t o = off[t];
-        while (gen.next(g, m, ds, nd))
+        for (int r = 0; r == 0 || r == 1;)
         {
+            r = gen.advance(g, m, ds, nd);
+            if (r <= 0) continue;
             mo[o] = m;
             dso[o] = ds;
             ++o;
@@ -84,16 +89,20 @@ namespace skg
     template<int GT> __global__ void trace_count_off(GridView g, const double* __restrict__ rays, int64_t n, int64_t* off)
     {
         int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
-        stage_top(g);
+        stage_planes<GT>(g);
         if (t == 0) off[0] = 0;
         if (t >= n) return;
-        const double* r = rays + 6 * t;
+        const double* ray = rays + 6 * t;
         Gen<GT> gen;
-        gen.start(r[0], r[1], r[2], r[3], r[4], r[5]);
+        gen.start(ray[0], ray[1], ray[2], ray[3], ray[4], ray[5]);
         int m;
         double ds, nd;
         int64_t c = 0;
-        while (gen.next(g, m, ds, nd)) ++c;
+        for (int r = 0; r == 0 || r == 1;)
+        {
+            r = gen.advance(g, m, ds, nd);
+            if (r > 0) ++c;
+        }
         off[t + 1] = c;
     }
 
@@ -170,7 +179,16 @@ namespace skg
         }
     }
 
-    // copies the cell densities into the cell records (octree leaves, Voronoi cells, tetrahedra)
+    // copies the cell densities into the leaves' node records
+    __global__ void fill_node_density(OctNode* node, const double* dens, int64_t n)
+    {
+        int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
+        if (i >= n) return;
+        const int c = node[i].cell;
+        if (c >= 0) node[i].dens = dens[c];
+    }
+
+    // and into the cell records (Voronoi cells, tetrahedra)
     template<typename Rec> __global__ void fill_record_density(Rec* rec, const double* dens, int64_t n)
     {
         int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
@@ -190,23 +208,24 @@ namespace skg
                               double* tau_path, double* tau_obs, const int64_t* toff, double* tau_cum)
     {
         int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
-        stage_top(g);
+        stage_planes<GT>(g);
         if (t >= n) return;
-        const double* r = rays + 6 * t;
+        const double* ray = rays + 6 * t;
         Gen<GT> gen;
         int m;
         double ds, nd;
         // complete path, cumulative tau over stored (ds > 0) segments
-        gen.start(r[0], r[1], r[2], r[3], r[4], r[5]);
+        gen.start(ray[0], ray[1], ray[2], ray[3], ray[4], ray[5]);
         double tau = 0.;
         Kahan32 k32;
         k32.reset();
         const float s32 = static_cast<float>(section);
         int64_t o = toff ? toff[t] : 0;
         const int64_t oend = toff ? toff[t + 1] : 0;
-        while (gen.next(g, m, ds, nd))
+        for (int r = 0; r == 0 || r == 1;)
         {
-            if (ds > 0.)
+            r = gen.advance(g, m, ds, nd);
+            if (r > 0 && ds > 0.)
             {
                 if (m >= 0)
                 {
@@ -220,14 +239,15 @@ namespace skg
         }
         tau_path[t] = (FP == SKG_FP64) ? tau : static_cast<double>(k32.sum);
         // observer optical depth with early-out (every segment from next() counts)
-        gen.start(r[0], r[1], r[2], r[3], r[4], r[5]);
+        gen.start(ray[0], ray[1], ray[2], ray[3], ray[4], ray[5]);
         tau = 0.;
         k32.reset();
         double res = 0.;
         bool inf = false;
-        while (gen.next(g, m, ds, nd))
+        for (int r = 0; r == 0 || r == 1;)
         {
-            if (m >= 0)
+            r = gen.advance(g, m, ds, nd);
+            if (r > 0 && m >= 0)
             {
                 if (FP == SKG_FP64)
                 {
@@ -256,16 +276,19 @@ namespace skg
     // ------------------------------------------------------------------ cell densities
     constexpr uint32_t kTagDensity = 0x44454e53u;  // the host samplers' stream tag for cell densities
 
-    // Cell-averaged number density of the disk model in every cell of the resident grid from
+    // Cell-averaged number density of the disk model in every cell of the resident grid (one thread
+    // per cell, for the octree per node) from
     // n random points per cell, drawn from the same Philox stream (seed, cell, tag) and placed
     // the same way as the host samplers do (uniform in the Cartesian / octree cell box, x then
     // y then z; folded barycentric weights in a tetra), as MediumSystem's PropertySampler
     // (MediumSystem.cpp:129-155) averages a medium over random positions in each cell.
     template<int GT>
-    __global__ void sample_density_kernel(GridView g, DiskModel md, int n, uint64_t seed, int64_t ncells, double* out)
+    __global__ void sample_density_kernel(GridView g, DiskModel md, int n, uint64_t seed, int64_t count, double* out)
     {
-        const int64_t m = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-        if (m >= ncells) return;
+        const int64_t at = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+        if (at >= count) return;
+        const int64_t m = GT == kOctree ? g.node[at].cell : at;
+        if (m < 0) return;  // an inner node
         Philox rng;
         rng.init(seed, static_cast<uint64_t>(m), kTagDensity);
         double sum = 0.;
@@ -315,11 +338,11 @@ namespace skg
         }
         else
         {
-            const OctLeaf& L = g.leaf[m];
+            const OctNode& L = g.node[at];
             for (int a = 0; a < 3; ++a)
             {
-                b[a] = L.lo[a];
-                b[3 + a] = L.hi[a];
+                b[a] = g.planes[L.lo[a]];
+                b[3 + a] = g.planes[L.hi[a]];
             }
         }
         for (int q = 0; q < n; ++q)
@@ -336,27 +359,8 @@ namespace skg
 
 namespace skg
 {
-    // TreeNode::leafChild from the root over the node records (TreeSpatialGrid.cpp:190-219): the
-    // cell of the leaf holding (x, y, z), -1 outside the root's closed box (one thread)
-    __global__ void octree_locate(GridView g, double x, double y, double z, int* out)
-    {
-        if (!(x >= g.box[0] && x <= g.box[3] && y >= g.box[1] && y <= g.box[4] && z >= g.box[2] && z <= g.box[5]))
-        {
-            *out = -1;
-            return;
-        }
-        int nd = 0;
-        while (true)
-        {
-            const TopNode t = g.top[nd];
-            if (t.child < 0)
-            {
-                *out = t.cell;
-                return;
-            }
-            nd = t.child + (x < t.sx ? 0 : 1) + (y < t.sy ? 0 : 2) + (z < t.sz ? 0 : 4);
-        }
-    }
+    // the node of the leaf holding (x, y, z), -1 outside the root's closed box (one thread)
+    __global__ void octree_locate(GridView g, double x, double y, double z, int* out) { *out = oct_search(g.node, g.planes, x, y, z); }
 }
 
 // ==================================================================== host side
@@ -399,6 +403,7 @@ struct skg_engine
     int gridType = -1;
     GridView grid{};
     int64_t ncells = 0;
+    int64_t nnodes = 0;  // octree: number of node records
     std::vector<void*> gridBufs;
     // medium
     double* dens = nullptr;
@@ -549,7 +554,8 @@ namespace
         int64_t n = e->ncells;
         dim3 grid(static_cast<unsigned>((n + 255) / 256)), block(256);
         if (e->gridType == SKG_GRID_OCTREE)
-            hipLaunchKernelGGL(fill_record_density<OctLeaf>, grid, block, 0, e->stream, const_cast<OctLeaf*>(e->grid.leaf), e->dens, n);
+            hipLaunchKernelGGL(fill_node_density, dim3(static_cast<unsigned>((e->nnodes + 255) / 256)), block, 0, e->stream,
+                               const_cast<OctNode*>(e->grid.node), e->dens, e->nnodes);
         else if (e->gridType == SKG_GRID_VORONOI)
         {
             hipLaunchKernelGGL(fill_record_density<VorCell>, grid, block, 0, e->stream, const_cast<VorCell*>(e->grid.vcell), e->dens, n);
@@ -659,23 +665,27 @@ namespace
         return SKG_OK;
     }
 
+    // dynamic LDS of the kernels that walk the grid: the octree's coordinate table
+    size_t planeBytes(const GridView& g) { return g.ldsPlanes ? static_cast<size_t>(g.nplanes) * sizeof(double) : 0; }
+
     template<int GT, int FP>
     hipError_t launchLifecycle(const SimParams& p, bool guided, int blocks, int threads, hipStream_t s)
     {
+        const size_t lds = planeBytes(p.grid);
         // batched instances, guided sampling and radiation-field storage take their own
         // instantiations; the plain run carries none of them
         if (p.ninst)
-            hipLaunchKernelGGL((lifecycle<GT, FP, kBatched>), dim3(blocks), dim3(threads), 0, s, p);
+            hipLaunchKernelGGL((lifecycle<GT, FP, kBatched>), dim3(blocks), dim3(threads), lds, s, p);
         else if (p.rf)
-            hipLaunchKernelGGL((lifecycle<GT, FP, kStoreRF>), dim3(blocks), dim3(threads), 0, s, p);
+            hipLaunchKernelGGL((lifecycle<GT, FP, kStoreRF>), dim3(blocks), dim3(threads), lds, s, p);
         else if (p.persp)
-            hipLaunchKernelGGL((lifecycle<GT, FP, kPersp>), dim3(blocks), dim3(threads), 0, s, p);
+            hipLaunchKernelGGL((lifecycle<GT, FP, kPersp>), dim3(blocks), dim3(threads), lds, s, p);
         else if (p.nent)
-            hipLaunchKernelGGL((lifecycle<GT, FP, kParticles>), dim3(blocks), dim3(threads), 0, s, p);
+            hipLaunchKernelGGL((lifecycle<GT, FP, kParticles>), dim3(blocks), dim3(threads), lds, s, p);
         else if (guided)
-            hipLaunchKernelGGL((lifecycle<GT, FP, kGuided>), dim3(blocks), dim3(threads), 0, s, p);
+            hipLaunchKernelGGL((lifecycle<GT, FP, kGuided>), dim3(blocks), dim3(threads), lds, s, p);
         else
-            hipLaunchKernelGGL((lifecycle<GT, FP, kPlain>), dim3(blocks), dim3(threads), 0, s, p);
+            hipLaunchKernelGGL((lifecycle<GT, FP, kPlain>), dim3(blocks), dim3(threads), lds, s, p);
         return hipGetLastError();
     }
 }
@@ -697,6 +707,50 @@ namespace
             case SKG_GRID_VORONOI: return f(std::integral_constant<int, kVoronoi>());
             default: return f(std::integral_constant<int, kTetra>());
         }
+    }
+
+    // The node a crossing of wall w (BACK..TOP) of leaf n enters (OctNode::first).  A neighbour
+    // list is sorted by decreasing overlap with the wall and may end with leaves that only touch
+    // the wall's edge.  When its first leaf covers the wall, that leaf; when the leaves that
+    // overlap the wall are exactly the descendants behind it of a node of the leaf's own size
+    // (their areas add up to the wall), that node; otherwise the list itself is walked.
+    int32_t octAcross(const double* bounds, const int32_t* parent, const int8_t* level, int32_t n, int w,
+                      const int32_t* ids, int64_t count)
+    {
+        if (count == 0) return kOctNoNb;
+        const int axis = w >> 1, u = (axis + 1) % 3, v = (axis + 2) % 3;
+        const double* b = bounds + 6 * static_cast<int64_t>(n);
+        const double plane = b[(w & 1) ? 3 + axis : axis];
+        auto touches = [&](const double* a) { return a[(w & 1) ? axis : 3 + axis] == plane; };
+        const double* f = bounds + 6 * static_cast<int64_t>(ids[0]);
+        if (ids[0] != n
+            && (count == 1
+                || (touches(f) && f[u] <= b[u] && f[3 + u] >= b[3 + u] && f[v] <= b[v] && f[3 + v] >= b[3 + v])))
+            return ids[0];
+        int32_t top = -1;
+        double area = 0.;
+        bool edges = false;  // past the last overlapping leaf
+        for (int64_t q = 0; q < count; ++q)
+        {
+            int32_t a = ids[q];
+            const double* c = bounds + 6 * static_cast<int64_t>(a);
+            if (!(std::min(c[3 + u], b[3 + u]) > std::max(c[u], b[u]) && std::min(c[3 + v], b[3 + v]) > std::max(c[v], b[v])))
+            {
+                edges = true;
+                continue;
+            }
+            const int d = level[a] - level[n];
+            if (edges || d < 1 || d > 24 || !touches(c)) return kOctList;
+            for (int64_t o = 0; o < q; ++o)
+                if (ids[o] == a) return kOctList;
+            area += std::ldexp(1., -2 * d);
+            for (int l = 0; l < d; ++l) a = parent[a];
+            if (top >= 0 && a != top) return kOctList;
+            top = a;
+        }
+        if (area != 1.) return kOctList;
+        const double* t = bounds + 6 * static_cast<int64_t>(top);
+        return touches(t) && t[u] == b[u] && t[3 + u] == b[3 + u] && t[v] == b[v] && t[3 + v] == b[3 + v] ? top : kOctList;
     }
 
     // block search lists for a tetrahedral grid: tbn^3 equal blocks over the domain; a tetra is
@@ -922,41 +976,82 @@ int skg_grid_octree(skg_engine* e, int64_t nnodes, const double* bounds, const i
             return fail(e, SKG_ERR_ARGUMENT, "skg_grid_octree: non-leaf node with a cell index");
     }
     if (ncells > INT32_MAX) return fail(e, SKG_ERR_ARGUMENT, "skg_grid_octree: too many cells");
-    // cell-indexed leaf records with the neighbour lists translated to cell ids
-    std::vector<OctLeaf> leaves(ncells);
+    // one record per node; the leaves' neighbour lists keep their node ids
+    std::vector<OctNode> nodes(nnodes);
+    std::memset(nodes.data(), 0, nodes.size() * sizeof(OctNode));
     std::vector<int32_t> nbc;
     nbc.reserve(static_cast<size_t>(nb_off[6 * nnodes]));
     std::vector<char> seen(ncells, 0);
+    std::vector<int32_t> parent(nnodes, -1);
+    std::vector<int8_t> level(nnodes, 0);
+    for (int64_t n = 0; n < nnodes; ++n)
+        if (child_first[n] >= 0)
+            for (int32_t c = child_first[n]; c < child_first[n] + 8; ++c)
+            {
+                parent[c] = static_cast<int32_t>(n);
+                level[c] = static_cast<int8_t>(std::min<int>(level[n] + 1, INT8_MAX));
+            }
+    // the distinct coordinates: a child's bounds are its parent's or its siblings' split point, so
+    // that nearly every coordinate is found by a comparison, the others by their value
+    std::vector<double> planes;
+    std::unordered_map<uint64_t, int32_t> planeOf;
+    auto plane = [&](double v) {
+        uint64_t bits;
+        std::memcpy(&bits, &v, sizeof(bits));
+        auto [it, fresh] = planeOf.try_emplace(bits, static_cast<int32_t>(planes.size()));
+        if (fresh) planes.push_back(v);
+        return it->second;
+    };
+    std::vector<int32_t> nbOff;
+    nbOff.reserve(static_cast<size_t>(6 * nnodes + 1));
+    nbOff.push_back(0);
     for (int64_t n = 0; n < nnodes; ++n)
     {
-        if (child_first[n] >= 0) continue;
+        OctNode& L = nodes[n];
+        const double* b = bounds + 6 * n;
+        if (parent[n] >= 0)
+        {
+            const OctNode& P = nodes[parent[n]];
+            for (int q = 0; q < 3; ++q)
+            {
+                auto known = [&](double v) {
+                    return planes[P.lo[q]] == v ? P.lo[q] : planes[P.hi[q]] == v ? P.hi[q] : planes[P.split[q]] == v ? P.split[q] : plane(v);
+                };
+                L.lo[q] = known(b[q]);
+                L.hi[q] = known(b[3 + q]);
+            }
+        }
+        else
+            for (int q = 0; q < 3; ++q)
+            {
+                L.lo[q] = plane(b[q]);
+                L.hi[q] = plane(b[3 + q]);
+            }
+        if (child_first[n] >= 0)
+        {
+            L.cell = ~child_first[n];
+            for (int q = 0; q < 3; ++q) L.split[q] = plane(bounds[6 * static_cast<int64_t>(child_first[n]) + 3 + q]);
+            nbOff.insert(nbOff.end(), 6, static_cast<int32_t>(nbc.size()));
+            continue;
+        }
         int32_t m = cell_index[n];
         if (seen[m]) return fail(e, SKG_ERR_ARGUMENT, "skg_grid_octree: duplicate cell index");
         seen[m] = 1;
-        OctLeaf& L = leaves[m];
-        std::memset(&L, 0, sizeof(L));
-        for (int q = 0; q < 3; ++q)
-        {
-            L.lo[q] = bounds[6 * n + q];
-            L.hi[q] = bounds[6 * n + 3 + q];
-        }
-        L.node = static_cast<int32_t>(n);
+        L.cell = m;
         for (int w = 0; w < 6; ++w)
         {
             int64_t b0 = nb_off[6 * n + w], b1 = nb_off[6 * n + w + 1];
             if (b1 < b0) return fail(e, SKG_ERR_ARGUMENT, "skg_grid_octree: offsets must not decrease");
-            L.off[w] = static_cast<int32_t>(nbc.size());
-            L.first[w] = -1;
             for (int64_t q = b0; q < b1; ++q)
             {
                 int32_t id = nb_id[q];
                 if (id < 0 || id >= nnodes || cell_index[id] < 0)
                     return fail(e, SKG_ERR_ARGUMENT, "skg_grid_octree: a leaf's neighbour must be a leaf");
-                if (q == b0) L.first[w] = cell_index[id];
-                nbc.push_back(cell_index[id]);
+                nbc.push_back(id);
             }
+            nbOff.push_back(static_cast<int32_t>(nbc.size()));
+            L.first[w] = octAcross(bounds, parent.data(), level.data(), static_cast<int32_t>(n), w, nb_id + b0, b1 - b0);
         }
-        L.off_end = static_cast<int32_t>(nbc.size());
     }
     for (int64_t m = 0; m < ncells; ++m)
         if (!seen[m]) return fail(e, SKG_ERR_ARGUMENT, "skg_grid_octree: cell indices must be 0..ncells-1");
@@ -965,33 +1060,19 @@ int skg_grid_octree(skg_engine* e, int64_t nnodes, const double* bounds, const i
     freeGrid(e);
     GridView g{};
     int st;
-    if ((st = gridUpload(e, leaves.data(), leaves.size(), &g.leaf))) return st;
-    // the octree step machine loads 112 bytes from any entry: 28 ints of padding
-    nbc.resize(nbc.size() + 28, 0);
-    if ((st = gridUpload(e, nbc.data(), nbc.size(), &g.nbc))) return st;
-    // every node in the search's form; the kernels stage ids below kTopNodes in LDS (the
-    // level-by-level construction numbers the top levels first)
-    {
-        std::vector<TopNode> top(nnodes + 3);  // + 96 bytes: the step machine loads 112 from an entry
-        for (int64_t n = 0; n < nnodes; ++n)
-        {
-            const int32_t c = child_first[n];
-            top[n].child = c;
-            top[n].cell = c >= 0 ? -1 : cell_index[n];
-            top[n].sx = c >= 0 ? bounds[6 * static_cast<int64_t>(c) + 3] : 0.;
-            top[n].sy = c >= 0 ? bounds[6 * static_cast<int64_t>(c) + 4] : 0.;
-            top[n].sz = c >= 0 ? bounds[6 * static_cast<int64_t>(c) + 5] : 0.;
-        }
-        for (int64_t n = nnodes; n < nnodes + 3; ++n) top[n] = TopNode{0., 0., 0., -1, 0};
-        if ((st = gridUpload(e, top.data(), top.size(), &g.top))) return st;
-        g.topN = static_cast<int>(std::min<int64_t>(nnodes, kTopNodes));
-    }
+    if ((st = gridUpload(e, nodes.data(), nodes.size(), &g.node))) return st;
+    if ((st = gridUpload(e, planes.data(), planes.size(), &g.planes))) return st;
+    if ((st = gridUpload(e, nbOff.data(), nbOff.size(), &g.nbOff))) return st;
+    if (!nbc.empty() && (st = gridUpload(e, nbc.data(), nbc.size(), &g.nbc))) return st;
+    g.nplanes = static_cast<int>(planes.size());
+    g.ldsPlanes = planes.size() <= static_cast<size_t>(kLdsPlanes);
     for (int q = 0; q < 6; ++q) g.box[q] = bounds[q];
     double dx = g.box[3] - g.box[0], dy = g.box[4] - g.box[1], dz = g.box[5] - g.box[2];
     g.eps = 1e-12 * std::sqrt(dx * dx + dy * dy + dz * dz);  // TreeSpatialGrid.cpp:28
     e->grid = g;
     e->gridType = SKG_GRID_OCTREE;
     e->ncells = ncells;
+    e->nnodes = nnodes;
     return refreshLeafDensity(e);
 }
 
@@ -1190,7 +1271,7 @@ int skg_trace_paths(skg_engine* e, const double* rays, int64_t n, int64_t cap, i
     GridView g = e->grid;
     g.dens = e->dens;
     dispatchGrid(e, [&](auto gt) {
-        hipLaunchKernelGGL((trace_count<decltype(gt)::value>), dim3(blocks), dim3(256), 0, e->stream, g, dRays, n, dCnt);
+        hipLaunchKernelGGL((trace_count<decltype(gt)::value>), dim3(blocks), dim3(256), planeBytes(g), e->stream, g, dRays, n, dCnt);
         return 0;
     });
     std::vector<int64_t> cnt(2 * n);
@@ -1219,7 +1300,7 @@ int skg_trace_paths(skg_engine* e, const double* rays, int64_t n, int64_t cap, i
     if (t)
     {
         dispatchGrid(e, [&](auto gt) {
-            hipLaunchKernelGGL((trace_write<decltype(gt)::value>), dim3(blocks), dim3(256), 0, e->stream, g, dRays, n, dOff,
+            hipLaunchKernelGGL((trace_write<decltype(gt)::value>), dim3(blocks), dim3(256), planeBytes(g), e->stream, g, dRays, n, dOff,
                                dM, dDs);
             return 0;
         });
@@ -1258,7 +1339,7 @@ int skg_trace_paths_noalloc(skg_engine* e, const double* rays, int64_t n, int64_
     g.dens = e->dens;
     const int blocks = static_cast<int>((n + 255) / 256);
     dispatchGrid(e, [&](auto gt) {
-        hipLaunchKernelGGL((trace_count_off<decltype(gt)::value>), dim3(blocks), dim3(256), 0, e->stream, g, rays, n, off);
+        hipLaunchKernelGGL((trace_count_off<decltype(gt)::value>), dim3(blocks), dim3(256), planeBytes(g), e->stream, g, rays, n, off);
         return 0;
     });
     hipLaunchKernelGGL(scan_block_sums, dim3(static_cast<unsigned>(nb)), dim3(256), 0, e->stream, off, n, e->scan);
@@ -1274,7 +1355,7 @@ int skg_trace_paths_noalloc(skg_engine* e, const double* rays, int64_t n, int64_
     if (t)
     {
         dispatchGrid(e, [&](auto gt) {
-            hipLaunchKernelGGL((trace_write<decltype(gt)::value>), dim3(blocks), dim3(256), 0, e->stream, g, rays, n, off, m, ds);
+            hipLaunchKernelGGL((trace_write<decltype(gt)::value>), dim3(blocks), dim3(256), planeBytes(g), e->stream, g, rays, n, off, m, ds);
             return 0;
         });
         HIPCHK(e, hipGetLastError());
@@ -1315,10 +1396,10 @@ int skg_trace_tau(skg_engine* e, const double* rays, int64_t n, int32_t ell, dou
     g.dens = e->dens;
     dispatchGrid(e, [&](auto gt) {
         if (fp_mode == SKG_FP64)
-            hipLaunchKernelGGL((trace_tau<decltype(gt)::value, SKG_FP64>), dim3(blocks), dim3(256), 0, e->stream, g, e->dens,
+            hipLaunchKernelGGL((trace_tau<decltype(gt)::value, SKG_FP64>), dim3(blocks), dim3(256), planeBytes(g), e->stream, g, e->dens,
                                e->dens32, section, taumax, dRays, n, dTp, dTo, dToff, dCum);
         else
-            hipLaunchKernelGGL((trace_tau<decltype(gt)::value, SKG_FP32_KAHAN>), dim3(blocks), dim3(256), 0, e->stream, g,
+            hipLaunchKernelGGL((trace_tau<decltype(gt)::value, SKG_FP32_KAHAN>), dim3(blocks), dim3(256), planeBytes(g), e->stream, g,
                                e->dens, e->dens32, section, taumax, dRays, n, dTp, dTo, dToff, dCum);
         return 0;
     });
@@ -1588,7 +1669,8 @@ int skg_sample_density(skg_engine* e, const skg_disk_model* model, int32_t num_s
     if (e->gridType == SKG_GRID_CARTESIAN)
         hipLaunchKernelGGL(sample_density_kernel<kCartesian>, grid, block, 0, e->stream, e->grid, md, num_samples, seed, e->ncells, d);
     else if (e->gridType == SKG_GRID_OCTREE)
-        hipLaunchKernelGGL(sample_density_kernel<kOctree>, grid, block, 0, e->stream, e->grid, md, num_samples, seed, e->ncells, d);
+        hipLaunchKernelGGL(sample_density_kernel<kOctree>, dim3(static_cast<unsigned>((e->nnodes + 255) / 256)), block, 0,
+                           e->stream, e->grid, md, num_samples, seed, e->nnodes, d);
     else
         hipLaunchKernelGGL(sample_density_kernel<kTetra>, grid, block, 0, e->stream, e->grid, md, num_samples, seed, e->ncells, d);
     hipError_t st = hipGetLastError();
@@ -1853,8 +1935,14 @@ static int runPersistent(skg_engine* e, uint64_t first_history, uint64_t count)
     (void)hipGetLastError();
     int threads = e->threads;
     int blocks = e->workgroups > 0 ? e->workgroups : e->cus * 8;
-    // never more lanes than packets (rounded up to whole workgroups)
-    int64_t needBlocks = static_cast<int64_t>((count + threads - 1) / threads);
+    // Never more lanes than packets, and a run that does not fill two wavefronts per SIMD is
+    // spread over that many, with fewer lanes of each: a wave waits for the longest of its lanes
+    // at every step, and 4096 packets in full wavefronts would use 16 of the 256 CUs (Cartesian
+    // 32^3, 4096 packets: 0.92 -> 0.64 ms).  Below four lanes the waves only add up.
+    p.lanes = static_cast<int>(
+        std::clamp<int64_t>((static_cast<int64_t>(count) + 8 * e->cus - 1) / (8 * e->cus), 4, 64));
+    const int64_t perBlock = static_cast<int64_t>(p.lanes) * (threads / 64);
+    int64_t needBlocks = (static_cast<int64_t>(count) + perBlock - 1) / perBlock;
     blocks = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(blocks, needBlocks)));
     HIPCHK(e, hipEventRecord(e->ev0, e->stream));
     hipError_t err;
@@ -1939,7 +2027,7 @@ namespace
                 hipLaunchKernelGGL((pipe_event<GT, 0>), dim3(eventBlocks), dim3(256), 0, e->stream, p, par);
             // external event nodes: recorded on every replay, so each trace launch is timed
             hipError_t r1 = hipEventRecordWithFlags(e->traceEv[2 * i], e->stream, hipEventRecordExternal);
-            hipLaunchKernelGGL((pipe_trace<GT, FP>), dim3(traceBlocks), dim3(256), 0, e->stream, p, par);
+            hipLaunchKernelGGL((pipe_trace<GT, FP>), dim3(traceBlocks), dim3(256), planeBytes(p.grid), e->stream, p, par);
             hipError_t r2 = hipEventRecordWithFlags(e->traceEv[2 * i + 1], e->stream, hipEventRecordExternal);
             if (r1 != hipSuccess || r2 != hipSuccess)
             {

@@ -38,6 +38,7 @@ namespace skg
         double xi, min_weight_reduction;
         int min_scatt;
         int threshold;
+        int lanes;  // lanes of each wavefront that take packets
         uint64_t seed;
         uint64_t first, count;
         unsigned long long* queue;     // next history offset (work queue head)
@@ -53,7 +54,7 @@ namespace skg
         uint32_t contKey;         // nonzero: histories continue on Philox tag contKey from their first
                                   // scattering on (same emission and first interaction, independent
                                   // continuations)
-        int32_t srcHint;          // octree: the leaf of the point source (the start hint of new packets), -1: none
+        int32_t srcHint;          // octree: the leaf node of the point source (the start hint of new packets), -1: none
         double* rf;               // radiation-field variant: ncells x nlambda table
         int persp;                // some instruments are perspective instruments
         int nent;                 // particle-source variant: number of entities (0: the point source)
@@ -131,17 +132,27 @@ namespace skg
     constexpr int kLcThreads = 256;
     constexpr int kColdBytes = kLcThreads * (8 * kColdF64 + 4 * kColdU32);  // 34 KB per workgroup
 
+    // LDS pointers: the event function, a call of its own, then reads the packet with LDS
+    // instructions (a generic pointer would make them flat ones)
+    typedef __attribute__((address_space(3))) double LdsF64;
+    typedef __attribute__((address_space(3))) uint32_t LdsU32;
+
+    __device__ __forceinline__ void lds_count(LdsU32* c, uint32_t v = 1u)
+    {
+        __hip_atomic_fetch_add(c, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+
     struct Packet
     {
         Philox rng;
         double rx, ry, rz, kx, ky, kz;
         double W, lam, Lthr, taupath, tauCached, Wp;
         int ell, nscatt, f, pix, inst;
-        int hint;  // a cell that probably holds the packet's position (-1: none)
+        int hint;  // a cell (octree: a leaf's node) that probably holds the packet's position (-1: none)
         bool scat, haveTau;
 
         template<bool INST>
-        __device__ __forceinline__ void load(const double* cd, const uint32_t* cu, int t, const SimParams& p)
+        __device__ __forceinline__ void load(const LdsF64* cd, const LdsU32* cu, int t, const SimParams& p)
         {
             rx = cd[cRx * kLcThreads + t];
             ry = cd[cRy * kLcThreads + t];
@@ -170,7 +181,7 @@ namespace skg
             haveTau = (fl >> 1) & 1u;
         }
 
-        __device__ __forceinline__ void store(double* cd, uint32_t* cu, int t) const
+        __device__ __forceinline__ void store(LdsF64* cd, LdsU32* cu, int t) const
         {
             cd[cRx * kLcThreads + t] = rx;
             cd[cRy * kLcThreads + t] = ry;
@@ -197,6 +208,19 @@ namespace skg
         }
     };
 
+    // What an event (life_event) returns: the packet's next phase and traversal -- direction, start
+    // cell, section, the optical depth that ends it early (lim), the path length that does (slim) --
+    // and the event's detector deposit (off < 0: none).  The traversal starts at the packet's
+    // position.
+    struct EventOut
+    {
+        int phase, hint, ell;
+        double kx, ky, kz;
+        double section, lim, slim, rfL;
+        int64_t off;
+        double v;
+    };
+
     // traversal state of one lane: the generator, the running sums and the phase
     template<int GT, int FP> struct Trav
     {
@@ -204,15 +228,13 @@ namespace skg
         int phase;
         bool ended;
         int steps;
-        double tau, s, tprev, sprev;  // FP64 sums
-        Kahan32 tau32, s32;           // FP32 sums
-        int lastm;
+        double tau, s;         // FP64 sums (s of a finished forced path: the distance of the interaction
+                               // or of the path's end)
+        Kahan32 tau32, s32;    // FP32 sums
+        int last;              // cell (octree: node) of the last stored segment; the interaction's
         double section;
-        float section32;
-        double taumax;  // peel-off: early-out optical depth
-        double tint;    // second forced pass: interaction optical depth
-        int mint;
-        double sint;
+        double lim;            // the traversal ends where the optical depth exceeds it: the early-out
+                               // of a peel-off, the interaction of a second forced pass
         int ell;        // radiation-field variant: the packet's bin, luminosity and the
         double rfL;     // extinction factor at the start of the current segment
         double rfExt;
@@ -226,161 +248,172 @@ namespace skg
         {
             return FP == SKG_FP64 ? s : static_cast<double>(s32.sum);
         }
-
-        __device__ __forceinline__ void start(const Packet& pk, double dx, double dy, double dz, int ph)
+        // the distance a finished forced path reached
+        __device__ __forceinline__ double s_end(bool interaction) const
         {
-            gen.start(pk.rx, pk.ry, pk.rz, dx, dy, dz, pk.hint);
-            phase = ph;
+            return FP == SKG_FP64 || interaction ? s : static_cast<double>(s32.sum);
+        }
+        __device__ __forceinline__ void add_length(double ds)
+        {
+            if (FP == SKG_FP64)
+                s += ds;
+            else
+                s32.add(static_cast<float>(ds));
+        }
+
+        __device__ __forceinline__ void finish(LdsU32* lds)
+        {
+            ended = true;
+            // the crossing counters are added once, where a traversal ends
+            lds_count(lds + 4, static_cast<uint32_t>(steps));
+            if (phase == kFwd2) lds_count(lds + 7, static_cast<uint32_t>(steps));
+        }
+
+        // starts the traversal an event asked for and enters the domain; the path's length before
+        // the domain, if any, is its first segment
+        template<bool PERSP>
+        __device__ __forceinline__ void start(const GridView& grid, const EventOut& io, LdsF64* cd, LdsU32* cu, LdsU32* lds,
+                                              int t)
+        {
+            gen.start(cd[cRx * kLcThreads + t], cd[cRy * kLcThreads + t], cd[cRz * kLcThreads + t], io.kx, io.ky, io.kz,
+                      io.hint);
+            phase = io.phase;
             ended = false;
             steps = 0;
             tau = 0.;
             s = 0.;
-            tprev = 0.;
-            sprev = 0.;
             tau32.reset();
             s32.reset();
-            lastm = -1;
+            last = -1;
+            section = io.section;
+            lim = io.lim;
             // radiation-field variant: the luminosity at the start of a forced path and the
             // extinction factor before its first segment (unused, and removed, elsewhere)
-            ell = pk.ell;
-            rfL = pk.W / pk.lam;
+            ell = io.ell;
+            rfL = io.rfL;
             rfExt = 1.;
-            slim = INFINITY;
+            slim = io.slim;
+            double entry;
+            bool fin = !gen.begin(grid, entry);
+            // every traversal starts at the packet's position: its start cell is the hint for the
+            // next traversal from there (octree, Voronoi and tetrahedral grids)
+            if constexpr (GT != kCartesian)
+                if (gen.hint >= 0) cu[cHint * kLcThreads + t] = static_cast<uint32_t>(gen.hint);
+            if (!fin && entry > 0.)
+            {
+                steps = 1;
+                if (phase != kPeel)
+                    add_length(entry);
+                else if (PERSP)
+                {
+                    s += entry;
+                    fin = s > slim;
+                }
+            }
+            if (fin) finish(lds);
         }
 
         // one cell crossing of the current traversal; with RF, the first forced pass also
         // stores the radiation field (MonteCarloSimulation::storeRadiationField, :909-925):
         // L * lnmean(e^-tau_end, e^-tau_begin) * ds per stored segment in a cell
         template<bool RF, bool PERSP>
-        __device__ __forceinline__ void step(const GridView& grid, unsigned int* lds, double* rf, int nl)
+        __device__ __forceinline__ void step(const GridView& grid, LdsU32* lds, double* rf, int nl)
         {
+            const int at = gen.i;  // the octree's leaves are named by their node, other cells by m
             int m;
             double ds, nd;
-            const int r = gen.advance(grid, m, ds, nd);
-            if (r == 0) return;  // an octree step that loaded a search node or list entry
-            // the traversal ends at the path's end (r < 0, or r == 2 after its last segment), at
-            // the early-out optical depth of a peel-off, past a perspective peel-off's distance, or
-            // at a second pass's interaction; the crossing counters are added once, where it ends
+            const int r = gen.cross(grid, m, ds, nd);
+            if (r == 0) return;  // one level of the octree's descent
+            // the traversal ends at the path's end (r < 0, or r == 2 after its last segment), where
+            // its optical depth exceeds lim, or past a perspective peel-off's distance
             bool fin = r < 0 || ++steps > kMaxSteps;
             if (!fin)
             {
-                if (phase == kPeel)
+                const bool peel = phase == kPeel;
+                const double tprev = tau_value(), sprev = s_value();
+                // a peel-off's optical depth counts every segment, a forced path stores those of
+                // positive length
+                if (peel || ds > 0.)
                 {
-                    if (m >= 0)
+                    if (FP == SKG_FP64)
+                        tau += section * nd * ds;
+                    else
+                        tau32.add(static_cast<float>(section) * static_cast<float>(nd) * static_cast<float>(ds));
+                    if (!peel)
                     {
-                        if (FP == SKG_FP64)
+                        add_length(ds);
+                        last = GT == kOctree ? at : m;
+                        if constexpr (RF)
                         {
-                            tau += section * nd * ds;
-                            if (tau >= taumax)
+                            if (phase == kFwd1)
                             {
-                                tau = INFINITY;
-                                fin = true;
-                            }
-                        }
-                        else
-                        {
-                            tau32.add(section32 * static_cast<float>(nd) * static_cast<float>(ds));
-                            if (static_cast<double>(tau32.sum) >= taumax)
-                            {
-                                tau32.sum = INFINITY;
-                                fin = true;
+                                const double lnEnd = -tau_value();
+                                const double extEnd = exp(lnEnd);
+                                const double em = ln_mean(extEnd, rfExt, lnEnd, -tprev);
+                                unsafeAtomicAdd(rf + static_cast<int64_t>(m) * nl + ell, rfL * em * ds);
+                                rfExt = extEnd;
                             }
                         }
                     }
-                    if constexpr (PERSP)
+                }
+                if (__builtin_expect(tau_value() > lim, 0))
+                {
+                    fin = true;
+                    if (peel)
                     {
-                        // MediumSystem::getExtinctionOpticalDepth(pp, distance) (MediumSystem.cpp:
-                        // 2376-2382): the segment that passes the distance still counts
+                        if (FP == SKG_FP64)
+                            tau = INFINITY;
+                        else
+                            tau32.sum = INFINITY;
+                    }
+                    else
+                    {
+                        // the second pass stops at the first segment whose exit optical depth
+                        // exceeds the interaction's
+                        s = sprev + ((lim - tprev) / (tau_value() - tprev)) * (s_value() - sprev);
+                    }
+                }
+                if constexpr (PERSP)
+                {
+                    // MediumSystem::getExtinctionOpticalDepth(pp, distance) (MediumSystem.cpp:
+                    // 2376-2382): the segment that passes the distance still counts
+                    if (peel)
+                    {
                         s += ds;
                         if (s > slim) fin = true;
                     }
                 }
-                else if (ds > 0.)
-                {
-                    if (FP == SKG_FP64)
-                    {
-                        tprev = tau;
-                        sprev = s;
-                        s += ds;
-                        if (m >= 0) tau += section * nd * ds;
-                    }
-                    else
-                    {
-                        tprev = static_cast<double>(tau32.sum);
-                        sprev = static_cast<double>(s32.sum);
-                        s32.add(static_cast<float>(ds));
-                        if (m >= 0) tau32.add(section32 * static_cast<float>(nd) * static_cast<float>(ds));
-                    }
-                    lastm = m;
-                    if constexpr (RF)
-                    {
-                        if (phase == kFwd1)
-                        {
-                            const double lnEnd = -tau_value();
-                            const double extEnd = exp(lnEnd);
-                            if (m >= 0)
-                            {
-                                const double em = ln_mean(extEnd, rfExt, lnEnd, -tprev);
-                                unsafeAtomicAdd(rf + static_cast<int64_t>(m) * nl + ell, rfL * em * ds);
-                            }
-                            rfExt = extEnd;
-                        }
-                    }
-                    // second pass: stop at the first segment whose exit optical depth exceeds tau_int
-                    if (phase == kFwd2 && tint < tau_value())
-                    {
-                        mint = m;
-                        double tv = tau_value(), sv = s_value();
-                        sint = sprev + ((tint - tprev) / (tv - tprev)) * (sv - sprev);
-                        fin = true;
-                    }
-                }
             }
-            fin = fin || r == 2;
-            if (fin)
-            {
-                ended = true;
-                atomicAdd(lds + 4, static_cast<unsigned int>(steps));
-                if (phase == kFwd2) atomicAdd(lds + 7, static_cast<unsigned int>(steps));
-            }
+            if (__builtin_expect(fin || r == 2, 0)) finish(lds);
         }
-    };
-
-    // A lane's detector deposit of the current transition round, held until the wave
-    // combines the round's deposits (flush_deposits); off < 0: none
-    struct Pending
-    {
-        int64_t off;
-        double v;
     };
 
     // The deposits of one transition round into the frames (FluxRecorder::detect,
     // FluxRecorder.cpp:414-418, with LockFree::add, LockFree.hpp:23-36), combined across the
     // wavefront: the deposits into the pixel of the first depositing lane are summed by a
     // shuffle reduction over the whole (converged) wave into one FP64 atomic, the others are
-    // added directly.  Counter 5 counts the atomics issued.
-    __device__ __forceinline__ void flush_deposits(double* frame, Pending& pd, unsigned int* lds)
+    // added directly.  off < 0: no deposit.  Counter 5 counts the atomics issued.
+    __device__ __forceinline__ void flush_deposits(double* frame, int64_t off, double val, LdsU32* lds)
     {
-        const bool has = pd.off >= 0;
+        const bool has = off >= 0;
         const unsigned long long m = __ballot(has);
         if (!m) return;
         const int leader = __ffsll(static_cast<long long>(m)) - 1;
-        const int64_t key = __shfl(pd.off, leader);
-        const bool same = has && pd.off == key;
-        double v = same ? pd.v : 0.;
+        const int64_t key = __shfl(off, leader);
+        const bool same = has && off == key;
+        double v = same ? val : 0.;
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
         if (__lane_id() == leader)
         {
             unsafeAtomicAdd(frame + key, v);
-            atomicAdd(lds + 5, 1u);
+            lds_count(lds + 5);
         }
         if (has && !same)
         {
-            unsafeAtomicAdd(frame + pd.off, pd.v);
-            atomicAdd(lds + 5, 1u);
+            unsafeAtomicAdd(frame + off, val);
+            lds_count(lds + 5);
         }
-        pd.off = -1;
     }
 
     // The guided scattering direction (defensive mixture of the guide's lobes and HG) and its
@@ -405,20 +438,47 @@ namespace skg
     }
 
     // The event transitions of the life cycle, on a packet loaded from LDS.
-    template<int GT, int FP, int V> struct Events
+    template<int GT, int V> struct Events
     {
         static constexpr bool INST = V == kBatched;
         const SimParams& p;
-        Trav<GT, FP>& T;
+        EventOut& io;
         Packet& pk;
-        unsigned int* lds;
-        Pending& pd;
+        LdsU32* lds;
 
         __device__ __forceinline__ void finish()
         {
-            atomicAdd(lds + 0, 1u);
-            T.phase = kFetch;
-            T.ended = false;
+            lds_count(lds + 0);
+            io.phase = kFetch;
+        }
+
+        // the packet's next traversal, from its position
+        __device__ __forceinline__ void travel(double dx, double dy, double dz, int ph, double lim)
+        {
+            io.phase = ph;
+            io.kx = dx;
+            io.ky = dy;
+            io.kz = dz;
+            io.hint = pk.hint;
+            io.section = INST ? p.sext[pk.ell] * p.inst[pk.inst].scale : p.sext[pk.ell];
+            io.lim = lim;
+            io.slim = INFINITY;
+            io.ell = pk.ell;
+            io.rfL = pk.W / pk.lam;
+        }
+
+        // a peel-off of luminosity L: it ends at the optical depth log(L) + 745 (MediumSystem.cpp:
+        // 2335), that is where the sum exceeds the next smaller number
+        __device__ __forceinline__ void peel(double dx, double dy, double dz, double L)
+        {
+            lds_count(lds + 1);
+            travel(dx, dy, dz, kPeel, nextafter(log(L) + 745, -INFINITY));
+        }
+
+        __device__ __forceinline__ void forced()
+        {
+            lds_count(lds + 2);
+            travel(pk.kx, pk.ky, pk.kz, kFwd1, INFINITY);
         }
 
         // L exp(-tau) into the packet's pixel: held for the wave's combined flush at the end of
@@ -426,19 +486,19 @@ namespace skg
         __device__ __forceinline__ void deposit(const FrameGeom& fg, double L, double t)
         {
             double v = L * exp(-t);
-            if (pd.off >= 0)
+            if (io.off >= 0)
             {
-                unsafeAtomicAdd(p.frame + pd.off, pd.v);
-                atomicAdd(lds + 5, 1u);
+                unsafeAtomicAdd(p.frame + io.off, io.v);
+                lds_count(lds + 5);
             }
-            pd.off = fg.offset + pk.pix + static_cast<int64_t>(pk.ell) * fg.nx * fg.ny;
-            pd.v = v;
-            atomicAdd(lds + 8, 1u);
+            io.off = fg.offset + pk.pix + static_cast<int64_t>(pk.ell) * fg.nx * fg.ny;
+            io.v = v;
+            lds_count(lds + 8);
         }
 
         // MonteCarloSimulation::performLifeCycle launch + SourceSystem::launch; in a batched
         // launch, history h is history h - offset of its instance
-        __device__ __forceinline__ void launch(uint64_t h)
+        __device__ __forceinline__ bool launch(uint64_t h)
         {
             uint64_t seed = p.seed;
             const double* lp = p.lpack;
@@ -463,8 +523,6 @@ namespace skg
             pk.ell = static_cast<int>(pk.rng.uniform() * p.nlambda);
             if (pk.ell >= p.nlambda) pk.ell = p.nlambda - 1;
             pk.lam = p.lambda[pk.ell];
-            T.section = INST ? p.sext[pk.ell] * p.inst[pk.inst].scale : p.sext[pk.ell];
-            T.section32 = static_cast<float>(T.section);
             // the particle launch: its own variant, and a run-time branch of the radiation-field
             // and perspective variants
             bool particles = false;
@@ -534,17 +592,17 @@ namespace skg
             if (!(pk.W / pk.lam > 0))
             {
                 finish();
-                return;
+                return false;
             }
             pk.Lthr = (pk.W / pk.lam) / p.min_weight_reduction;
             begin_peel(false);
+            return true;
         }
 
         __device__ __forceinline__ void begin_peel(bool scattering)
         {
             pk.scat = scattering;
             pk.f = (INST ? p.inst[pk.inst].fbeg : 0) - 1;
-            next_peel();
         }
 
         // peel-off toward each instrument in turn (MonteCarloSimulation.cpp:698-715, :2034-2092;
@@ -591,10 +649,8 @@ namespace skg
                             pk.tauCached = INFINITY;
                             continue;
                         }
-                        T.taumax = log(L) + 745;
-                        atomicAdd(lds + 1, 1u);
-                        T.start(pk, ox, oy, oz, kPeel);
-                        T.slim = zp;
+                        peel(ox, oy, oz, L);
+                        io.slim = zp;
                         return;
                     }
                 }
@@ -622,9 +678,7 @@ namespace skg
                     pk.tauCached = INFINITY;
                     continue;
                 }
-                T.taumax = log(L) + 745;
-                atomicAdd(lds + 1, 1u);
-                T.start(pk, fg.kobs[0], fg.kobs[1], fg.kobs[2], kPeel);
+                peel(fg.kobs[0], fg.kobs[1], fg.kobs[2], L);
                 return;
             }
             // all instruments done: scatter (after a scattering peel-off) and start a forced path
@@ -633,17 +687,15 @@ namespace skg
                 if constexpr (V == kGuided)
                 {
                     // the wave's guided scattering round follows (guided_scatter)
-                    T.phase = kScatter;
-                    T.ended = false;
+                    io.phase = kScatter;
                     return;
                 }
                 if (p.contKey != 0u && pk.nscatt == 0) pk.rng.retag(p.contKey);
                 scatter_hg(pk.rng, p.gpar[pk.ell], pk.kx, pk.ky, pk.kz);
                 pk.nscatt++;
-                atomicAdd(lds + 3, 1u);
+                lds_count(lds + 3);
             }
-            atomicAdd(lds + 2, 1u);
-            T.start(pk, pk.kx, pk.ky, pk.kz, kFwd1);
+            forced();
         }
 
         // Guided scattering with the network outputs o of this packet's event: a direction from
@@ -658,22 +710,17 @@ namespace skg
             pk.W *= ratio;
             pk.Lthr *= ratio;
             pk.nscatt++;
-            atomicAdd(lds + 3, 1u);
-            atomicAdd(lds + 2, 1u);
-            T.start(pk, pk.kx, pk.ky, pk.kz, kFwd1);
+            lds_count(lds + 3);
+            forced();
         }
 
-        // event handling once a traversal ended
-        __device__ __forceinline__ void transition()
+        // event handling once a traversal ended; true when the packet peels off next
+        __device__ __forceinline__ bool transition(int phase, int last, double tau, double s)
         {
-            // every traversal starts at the packet's position: its start cell is the hint for
-            // the next traversal from there (octree, Voronoi and tetrahedral grids)
-            if constexpr (GT != kCartesian)
-                if (T.gen.hint >= 0) pk.hint = T.gen.hint;
-            if (T.phase == kPeel)
+            if (phase == kPeel)
             {
                 pk.haveTau = true;
-                pk.tauCached = T.tau_value();
+                pk.tauCached = tau;
                 const FrameGeom& fg = p.frames[pk.f];
                 double L = pk.Wp / pk.lam;
                 if constexpr (V == kPersp || V == kStoreRF)
@@ -686,17 +733,17 @@ namespace skg
                     }
                 }
                 deposit(fg, L, pk.tauCached);
-                next_peel();
+                return true;
             }
-            else if (T.phase == kFwd1)
+            if (phase == kFwd1)
             {
                 // MonteCarloSimulation::simulateForcedPropagation (:1492-1544)
-                pk.taupath = T.tau_value();
+                pk.taupath = tau;
                 if (pk.taupath <= 0.)
                 {
                     pk.W *= 0.;
                     finish();
-                    return;
+                    return false;
                 }
                 double xi = p.xi;
                 double tint;
@@ -709,67 +756,106 @@ namespace skg
                     double q = (1.0 - xi) * pp + xi / pk.taupath;
                     pk.W *= pp / q;
                 }
-                atomicAdd(lds + 6, 1u);
-                T.start(pk, pk.kx, pk.ky, pk.kz, kFwd2);
-                T.tint = tint;
-                T.mint = -1;
+                lds_count(lds + 6);
+                travel(pk.kx, pk.ky, pk.kz, kFwd2, tint);
+                return false;
             }
-            else if (T.phase == kFwd2)
+            // the second pass: SpatialGridPath::findInteractionPoint (SpatialGridPath.cpp:161-203):
+            // the interaction's cell and distance, or beyond the last segment that segment's
+            const int m = last;
+            double n = 0.;
+            if (m >= 0) n = GT == kOctree ? p.grid.node[m].dens : p.dens[m];
+            double ss = INST ? p.ssca[pk.ell] * p.inst[pk.inst].scale : p.ssca[pk.ell];
+            double se = INST ? p.sext[pk.ell] * p.inst[pk.inst].scale : p.sext[pk.ell];
+            double ksca = n > 0. ? n * ss : 0.;
+            double kext = n > 0. ? n * se : 0.;
+            double albedo = kext > 0. ? ksca / kext : 0.;
+            pk.W *= -expm1(-pk.taupath) * albedo;
+            if constexpr (GT != kCartesian)
+                pk.hint = m;  // the interaction point lies in the cell of its segment
+            pk.rx += s * pk.kx;
+            pk.ry += s * pk.ky;
+            pk.rz += s * pk.kz;
+            double L = pk.W / pk.lam;
+            if (L <= 0 || (L <= pk.Lthr && pk.nscatt >= p.min_scatt) || pk.nscatt >= kMaxScatterings)
             {
-                // SpatialGridPath::findInteractionPoint (SpatialGridPath.cpp:161-203): beyond the
-                // last segment, use the last segment's cell and exit distance
-                if (T.mint < 0 && !(T.tint < T.tau_value()))
-                {
-                    T.mint = T.lastm;
-                    T.sint = T.s_value();
-                }
-                int m = T.mint;
-                double n = m >= 0 ? p.dens[m] : 0.;
-                double ss = INST ? p.ssca[pk.ell] * p.inst[pk.inst].scale : p.ssca[pk.ell];
-                double ksca = n > 0. ? n * ss : 0.;
-                double kext = n > 0. ? n * T.section : 0.;
-                double albedo = kext > 0. ? ksca / kext : 0.;
-                pk.W *= -expm1(-pk.taupath) * albedo;
-                if constexpr (GT != kCartesian)
-                    pk.hint = m;  // the interaction point lies in the cell of its segment
-                pk.rx += T.sint * pk.kx;
-                pk.ry += T.sint * pk.ky;
-                pk.rz += T.sint * pk.kz;
-                double L = pk.W / pk.lam;
-                if (L <= 0 || (L <= pk.Lthr && pk.nscatt >= p.min_scatt) || pk.nscatt >= kMaxScatterings)
-                {
-                    finish();
-                    return;
-                }
-                begin_peel(true);
+                finish();
+                return false;
             }
+            begin_peel(true);
+            return true;
         }
     };
 
+    // The kernel's parameter block, passed to a function in vector registers, as the uniform
+    // address it is: its fields are then read with scalar loads
+    __device__ __forceinline__ const SimParams& uniform_params(const SimParams* q)
+    {
+        const uint64_t a = reinterpret_cast<uint64_t>(q);
+        const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(a));
+        const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(a >> 32));
+        typedef const __attribute__((address_space(4))) SimParams* KernargPtr;
+        return *(const SimParams*)(KernargPtr)(static_cast<uint64_t>(hi) << 32 | lo);
+    }
+
+    // One event of one packet: the launch of history `hist` (phase kFetch) or what follows the
+    // traversal of phase `phase` that ended with optical depth tau, cell `last` and distance s, up to
+    // the packet's next traversal, its end, or (guided) the wait for the network.  A call of its
+    // own, with the packet in LDS: its FP64 transcendentals need far more registers than the
+    // crossing loop, and inlined they spilled the loop's traversal state.
+    template<int GT, int V>
+    __device__ __attribute__((noinline)) void life_event(const SimParams* params, int phase, int last, double tau, double s,
+                                                         uint64_t hist, EventOut& out, LdsF64* cd, LdsU32* cu, LdsU32* lds,
+                                                         int t)
+    {
+        const SimParams& p = uniform_params(params);
+        EventOut io;
+        io.off = -1;
+        Packet pk;
+        Events<GT, V> E{p, io, pk, lds};
+        bool peels;
+        if (phase == kFetch)
+            peels = E.launch(hist);
+        else
+        {
+            pk.template load<V == kBatched>(cd, cu, t, p);
+            peels = E.transition(phase, last, tau, s);
+        }
+        if (peels) E.next_peel();
+        pk.store(cd, cu, t);
+        out = io;
+    }
+
+    // The guided scattering of one packet from the network outputs o (guided_scatter), likewise.
+    template<int GT>
+    __device__ __attribute__((noinline)) void life_guided(const SimParams* params, const float* o, EventOut& out,
+                                                          LdsF64* cd, LdsU32* cu, LdsU32* lds, int t)
+    {
+        const SimParams& p = uniform_params(params);
+        EventOut io;
+        io.off = -1;
+        Packet pk;
+        pk.template load<false>(cd, cu, t, p);
+        Events<GT, kGuided> E{p, io, pk, lds};
+        E.guided_scatter(o);
+        pk.store(cd, cu, t);
+        out = io;
+    }
+
     __device__ __forceinline__ int lane_id() { return __lane_id(); }
 
-// Minimum waves per SIMD of the persistent kernel on Cartesian and octree grids.  Two waves
-// give it 256 VGPRs: the event transitions (FP64 transcendentals on a loaded packet) need far
-// more than the crossing loop, and on the octree at three or four waves the register spills to
-// scratch cost more than the extra latency hiding gains.
-#ifndef SKG_LIFECYCLE_WAVES
-#define SKG_LIFECYCLE_WAVES 2
-#endif
-#ifndef SKG_LIFECYCLE_WAVES_CART
-#define SKG_LIFECYCLE_WAVES_CART 2
-#endif
-
-    // Minimum waves per SIMD per grid type.  The Voronoi and tetra kernels hold less
-    // traversal state and stage no octree nodes in LDS (35 KB per workgroup): measured on the
-    // clumpy Voronoi workload 1152 / 1086 / 1061 ms per 2^22-packet launch at 2 / 3 / 4 waves
-    // (each at its best transition threshold), on the batched tetra workload 6.72 / 5.80 /
-    // 5.27 s.  The octree kernel loses with a
-    // third wave (101.4 vs 142.5 ms per 2^22-packet launch on the spiral disk at tauV 50, the
-    // top-node table halved to fit three workgroups per CU: 168 VGPRs spill the traversal
-    // state), and the Cartesian one gains nothing (58.2 / 61.3 / 61.1 ms at 2 / 3 / 4 waves).
-    template<int GT> constexpr int lifecycle_waves()
+    // Minimum waves per SIMD, with the measured alternatives (ms at 2 / 3 / 4 waves):
+    //   Cartesian 64^3, 2^21 packets               25.1 / 23.0 / 22.4
+    //   octree disk, ten levels, tau_V 50, 2^21    50.1 / 43.3 / 46.0 (at four, spills around the
+    //   octree, nine levels, 40 wavelengths, 3e5    8.4 /  8.4 /  8.1  events double the writes)
+    //   octree with the radiation field, 2e5        7.8 / 11.6 / 13.2 (bound by its atomics, whose
+    //                                                  targets collide more with more waves)
+    // Voronoi and tetra as measured before the events became calls: 1152 / 1086 / 1061 ms and
+    // 6.72 / 5.80 / 5.27 s.  The guided variant's network call holds whole layers' weights in
+    // registers, and its four-wave build does not compile for the mesh grids.
+    template<int GT, int V> constexpr int lifecycle_waves()
     {
-        return GT == kTetra ? 4 : GT == kVoronoi ? 4 : GT == kCartesian ? SKG_LIFECYCLE_WAVES_CART : SKG_LIFECYCLE_WAVES;
+        return V == kGuided || V == kStoreRF ? 2 : GT == kOctree ? 3 : 4;
     }
 
     // The kernel's parameter block where it lies in the kernarg segment, behind a pointer the
@@ -785,47 +871,62 @@ namespace skg
     }
 
     template<int GT, int FP, int V>
-    __global__ void __launch_bounds__(kLcThreads, lifecycle_waves<GT>()) lifecycle(SimParams p)
+    __global__ void __launch_bounds__(kLcThreads, (lifecycle_waves<GT, V>())) lifecycle(SimParams p)
     {
-        constexpr bool INST = V == kBatched;
-        __shared__ unsigned int wgcnt[kNumCounters];
+        constexpr bool PERSP = V == kPersp || V == kStoreRF;
+        __shared__ uint32_t wgcnt[kNumCounters];
         __shared__ double coldD[kColdF64 * kLcThreads];
         __shared__ uint32_t coldU[kColdU32 * kLcThreads];
+        LdsF64* const cd = (LdsF64*)coldD;
+        LdsU32* const cu = (LdsU32*)coldU;
+        LdsU32* const cnt = (LdsU32*)wgcnt;
         if (threadIdx.x < kNumCounters) wgcnt[threadIdx.x] = 0;
-        if constexpr (GT == kOctree)
-            stage_top(p.grid);  // other grids allocate no top-node LDS (stage_top ends with a barrier)
-        else
-            __syncthreads();  // the counters are zero before any wave adds to them
+        stage_planes<GT>(p.grid);
+        __syncthreads();  // the counters are zero before any wave adds to them
         const int t = threadIdx.x;
-        Trav<GT, FP> T;
-        T.phase = kFetch;
-        T.ended = false;
-        Pending pd{-1, 0.};
         const int lane = lane_id();
+        Trav<GT, FP> T;
+        // the lanes that take packets (all of them unless the run is small); a lane without one
+        // waits in kFetch
+        T.phase = lane < p.lanes ? kFetch : kDone;
+        T.ended = false;
+        bool busy = false;  // the lane's traversal is under way
         while (true)
         {
-            // advance every busy lane by one cell crossing
-            bool busy = (T.phase == kPeel || T.phase == kFwd1 || T.phase == kFwd2) && !T.ended;
-            const SimParams& sp = kernel_params();
-            if (busy) T.template step<V == kStoreRF, V == kPersp || V == kStoreRF>(sp.grid, wgcnt, sp.rf, sp.nlambda);
-
-            // wave-wide transition round once enough lanes wait for an event (or, guided, for the
-            // network: lanes waiting to scatter call a round only once there are kGuideLanes of
-            // them, so that they do not call transition rounds with few events to handle)
-            const unsigned long long waiting = __ballot(T.ended || T.phase == kFetch);
-            const unsigned long long scatter = V == kGuided ? __ballot(T.phase == kScatter) : 0ull;
-            const unsigned long long active = __ballot(T.phase != kDone);
-            if (active == 0) break;
-            if (__popcll(waiting) >= sp.threshold || (waiting | scatter) == active
-                || (V == kGuided && __popcll(scatter) >= kGuideLanes))
+            // A transition round of the wave: events for the lanes whose traversal ended, new
+            // histories, the traversals that follow.
             {
                 const SimParams& kp = kernel_params();
-                if (T.ended)
+                EventOut io;
+                int64_t off = -1;  // this round's deposit
+                double v = 0.;
+                uint64_t hist = 0;
+                bool event = T.ended, go = false;
+                // new histories for the lanes without one, with one atomic per wavefront
+                const unsigned long long need = __ballot(T.phase == kFetch);
+                if (need)
                 {
-                    Packet pk;
-                    pk.load<INST>(coldD, coldU, t, kp);
-                    Events<GT, FP, V>{kp, T, pk, wgcnt, pd}.transition();
-                    pk.store(coldD, coldU, t);
+                    const int leader = __ffsll(static_cast<long long>(need)) - 1;
+                    unsigned long long base = 0;
+                    if (lane == leader) base = atomicAdd(kp.queue, static_cast<unsigned long long>(__popcll(need)));
+                    base = __shfl(base, leader);
+                    if (T.phase == kFetch)
+                    {
+                        const unsigned long long mine = base + __popcll(need & ((1ull << lane) - 1ull));
+                        hist = kp.first + mine;
+                        event = mine < kp.count;
+                        if (!event) T.phase = kDone;
+                    }
+                }
+                if (event)
+                {
+                    life_event<GT, V>(&kp, T.phase, T.last, T.tau_value(), T.s_end(T.tau_value() > T.lim), hist, io, cd, cu,
+                                      cnt, t);
+                    off = io.off;
+                    v = io.v;
+                    T.phase = io.phase;
+                    T.ended = false;
+                    go = io.phase == kPeel || io.phase == kFwd1 || io.phase == kFwd2;
                 }
                 if constexpr (V == kGuided)
                 {
@@ -833,50 +934,49 @@ namespace skg
                     // there are kGuideLanes of them or no lane of the wave is still traversing
                     const bool sc = T.phase == kScatter;
                     const unsigned long long scm = __ballot(sc);
-                    const unsigned long long trav =
-                        __ballot((T.phase == kPeel || T.phase == kFwd1 || T.phase == kFwd2) && !T.ended);
-                    if (scm && (__popcll(scm) >= kGuideLanes || trav == 0))
+                    if (scm && (__popcll(scm) >= kGuideLanes || __ballot(go || busy) == 0))
                     {
-                        Packet pk;
                         float feat[kGuideIn];
                         for (int q = 0; q < kGuideIn; ++q) feat[q] = 0.f;
                         if (sc)
-                        {
-                            pk.load<false>(coldD, coldU, t, kp);
-                            guide_features(kp.gframe, pk.rx, pk.ry, pk.rz, pk.kx, pk.ky, pk.kz, pk.lam, feat);
-                        }
+                            guide_features(kp.gframe, cd[cRx * kLcThreads + t], cd[cRy * kLcThreads + t],
+                                           cd[cRz * kLcThreads + t], cd[cKx * kLcThreads + t], cd[cKy * kLcThreads + t],
+                                           cd[cKz * kLcThreads + t], cd[cLam * kLcThreads + t], feat);
                         float o[kGuideOut];
                         guide_wave_infer_regs(kp.net, feat, sc, o);
                         if (sc)
                         {
-                            Events<GT, FP, V>{kp, T, pk, wgcnt, pd}.guided_scatter(o);
-                            pk.store(coldD, coldU, t);
+                            life_guided<GT>(&kp, o, io, cd, cu, cnt, t);
+                            T.phase = io.phase;
+                            go = true;
                         }
                     }
                 }
-                unsigned long long need = __ballot(T.phase == kFetch);
-                if (need)
+                flush_deposits(kp.frame, off, v, cnt);  // the wave is converged here
+                if (go)
                 {
-                    int cntNeed = __popcll(need);
-                    int leader = __ffsll(static_cast<long long>(need)) - 1;
-                    unsigned long long base = 0;
-                    if (lane == leader) base = atomicAdd(kp.queue, static_cast<unsigned long long>(cntNeed));
-                    base = __shfl(base, leader);
-                    if (T.phase == kFetch)
-                    {
-                        unsigned long long below = need & ((1ull << lane) - 1ull);
-                        unsigned long long mine = base + __popcll(below);
-                        if (mine < kp.count)
-                        {
-                            Packet pk;
-                            Events<GT, FP, V>{kp, T, pk, wgcnt, pd}.launch(kp.first + mine);
-                            pk.store(coldD, coldU, t);
-                        }
-                        else
-                            T.phase = kDone;
-                    }
+                    T.template start<PERSP>(kp.grid, io, cd, cu, cnt, t);
+                    busy = !T.ended;
                 }
-                flush_deposits(kp.frame, pd, wgcnt);  // the wave is converged here
+            }
+            // Crossings until enough lanes wait for a round.  The threshold is a share of the lanes
+            // that still take part: in a small run, and at the end of every run, a fixed number of
+            // waiting lanes would never come together and each packet would wait for the longest
+            // traversal of the wave.  Guided: the lanes that wait for the network do not count as
+            // waiting (they call no round with few events to handle).  A loop of its own, so that
+            // the registers' spills lie outside it.
+            const SimParams& sp = kernel_params();
+            const int nact = __popcll(__ballot(T.phase != kDone));
+            if (nact == 0) break;
+            const int nscat = V == kGuided ? __popcll(__ballot(T.phase == kScatter)) : 0;
+            const int stop = max(0, nact - nscat - ((sp.threshold * nact + 63) >> 6));
+            while (__popcll(__ballot(busy)) > stop)
+            {
+                if (busy)
+                {
+                    T.template step<V == kStoreRF, PERSP>(kernel_params().grid, cnt, kernel_params().rf, kernel_params().nlambda);
+                    busy = !T.ended;
+                }
             }
         }
         // workgroup event counters to the global counters

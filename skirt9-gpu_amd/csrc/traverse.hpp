@@ -75,42 +75,40 @@ namespace skg
     // valid geometry (such as a non-finite position).
     constexpr int kMaxNoExit = 4096;
 
-    // One 128-byte record per octree leaf (indexed by cell): everything a cell crossing
-    // reads -- the leaf's FP64 bounds, its number density, the first (largest-overlap)
-    // neighbour on each wall and the start of each wall's full neighbour list -- sits in one
-    // cache line, so the common crossing (the first neighbour contains the new position)
-    // touches a single line.
-    struct alignas(128) OctLeaf
+    // One 64-byte record per octree node, indexed by node id.  A leaf holds everything a cell
+    // crossing reads: its bounds, number density, cell index and, per wall, the node across it.  An
+    // inner node holds its bounds, its first child and its split point (the upper corner of the first
+    // child, TreeNode::leafChild's test point).  Bounds and split points are indices into the table
+    // of the tree's distinct coordinates (GridView::planes, 3075 FP64 values for ten levels), which
+    // the kernels keep in LDS: a crossing reads half a cache line instead of a whole one, two
+    // siblings share a line, and the 3.4e6 nodes of the spiral disk take 215 MB, less than the
+    // last-level cache, instead of 430 MB.
+    //
+    // first[w] of a leaf: the neighbour itself where one leaf covers the wall; where several
+    // smaller ones do, the node of the leaf's own size that they subdivide, so that a crossing
+    // into a finer region descends by the split points (one record per level) instead of testing
+    // the wall's list entry by entry; kOctNoNb at the domain boundary; kOctList where the table's
+    // list is neither of these (the crossing then walks it).
+    struct alignas(64) OctNode
     {
-        double lo[3], hi[3];  // bounds
-        double dens;          // number density of the cell
-        int32_t node;         // node id in the full tree
-        int32_t off_end;      // end of this leaf's neighbour lists in nbc
-        int32_t first[6];     // first neighbour cell per wall (BACK..TOP), -1 if none
-        int32_t off[6];       // start of each wall's neighbour list in nbc
-        int32_t pad[4];
+        int32_t lo[3], hi[3];  // bounds (planes)
+        union
+        {
+            int32_t first[6];  // leaf: node across each wall (BACK..TOP)
+            int32_t split[3];  // inner: split point (planes)
+        };
+        double dens;   // leaf: number density of the cell
+        int32_t cell;  // leaf: cell index; inner: ~first child (children are 8 consecutive ids)
+        int32_t pad;
     };
-    static_assert(sizeof(OctLeaf) == 128, "leaf record must be one 128-byte line");
+    static_assert(sizeof(OctNode) == 64, "node record must be half a cache line");
+    static_assert(offsetof(OctNode, first) == 24 && offsetof(OctNode, dens) == 48 && offsetof(OctNode, cell) == 56,
+                  "node record layout that OctRec reads");
+    constexpr int32_t kOctNoNb = -1, kOctList = -2;
+    constexpr int kLdsPlanes = 3200;  // coordinates kept in LDS at most (25.6 KB): ten levels have 3075
 
-    // An octree node in the form the top-down search reads (one 32-byte record per level): the
-    // split point (upper corner of the first child, TreeNode::leafChild's test point) and the
-    // first child id, or for a leaf (child -1) its cell index.  The records of the top levels
-    // are also staged in LDS.
-    struct TopNode
-    {
-        double sx, sy, sz;
-        int32_t child;
-        int32_t cell;
-    };
-    static_assert(sizeof(TopNode) == 32, "top node must be 32 bytes");
-#ifndef SKG_TOP_NODES
-#define SKG_TOP_NODES 1024
-#endif
-    constexpr int kTopNodes = SKG_TOP_NODES;  // 1024: 32 KB of LDS, levels 0-3 of a full octree and part of level 4
-
-    // Read-only grid tables resident in HBM.  Octree: the node records of the top-down search
-    // (TopNode, children are 8 consecutive ids), the cell-indexed leaf records and their
-    // neighbour lists (cell ids, sorted by decreasing overlap as TreeNode::sortNeighbors).
+    // Read-only grid tables resident in HBM.  Octree: the node records and the leaves' neighbour
+    // lists (node ids, sorted by decreasing overlap as TreeNode::sortNeighbors).
     struct GridView
     {
         double box[6];  // xmin, ymin, zmin, xmax, ymax, zmax of the domain
@@ -120,10 +118,12 @@ namespace skg
         const double* zb;
         int nx, ny, nz;
         const double* dens;  // Cartesian: number density per cell
-        const OctLeaf* leaf;
+        const OctNode* node;
+        const double* planes;   // the distinct coordinates of the tree's bounds
+        int nplanes;
+        int ldsPlanes;          // nonzero: the kernel staged them in LDS (stage_planes)
+        const int32_t* nbOff;   // start of each node's and wall's neighbour list (6 per node, and the end)
         const int32_t* nbc;
-        const TopNode* top;  // every node in TopNode form, indexed by node id
-        int topN;            // nodes with id < topN are staged in LDS (0: none, non-octree grids)
         // Voronoi: cell records, neighbour entries and the block search lists (CSR over vbn^3
         // blocks of cell ids, in the reference's order)
         const VorCell* vcell;
@@ -311,18 +311,6 @@ namespace skg
         return x >= b[0] && x <= b[3] && y >= b[1] && y <= b[4] && z >= b[2] && z <= b[5];
     }
 
-    // The top of the octree staged in LDS for the top-down search every path start makes:
-    // for node ids below GridView::topN, the split point (upper corner of the first child) and
-    // the first child id.  Every kernel that walks an octree fills it with stage_top() first;
-    // with topN = 0 the search reads only global memory.
-    __shared__ TopNode skg_top_lds[kTopNodes];
-
-    __device__ __forceinline__ void stage_top(const GridView& g)
-    {
-        for (int t = threadIdx.x; t < g.topN; t += blockDim.x) skg_top_lds[t] = g.top[t];
-        __syncthreads();
-    }
-
     // a ? x : b ? y : z on values (selecting among members by reference would make the
     // compiler select their addresses and keep the generator in scratch memory)
     template<typename T> __device__ __forceinline__ T pick3(bool a, bool b, T x, T y, T z)
@@ -331,48 +319,162 @@ namespace skg
         return a ? x : yz;
     }
 
-    // What the octree generator's next advance() call loads and does with the record.  Every
-    // call makes at most one dependent global load (a leaf record, a search node or a
-    // neighbour-list entry), so lanes of a wavefront in different phases share one memory
-    // round trip per call instead of the wave waiting for each lane's chain of loads.
-    enum OctStep : int
+    // a / b for a correctly rounded reciprocal y = RN(1 / b): the product with y, one Newton step
+    // that makes the quotient faithful, and Markstein's correction with the exact remainder, which
+    // gives the correctly rounded quotient -- the same value as the division (P. Markstein, IBM
+    // J. Res. Dev. 34, 1990), in five FP64 operations instead of the division's eleven.  Positions
+    // and directions along a path share the three divisors, so y is made once per path.
+    __device__ __forceinline__ double quotient(double a, double b, double y)
     {
-        kOsStart = 0,     // enter the domain, then the start hint's record (or the search)
-        kOsCross = 1,     // the crossing of the current leaf, then the wall's first neighbour
-        kOsListStart = 2, // the current leaf's record again: the wall's neighbour-list range
-        kOsListId = 3,    // a neighbour-list entry (cell id)
-        kOsListRec = 4,   // that neighbour's record
-        kOsNode = 5,      // a search node below the LDS-staged levels
-        kOsLeaf = 6,      // the record of the leaf the search found
-        kOsEnd = 7,       // no more segments
-        kOsSearch = 8     // (a step's action only) the search from the root after a load of no use:
-                          // a start without hint, a wall on the domain boundary
+        double q = a * y;
+        q = fma(fma(-b, q, a), y, q);
+        return fma(fma(-b, q, a), y, q);
+    }
+
+    // The octree's coordinate table in LDS (dynamic shared memory of nplanes doubles when
+    // GridView::ldsPlanes is set); every kernel that walks an octree calls stage_planes first.
+    extern __shared__ double skg_planes[];
+
+    template<int GT> __device__ __forceinline__ void stage_planes(const GridView& g)
+    {
+        if constexpr (GT == kOctree)
+        {
+            if (g.ldsPlanes)
+                for (int t = threadIdx.x; t < g.nplanes; t += blockDim.x) skg_planes[t] = g.planes[t];
+            __syncthreads();
+        }
+    }
+
+    // What a crossing reads of an octree node's record, in registers (no member is selected by
+    // reference, which would leave the record in scratch memory)
+    struct OctRec
+    {
+        int4 a, b, c, d;
+        __device__ __forceinline__ void load(const OctNode* nd)
+        {
+            const int4* p = reinterpret_cast<const int4*>(nd);
+            a = p[0];
+            b = p[1];
+            c = p[2];
+            d = p[3];
+        }
+        __device__ __forceinline__ int cell() const { return d.z; }
+        __device__ __forceinline__ double dens() const { return __hiloint2double(d.y, d.x); }
     };
+
+    // bounds of a node
+    struct OctBox
+    {
+        double x0, y0, z0, x1, y1, z1;
+        __device__ __forceinline__ void load(const GridView& g, const OctRec& R)
+        {
+            if (g.ldsPlanes)
+            {
+                x0 = skg_planes[R.a.x];
+                y0 = skg_planes[R.a.y];
+                z0 = skg_planes[R.a.z];
+                x1 = skg_planes[R.a.w];
+                y1 = skg_planes[R.b.x];
+                z1 = skg_planes[R.b.y];
+            }
+            else
+            {
+                x0 = g.planes[R.a.x];
+                y0 = g.planes[R.a.y];
+                z0 = g.planes[R.a.z];
+                x1 = g.planes[R.a.w];
+                y1 = g.planes[R.b.x];
+                z1 = g.planes[R.b.y];
+            }
+        }
+        __device__ __forceinline__ bool closed_contains(double x, double y, double z) const
+        {
+            return x >= x0 && x <= x1 && y >= y0 && y <= y1 && z >= z0 && z <= z1;
+        }
+    };
+
+    // TreeNode::leafChild from the root (TreeSpatialGrid.cpp:190-219, OctTreeNode.cpp:37-42): the
+    // leaf containing the position by the half-open rule of the split points, -1 outside the
+    // root's closed box
+    __device__ __forceinline__ int oct_search(const OctNode* node, const double* planes, double x, double y, double z)
+    {
+        if (!(x >= planes[node->lo[0]] && x <= planes[node->hi[0]] && y >= planes[node->lo[1]]
+              && y <= planes[node->hi[1]] && z >= planes[node->lo[2]] && z <= planes[node->hi[2]]))
+            return -1;
+        int nd = 0;
+        while (true)
+        {
+            const OctNode& N = node[nd];
+            const int c = N.cell;
+            if (c >= 0) return nd;
+            nd = ~c + (x < planes[N.split[0]] ? 0 : 1) + (y < planes[N.split[1]] ? 0 : 2)
+                 + (z < planes[N.split[2]] ? 0 : 4);
+        }
+    }
+
+    struct OctNext
+    {
+        int node;
+        double x, y, z;
+    };
+
+    // The next leaf after a crossing of wall `wall` of leaf i at the position (x, y, z), by the
+    // reference's own sequence (TreeSpatialGrid.cpp:184-219): the wall's neighbour list in order,
+    // then the search from the root, then, still in leaf i, the same search with the position one
+    // ulp further along the path; node -1 where the path ends.  Called where the crossing's shorter
+    // rules do not decide (a position on a split plane or outside the node across the wall), and
+    // kept out of the crossing's registers.
+    __device__ __attribute__((noinline)) OctNext oct_next_exact(const OctNode* node, const double* planes,
+                                                                const int32_t* nbOff, const int32_t* nbc, int i, int wall,
+                                                                double x, double y, double z, double kx, double ky,
+                                                                double kz)
+    {
+        int c = -2;
+        const int64_t at = 6 * static_cast<int64_t>(i) + wall;
+        for (int q = nbOff[at], e = nbOff[at + 1]; q < e; ++q)
+        {
+            const int id = nbc[q];
+            const OctNode& N = node[id];
+            if (x >= planes[N.lo[0]] && x <= planes[N.hi[0]] && y >= planes[N.lo[1]] && y <= planes[N.hi[1]]
+                && z >= planes[N.lo[2]] && z <= planes[N.hi[2]])
+            {
+                c = id;
+                break;
+            }
+        }
+        if (c == -2) c = oct_search(node, planes, x, y, z);
+        if (c == i)
+        {
+            x = nextafter(x, (kx < 0.) ? -DBL_MAX : DBL_MAX);
+            y = nextafter(y, (ky < 0.) ? -DBL_MAX : DBL_MAX);
+            z = nextafter(z, (kz < 0.) ? -DBL_MAX : DBL_MAX);
+            c = oct_search(node, planes, x, y, z);
+        }
+        return OctNext{c == i ? -1 : c, x, y, z};
+    }
 
     template<int GT> struct Gen
     {
         double rx, ry, rz, kx, ky, kz;
         int state;
-        int i, j, k;  // Cartesian cell indices; octree, Voronoi, tetra: i = current cell
-                      // (tetra: j = entering face, -1 if unknown; Voronoi: j = the header slot
-                      // of the cell's run in the entry table)
-        double sx, sy, sz;  // Voronoi: the current cell's site
+        int i, j, k;  // Cartesian cell indices; octree: i = current leaf's node; Voronoi, tetra: i =
+                      // current cell (tetra: j = entering face, -1 if unknown; Voronoi: j = the
+                      // header slot of the cell's run in the entry table)
+        double sx, sy, sz;      // Voronoi: the current cell's site
+        double ikx, iky, ikz;   // Cartesian, octree: reciprocals of the direction
         double b0, b1, b2, bn;  // octree: the current cell's wall ahead on each axis, its density
-        int f0, f1, f2;         // octree: the first neighbour across each of those walls
-        int hint;  // octree, Voronoi, tetra: a cell that probably contains the start point (-1:
-                   // none); after the first step, the start cell
-        // octree step machine (advance): the next step, the crossed wall, a candidate cell,
-        // the neighbour-list cursor and end, the search node, and the flags for the start
-        // search and the nextafter retry (TreeSpatialGrid.cpp:210-215)
-        int ost, wall, cand, q, qe, node;
-        bool locating, na;
-        float rkx, rky, rkz;  // FP32 reciprocals of the direction, for the exit-axis estimates
+        int f0, f1, f2;         // octree: the node across each of those walls
+        int cell;               // octree: the current leaf's cell index
+        uint32_t pend;  // octree: a node to descend into next and the crossed wall (node << 3 | wall),
+                        // or kNoPend
+        int hint;  // octree (a node), Voronoi, tetra: a cell that probably contains the start point
+                   // (-1: none); after the first step, the start cell
+        static constexpr uint32_t kNoPend = 0xFFFFFFFFu;  // node ids stay below 2^29
 
         __device__ __forceinline__ void start(double r0, double r1, double r2, double k0, double k1, double k2,
                                               int start_hint = -1)
         {
             hint = start_hint;
-            ost = kOsStart;
             rx = r0;
             ry = r1;
             rz = r2;
@@ -448,486 +550,267 @@ namespace skg
             return true;
         }
 
-        // ---------------------------------------------------------------- octree step machine
-        // The record fields a step reads, from the 112 bytes it loads (an OctLeaf, a TopNode or
-        // neighbour-list entries; the tables are padded so that 112 bytes past any entry stay
-        // inside them)
-        struct RawRec
-        {
-            // the 112 bytes as 14 doubles in registers (plain scalars: no member is selected by
-            // reference, which would leave the record in scratch memory)
-            double q0, q1, q2, q3, q4, q5, q6, q7, q8, q9, q10, q11, q12, q13;
-            __device__ __forceinline__ void load(const char* addr)
-            {
-                const double* p = reinterpret_cast<const double*>(addr);
-                q0 = p[0];
-                q1 = p[1];
-                q2 = p[2];
-                q3 = p[3];
-                q4 = p[4];
-                q5 = p[5];
-                q6 = p[6];
-                q7 = p[7];
-                q8 = p[8];
-                q9 = p[9];
-                q10 = p[10];
-                q11 = p[11];
-                q12 = p[12];
-                q13 = p[13];
-                // the words only the neighbour-list states use (node / off_end and the walls'
-                // list starts) are marked as needed here: the compiler would otherwise issue
-                // their loads inside those states, after the wait for the first words, and the
-                // step would read the line twice in a row (101.6 -> 99.6 ms per 2^22-packet
-                // launch on the spiral disk at tauV 50 with all of it issued at once)
-                asm volatile("" : "+v"(q7), "+v"(q11), "+v"(q12), "+v"(q13));
-            }
-            // double k (bytes 8k..8k+7), k a compile-time constant
-            __device__ __forceinline__ double d(int k) const
-            {
-                switch (k)
-                {
-                    case 0: return q0;
-                    case 1: return q1;
-                    case 2: return q2;
-                    case 3: return q3;
-                    case 4: return q4;
-                    case 5: return q5;
-                    case 6: return q6;
-                    case 7: return q7;
-                    case 8: return q8;
-                    case 9: return q9;
-                    case 10: return q10;
-                    case 11: return q11;
-                    case 12: return q12;
-                    default: return q13;
-                }
-            }
-            // int k (bytes 4k..4k+3), k a compile-time constant
-            __device__ __forceinline__ int i32(int k) const
-            {
-                const double v = d(k >> 1);
-                return (k & 1) ? __double2hiint(v) : __double2loint(v);
-            }
-            // the entry r (run time) of the first four ints
-            __device__ __forceinline__ int first4(int r) const
-            {
-                const int e0 = __double2loint(q0), e1 = __double2hiint(q0), e2 = __double2loint(q1),
-                          e3 = __double2hiint(q1);
-                const int e23 = r == 2 ? e2 : e3;
-                const int e123 = r == 1 ? e1 : e23;
-                return r == 0 ? e0 : e123;
-            }
-            // OctLeaf::off[wl] (ints 22..27) and the end of the wall's list (the next wall's
-            // start, or off_end, int 15, after the last wall), wl at run time
-            __device__ __forceinline__ int off_at(int wl) const
-            {
-                const int o0 = __double2loint(q11), o1 = __double2hiint(q11), o2 = __double2loint(q12),
-                          o3 = __double2hiint(q12), o4 = __double2loint(q13), o5 = __double2hiint(q13);
-                return pick6(wl, o0, o1, o2, o3, o4, o5);
-            }
-            __device__ __forceinline__ int off_end_at(int wl) const
-            {
-                const int o1 = __double2hiint(q11), o2 = __double2loint(q12), o3 = __double2hiint(q12),
-                          o4 = __double2loint(q13), o5 = __double2hiint(q13), oe = __double2hiint(q7);
-                return pick6(wl, o1, o2, o3, o4, o5, oe);
-            }
-            __device__ __forceinline__ static int pick6(int w, int a, int b, int c, int d, int e, int f)
-            {
-                const int ef = w == 4 ? e : f;
-                const int def = w == 3 ? d : ef;
-                const int cdef = w == 2 ? c : def;
-                const int bcdef = w == 1 ? b : cdef;
-                return w == 0 ? a : bcdef;
-            }
-        };
-        // OctLeaf: lo/hi doubles 0..5, dens double 6, node int 14, off_end int 15, first ints
-        // 16..21, off ints 22..27.  TopNode: split point doubles 0..2, child int 6, cell int 7.
-        static_assert(offsetof(OctLeaf, dens) == 48 && offsetof(OctLeaf, off_end) == 60 && offsetof(OctLeaf, first) == 64
-                          && offsetof(OctLeaf, off) == 88,
-                      "leaf record layout the step machine reads");
-        static_assert(offsetof(TopNode, child) == 24 && offsetof(TopNode, cell) == 28, "node layout the step machine reads");
-
-        // the leaf c becomes the current cell: of its record, the crossing needs only the wall
+        // ---------------------------------------------------------------- octree
+        // the leaf nd becomes the current one: of its record, the crossing needs only the wall
         // ahead on each axis (the direction does not change along a path) -- its coordinate
-        // (TreeSpatialGrid.cpp:157-159) and its first neighbour -- and the density
-        __device__ __forceinline__ void adopt(const RawRec& R, int c)
+        // (TreeSpatialGrid.cpp:157-159) and the node across it -- the density and the cell
+        __device__ __forceinline__ void adopt(const OctRec& R, const OctBox& B, int nd)
         {
-            i = c;
-            b0 = (kx < 0.0) ? R.d(0) : R.d(3);
-            b1 = (ky < 0.0) ? R.d(1) : R.d(4);
-            b2 = (kz < 0.0) ? R.d(2) : R.d(5);
-            bn = R.d(6);
-            f0 = (kx < 0.0) ? R.i32(16) : R.i32(17);
-            f1 = (ky < 0.0) ? R.i32(18) : R.i32(19);
-            f2 = (kz < 0.0) ? R.i32(20) : R.i32(21);
-            ost = kOsCross;
+            i = nd;
+            cell = R.cell();
+            b0 = (kx < 0.0) ? B.x0 : B.x1;
+            b1 = (ky < 0.0) ? B.y0 : B.y1;
+            b2 = (kz < 0.0) ? B.z0 : B.z1;
+            bn = R.dens();
+            f0 = (kx < 0.0) ? R.b.z : R.b.w;
+            f1 = (ky < 0.0) ? R.c.x : R.c.y;
+            f2 = (kz < 0.0) ? R.c.z : R.c.w;
+            pend = kNoPend;
         }
 
-        __device__ __forceinline__ static bool closed_contains(const RawRec& R, double x, double y, double z)
+        // the start leaf: the hint, when the point lies in its box the way the top-down search
+        // assigns points to leaves -- lo <= r < hi on each axis (a point on a split plane goes to
+        // the upper child), hi included at the domain's upper boundary, so that every split plane
+        // of the leaf's ancestors sends the search toward it -- else the search's leaf
+        __device__ __forceinline__ bool oct_begin(const GridView& g)
         {
-            return x >= R.d(0) && x <= R.d(3) && y >= R.d(1) && y <= R.d(4) && z >= R.d(2) && z <= R.d(5);
-        }
-
-        // TreeNode::leafChild (TreeSpatialGrid.cpp:190-219, OctTreeNode.cpp:37-42) from node nd
-        // through the LDS-staged levels, with no global load: the cell of the leaf containing r
-        // (-1 outside the root's closed box), or -2 with the first node below the staged levels
-        // in `node`, whose record a later step loads
-        __device__ __forceinline__ int search_lds(const GridView& g, int nd)
-        {
-            if (nd == 0
-                && !(rx >= g.box[0] && rx <= g.box[3] && ry >= g.box[1] && ry <= g.box[4] && rz >= g.box[2]
-                     && rz <= g.box[5]))
-                return -1;
-            while (nd < g.topN)
+            OctRec R;
+            OctBox B;
+            int nd = hint;
+            bool found = false;
+            if (nd >= 0)
             {
-                const TopNode t = skg_top_lds[nd];
-                if (t.child < 0) return t.cell;
-                nd = t.child + (rx < t.sx ? 0 : 1) + (ry < t.sy ? 0 : 2) + (rz < t.sz ? 0 : 4);
+                R.load(g.node + nd);
+                B.load(g, R);
+                const bool inx = rx >= B.x0 && (rx < B.x1 || B.x1 == g.box[3]);
+                const bool iny = ry >= B.y0 && (ry < B.y1 || B.y1 == g.box[4]);
+                const bool inz = rz >= B.z0 && (rz < B.z1 || B.z1 == g.box[5]);
+                found = inx && iny && inz;
             }
-            node = nd;
-            return -2;
-        }
-
-        // a search result c (-2: the search continues at `node`).  Starting a path, c is the
-        // start cell.  After a crossing, c is the next cell unless it is the current one: then
-        // the position moves by one ulp toward the direction and the search is made once more;
-        // outside, or still the current cell, the path ends (TreeSpatialGrid.cpp:204-218).
-        __device__ __forceinline__ void resolve(const GridView& g, int c)
-        {
-            if (c == -2)
+            if (!found)
             {
-                ost = kOsNode;
-                return;
+                nd = oct_search(g.node, g.planes, rx, ry, rz);
+                if (nd < 0) return false;
+                R.load(g.node + nd);
+                B.load(g, R);
             }
-            if (!locating && c == i && !na)
-            {
-                na = true;
-                rx = nextafter(rx, (kx < 0.) ? -DBL_MAX : DBL_MAX);
-                ry = nextafter(ry, (ky < 0.) ? -DBL_MAX : DBL_MAX);
-                rz = nextafter(rz, (kz < 0.) ? -DBL_MAX : DBL_MAX);
-                c = search_lds(g, 0);
-                if (c == -2)
-                {
-                    ost = kOsNode;
-                    return;
-                }
-            }
-            // the same members are written on both outcomes (as values), so that the compiler
-            // keeps them in registers
-            const bool end = c < 0 || (!locating && c == i);
-            ost = end ? kOsEnd : kOsLeaf;
-            state = end ? kOutside : state;
-            cand = end ? cand : c;
+            adopt(R, B, nd);
+            hint = nd;
+            return true;
         }
 
         // One step of the octree generator (TreeSpatialGrid::MySegmentGenerator::next,
-        // TreeSpatialGrid.cpp:143-228, split so that a step makes at most one dependent global
-        // load): 1 with the segment (m, ds, n) when the step completed one, 2 with the path's last
-        // segment (the path ends after it), 0 when it only progressed (a start, a neighbour-list
-        // entry, a search level), -1 at the end of the path.  The sequence of segments equals
-        // next()'s.
-        __device__ __forceinline__ int advance_octree(const GridView& g, int& m, double& ds, double& n)
+        // TreeSpatialGrid.cpp:143-228), with one dependent record load: the crossing of the current
+        // leaf and the record of the node across the exit wall, or one level of the descent into a
+        // finer region.  Returns as cross() does.
+        __device__ __forceinline__ int cross_octree(const GridView& g, int& m, double& ds, double& n)
         {
             int out = 0;
-            int act = ost;
-            const char* addr = nullptr;
-            // phase 1: the step's own computation and the address of the record it needs
-            if (ost == kOsEnd) return -1;
-            if (ost == kOsStart)
+            int nd = static_cast<int>(pend >> 3), wall = static_cast<int>(pend & 7u);
+            if (pend == kNoPend)
             {
-                double cumds;
-                if (!move_inside(g, cumds))
-                {
-                    ost = kOsEnd;
-                    return -1;
-                }
-                locating = true;
-                na = false;
-                rkx = 1.f / static_cast<float>(kx);
-                rky = 1.f / static_cast<float>(ky);
-                rkz = 1.f / static_cast<float>(kz);
-                if (cumds > 0.)
-                {
-                    m = -1;
-                    ds = cumds;
-                    n = 0.;
-                    out = 1;
-                }
-                act = hint >= 0 ? kOsStart : kOsSearch;  // the hint's record follows, or the search
-            }
-            else if (ost == kOsCross)
-            {
-                const int cur = i;
-                // The exit distance along each axis to the wall ahead (b0..b2, from adopt):
-                // (wall - r) / k, or DBL_MAX for a component within 1e-15 of zero, and the
-                // smallest wins with the ties of TreeSpatialGrid.cpp:157-181 (x if dsx <= dsy &&
-                // dsx <= dsz, y if dsy <= dsx && dsy <= dsz, else z).  FP32 estimates (relative
-                // error below 3e-7) pick the axis when the two smallest differ by more than 1e-6
-                // of their size: the exact FP64 quotients then order the same way and differ,
-                // so only the winner's is computed (one FP64 division instead of three).  Close
-                // estimates, infinities and NaNs take the three exact quotients.
-                const double dx = b0 - rx, dy = b1 - ry, dz = b2 - rz;
-                const bool tx = fabs(kx) > 1e-15, ty = fabs(ky) > 1e-15, tz = fabs(kz) > 1e-15;
-                const float ex = tx ? static_cast<float>(dx) * rkx : INFINITY;
-                const float ey = ty ? static_cast<float>(dy) * rky : INFINITY;
-                const float ez = tz ? static_cast<float>(dz) * rkz : INFINITY;
-                const bool fx = ex <= ey && ex <= ez;
-                const bool fy = !fx && ey <= ez;
-                const float e1 = pick3(fx, fy, ex, ey, ez);
-                const float e2 = pick3(fx, fy, fminf(ey, ez), fminf(ex, ez), fminf(ex, ey));
-                const bool clear = e2 - e1 > 1e-6f * (fabsf(e1) + fabsf(e2));  // false for inf / NaN
-                bool ax, ay;
-                double d;
-                if (clear)
-                {
-                    ax = fx;
-                    ay = fy;
-                    d = pick3(ax, ay, dx, dy, dz) / pick3(ax, ay, kx, ky, kz);
-                }
-                else
-                {
-                    const double dsx = tx ? dx / kx : DBL_MAX;
-                    const double dsy = ty ? dy / ky : DBL_MAX;
-                    const double dsz = tz ? dz / kz : DBL_MAX;
-                    ax = dsx <= dsy && dsx <= dsz;
-                    ay = !ax && dsy <= dsx && dsy <= dsz;
-                    d = pick3(ax, ay, dsx, dsy, dsz);
-                }
+                // exit distance along each axis to the wall ahead, (wall - r) / k, or DBL_MAX for a
+                // component within 1e-15 of zero; the smallest wins with the ties of
+                // TreeSpatialGrid.cpp:157-181
+                const double dsx = fabs(kx) > 1e-15 ? quotient(b0 - rx, kx, ikx) : DBL_MAX;
+                const double dsy = fabs(ky) > 1e-15 ? quotient(b1 - ry, ky, iky) : DBL_MAX;
+                const double dsz = fabs(kz) > 1e-15 ? quotient(b2 - rz, kz, ikz) : DBL_MAX;
+                const bool ax = dsx <= dsy && dsx <= dsz;
+                const bool ay = !ax && dsy <= dsx && dsy <= dsz;
+                const double d = pick3(ax, ay, dsx, dsy, dsz);
                 wall = pick3(ax, ay, (kx < 0.0) ? 0 : 1, (ky < 0.0) ? 2 : 3, (kz < 0.0) ? 4 : 5);
-                const int f = pick3(ax, ay, f0, f1, f2);
-                double step = d + g.eps;
+                nd = pick3(ax, ay, f0, f1, f2);
+                const double step = d + g.eps;
                 rx += kx * step;
                 ry += ky * step;
                 rz += kz * step;
-                m = cur;
+                m = cell;
                 ds = d;
                 n = bn;
                 out = 1;
-                locating = false;
-                na = false;
-                cand = f;
-                act = f >= 0 ? kOsCross : kOsSearch;  // the first neighbour's record follows, or the search
                 // a wall without neighbours is on the domain's boundary: outside the root's closed
                 // box the search finds no leaf (TreeNode::leafChild), and the path ends here
-                if (f < 0 && !(rx >= g.box[0] && rx <= g.box[3] && ry >= g.box[1] && ry <= g.box[4] && rz >= g.box[2]
-                               && rz <= g.box[5]))
+                if (nd == kOctNoNb
+                    && !(rx >= g.box[0] && rx <= g.box[3] && ry >= g.box[1] && ry <= g.box[4] && rz >= g.box[2]
+                         && rz <= g.box[5]))
                 {
-                    ost = kOsEnd;
                     state = kOutside;
                     return 2;
                 }
             }
-            // one search for all lanes that need it, after the step's load (a start without hint
-            // and a wall on the domain boundary load a record they do not use, so that the search
-            // is written once, in phase 3)
-            switch (act)
+            OctRec R;
+            OctBox B;
+            R.load(g.node + max(nd, 0));
+            B.load(g, R);
+            const bool closed = nd >= 0 && B.closed_contains(rx, ry, rz);
+            const int c = R.cell();
+            if (__builtin_expect(closed && c >= 0, 1))
             {
-                case kOsSearch: addr = reinterpret_cast<const char*>(g.leaf); break;
-                case kOsStart: addr = reinterpret_cast<const char*>(g.leaf + hint); break;
-                case kOsCross:
-                case kOsListRec:
-                case kOsLeaf: addr = reinterpret_cast<const char*>(g.leaf + cand); break;
-                case kOsListStart: addr = reinterpret_cast<const char*>(g.leaf + i); break;
-                case kOsListId: addr = reinterpret_cast<const char*>(g.nbc + (q & ~3)); break;
-                default: addr = reinterpret_cast<const char*>(g.top + node); break;  // kOsNode
+                // the neighbour contains the new position (TreeNode::neighbor, TreeNode.cpp:103-112)
+                adopt(R, B, nd);
+                return out;
             }
-            // phase 2: the one load of this step
-            RawRec R;
-            R.load(addr);
-            // phase 3: what the record decides.  Each state ends by adopting the loaded record
-            // as cell `take`, by resolving a search from node `from` or a known cell `known`, or
-            // by a change of state; the adoption and the search are written once for all
-            // states, so a wave whose lanes are in different states executes each once.
-            const bool closed = closed_contains(R, rx, ry, rz);
-            int take = -1, from = -1, known = -1;
-            switch (act)
+            if (closed)
             {
-                case kOsStart:
+                // off the split planes exactly one of the finer neighbours contains the position
+                const double sx = g.planes[R.b.z], sy = g.planes[R.b.w], sz = g.planes[R.c.x];
+                if (__builtin_expect(rx != sx && ry != sy && rz != sz, 1))
                 {
-                    // the start hint, when the point lies in its box the way the top-down search
-                    // assigns points to leaves: lo <= r < hi on each axis (a point on a split
-                    // plane goes to the upper child), hi included at the domain's upper boundary.
-                    // Every split plane of the leaf's ancestors then sends leafChild's descent
-                    // toward it, so it is the leaf the search returns.
-                    const bool inx = rx >= R.d(0) && (rx < R.d(3) || R.d(3) == g.box[3]);
-                    const bool iny = ry >= R.d(1) && (ry < R.d(4) || R.d(4) == g.box[4]);
-                    const bool inz = rz >= R.d(2) && (rz < R.d(5) || R.d(5) == g.box[5]);
-                    if (inx && iny && inz)
-                        take = hint;
-                    else
-                        from = 0;
-                    break;
+                    pend = static_cast<uint32_t>(~c + (rx < sx ? 0 : 1) + (ry < sy ? 0 : 2) + (rz < sz ? 0 : 4)) << 3
+                           | static_cast<uint32_t>(wall);
+                    return out;
                 }
-                case kOsCross:
-                case kOsListRec:
-                    // a neighbour on the crossed wall (the first, largest-overlap one, then the
-                    // rest of the list in order), when its closed box contains the new position
-                    if (closed)
-                    {
-                        if (cand != i)
-                            take = cand;
-                        else
-                            known = cand;
-                    }
-                    else if (act == kOsCross)
-                        ost = kOsListStart;
-                    else if (++q < qe)
-                        ost = kOsListId;
-                    else
-                        from = 0;
-                    break;
-                case kOsListStart:
-                    q = R.off_at(wall) + 1;
-                    qe = R.off_end_at(wall);
-                    if (q < qe)
-                        ost = kOsListId;
-                    else
-                        from = 0;
-                    break;
-                case kOsListId:
-                    cand = R.first4(q & 3);
-                    ost = kOsListRec;
-                    break;
-                case kOsSearch:
-                    from = 0;
-                    break;
-                case kOsNode:
-                {
-                    const int child = R.i32(6);
-                    if (child < 0)
-                        known = R.i32(7);
-                    else
-                        from = child + (rx < R.d(0) ? 0 : 1) + (ry < R.d(1) ? 0 : 2) + (rz < R.d(2) ? 0 : 4);
-                    break;
-                }
-                default:  // kOsLeaf
-                    take = cand;
-                    break;
             }
-            if (take >= 0)
+            const OctNext e = oct_next_exact(g.node, g.planes, g.nbOff, g.nbc, i, wall, rx, ry, rz, kx, ky, kz);
+            nd = e.node;
+            rx = e.x;
+            ry = e.y;
+            rz = e.z;
+            if (nd < 0)
             {
-                adopt(R, take);
-                if (locating) hint = take;
+                state = kOutside;
+                return out ? 2 : -1;
             }
-            else if (from >= 0)
-                resolve(g, search_lds(g, from));
-            else if (known >= 0)
-                resolve(g, known);
-            if (ost == kOsEnd) return out ? 2 : -1;
+            R.load(g.node + nd);
+            B.load(g, R);
+            adopt(R, B, nd);
             return out;
         }
 
-        // one advance() per call for the octree (next() for the other grids)
-        __device__ __forceinline__ int advance(const GridView& g, int& m, double& ds, double& n)
+        // ---------------------------------------------------------------- all grids
+        // Enters the domain and finds the start cell; false when the path has no segment at all.
+        // entry: the length of the path before the domain (0 when it starts inside).
+        __device__ __forceinline__ bool begin(const GridView& g, double& entry)
         {
-            if constexpr (GT == kOctree)
-                return advance_octree(g, m, ds, n);
+            if (!move_inside(g, entry)) return false;
+            if constexpr (GT == kCartesian || GT == kOctree)
+            {
+                ikx = 1. / kx;
+                iky = 1. / ky;
+                ikz = 1. / kz;
+            }
+            if constexpr (GT == kCartesian)
+            {
+                i = locate_clip(g.xb, g.nx + 1, rx);
+                j = locate_clip(g.yb, g.ny + 1, ry);
+                k = locate_clip(g.zb, g.nz + 1, rz);
+            }
+            else if constexpr (GT == kOctree)
+            {
+                if (!oct_begin(g))
+                {
+                    state = kOutside;
+                    return false;
+                }
+            }
             else
-                return next(g, m, ds, n) ? 1 : -1;
+            {
+                if constexpr (GT == kVoronoi)
+                    i = hint >= 0 && vor_nearest_strict(g, hint, rx, ry, rz) ? hint : vor_cell_index(g, rx, ry, rz);
+                else
+                    i = hint >= 0 && tet_inside_strict(g.tcell[hint], rx, ry, rz) ? hint : tet_cell_index(g, rx, ry, rz);
+                hint = i;
+                if (i < 0)
+                {
+                    state = kOutside;
+                    return false;
+                }
+                if constexpr (GT == kVoronoi)
+                    vor_enter(g, i);
+                else
+                    j = -1;
+            }
+            return true;
         }
 
-        // Returns false when the path has no more segments; otherwise sets the cell m, the
-        // segment length ds and the cell's number density n (0 for m = -1).
-        __device__ __forceinline__ bool next(const GridView& g, int& m, double& ds, double& n)
+        // One step of a path that has begun: 1 with the segment (the cell m, the length ds and the
+        // cell's number density n) when the step completed one, 2 with the path's last segment, 0
+        // when it only progressed (the octree's descent), -1 at the end of the path.
+        __device__ __forceinline__ int cross(const GridView& g, int& m, double& ds, double& n)
         {
             if constexpr (GT == kOctree)
+                return cross_octree(g, m, ds, n);
+            else
             {
-                int r;
-                while ((r = advance_octree(g, m, ds, n)) == 0) {}
-                return r > 0;
+                bool more;
+                if constexpr (GT == kCartesian)
+                    more = next_cartesian(g, m, ds, n);
+                else if constexpr (GT == kVoronoi)
+                    more = next_voronoi(g, m, ds, n);
+                else
+                    more = next_tetra(g, m, ds, n);
+                return !more ? -1 : state == kOutside ? 2 : 1;
             }
-            if (state == kOutside) return false;
+        }
+
+        // One step of a path from its start on, as cross(); the first step begins the path and
+        // returns its segment before the domain, if any (m = -1).
+        __device__ __forceinline__ int advance(const GridView& g, int& m, double& ds, double& n)
+        {
+            if (state == kOutside) return -1;
             if (state == kUnknown)
             {
-                double cumds;
-                if (!move_inside(g, cumds)) return false;
-                if (GT == kCartesian)
-                {
-                    i = locate_clip(g.xb, g.nx + 1, rx);
-                    j = locate_clip(g.yb, g.ny + 1, ry);
-                    k = locate_clip(g.zb, g.nz + 1, rz);
-                }
-                else if (GT == kVoronoi)
-                {
-                    if (hint >= 0 && vor_nearest_strict(g, hint, rx, ry, rz))
-                        i = hint;
-                    else
-                        i = vor_cell_index(g, rx, ry, rz);
-                    hint = i;
-                    if (i < 0)
-                    {
-                        state = kOutside;
-                        return false;
-                    }
-                    vor_enter(g, i);
-                }
-                else
-                {
-                    if (hint >= 0 && tet_inside_strict(g.tcell[hint], rx, ry, rz))
-                        i = hint;
-                    else
-                        i = tet_cell_index(g, rx, ry, rz);
-                    j = -1;
-                    hint = i;
-                    if (i < 0)
-                    {
-                        state = kOutside;
-                        return false;
-                    }
-                }
-                if (cumds > 0.)
+                double entry;
+                if (!begin(g, entry)) return -1;
+                if (entry > 0.)
                 {
                     m = -1;
-                    ds = cumds;
+                    ds = entry;
                     n = 0.;
-                    return true;
+                    return 1;
                 }
             }
-            if (GT == kCartesian)
+            return cross(g, m, ds, n);
+        }
+
+        // The next segment of a path; false when it has no more.
+        __device__ __forceinline__ bool next(const GridView& g, int& m, double& ds, double& n)
+        {
+            int r;
+            while ((r = advance(g, m, ds, n)) == 0) {}
+            return r > 0;
+        }
+
+        // CartesianSpatialGrid.cpp:77-153
+        __device__ __forceinline__ bool next_cartesian(const GridView& g, int& m, double& ds, double& n)
+        {
+            int mm = k + g.nz * j + g.nz * g.ny * i;
+            double xE = (kx < 0.0) ? g.xb[i] : g.xb[i + 1];
+            double yE = (ky < 0.0) ? g.yb[j] : g.yb[j + 1];
+            double zE = (kz < 0.0) ? g.zb[k] : g.zb[k + 1];
+            double dsx = (fabs(kx) > 1e-15) ? (xE - rx) / kx : DBL_MAX;
+            double dsy = (fabs(ky) > 1e-15) ? (yE - ry) / ky : DBL_MAX;
+            double dsz = (fabs(kz) > 1e-15) ? (zE - rz) / kz : DBL_MAX;
+            m = mm;
+            n = g.dens ? g.dens[mm] : 0.;
+            if (dsx <= dsy && dsx <= dsz)
             {
-                int mm = k + g.nz * j + g.nz * g.ny * i;
-                double xE = (kx < 0.0) ? g.xb[i] : g.xb[i + 1];
-                double yE = (ky < 0.0) ? g.yb[j] : g.yb[j + 1];
-                double zE = (kz < 0.0) ? g.zb[k] : g.zb[k + 1];
-                double dsx = (fabs(kx) > 1e-15) ? (xE - rx) / kx : DBL_MAX;
-                double dsy = (fabs(ky) > 1e-15) ? (yE - ry) / ky : DBL_MAX;
-                double dsz = (fabs(kz) > 1e-15) ? (zE - rz) / kz : DBL_MAX;
-                m = mm;
-                n = g.dens ? g.dens[mm] : 0.;
-                if (dsx <= dsy && dsx <= dsz)
-                {
-                    ds = dsx;
-                    rx = xE;
-                    ry += ky * dsx;
-                    rz += kz * dsx;
-                    i += (kx < 0.0) ? -1 : 1;
-                    if (i >= g.nx || i < 0) state = kOutside;
-                }
-                else if (dsy < dsx && dsy <= dsz)
-                {
-                    ds = dsy;
-                    ry = yE;
-                    rx += kx * dsy;
-                    rz += kz * dsy;
-                    j += (ky < 0.0) ? -1 : 1;
-                    if (j >= g.ny || j < 0) state = kOutside;
-                }
-                else
-                {
-                    ds = dsz;
-                    rz = zE;
-                    rx += kx * dsz;
-                    ry += ky * dsz;
-                    k += (kz < 0.0) ? -1 : 1;
-                    if (k >= g.nz || k < 0) state = kOutside;
-                }
-                return true;
+                ds = dsx;
+                rx = xE;
+                ry += ky * dsx;
+                rz += kz * dsx;
+                i += (kx < 0.0) ? -1 : 1;
+                if (i >= g.nx || i < 0) state = kOutside;
             }
-            else if constexpr (GT == kVoronoi)
-                return next_voronoi(g, m, ds, n);
-            else if constexpr (GT == kTetra)
-                return next_tetra(g, m, ds, n);
-            return false;  // the octree steps through advance_octree
+            else if (dsy < dsx && dsy <= dsz)
+            {
+                ds = dsy;
+                ry = yE;
+                rx += kx * dsy;
+                rz += kz * dsy;
+                j += (ky < 0.0) ? -1 : 1;
+                if (j >= g.ny || j < 0) state = kOutside;
+            }
+            else
+            {
+                ds = dsz;
+                rz = zE;
+                rx += kx * dsz;
+                ry += ky * dsz;
+                k += (kz < 0.0) ? -1 : 1;
+                if (k >= g.nz || k < 0) state = kOutside;
+            }
+            return true;
         }
 
         // the cell c becomes the current cell, from its record: its site and its run
