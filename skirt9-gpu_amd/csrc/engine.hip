@@ -359,8 +359,54 @@ namespace skg
 
 namespace skg
 {
-    // the node of the leaf holding (x, y, z), -1 outside the root's closed box (one thread)
-    __global__ void octree_locate(GridView g, double x, double y, double z, int* out) { *out = oct_search(g.node, g.planes, x, y, z); }
+    // The start hint of paths from (x, y, z): the cell (octree: the leaf's node) that holds the
+    // position, -1 if none is found.  One wavefront; the candidates of a mesh grid's block are
+    // tested 64 at a time.
+    template<int GT> __global__ void locate_cell(GridView g, double x, double y, double z, int* out)
+    {
+        int best = -1;
+        if constexpr (GT == kOctree)
+            best = oct_search(g.node, g.planes, x, y, z);
+        else if (x >= g.box[0] && x <= g.box[3] && y >= g.box[1] && y <= g.box[4] && z >= g.box[2] && z <= g.box[5])
+        {
+            double dist = DBL_MAX;  // Voronoi: squared distance to the nearest site; tetra: 0 where inside
+            if constexpr (GT == kVoronoi)
+            {
+                const int b = vor_block(g, x, y, z);
+                for (int q = g.vbl_off[b] + threadIdx.x; q < g.vbl_off[b + 1]; q += 64)
+                {
+                    const VorCell& c = g.vcell[g.vbl_id[q]];
+                    const double dx = x - c.x, dy = y - c.y, dz = z - c.z, d = dx * dx + dy * dy + dz * dz;
+                    if (d < dist)
+                    {
+                        dist = d;
+                        best = g.vbl_id[q];
+                    }
+                }
+            }
+            else
+            {
+                const int b = tet_block(g, x, y, z);
+                for (int q = g.tbl_off[b] + threadIdx.x; q < g.tbl_off[b + 1]; q += 64)
+                    if (best < 0 && tet_contains(g.tcell[g.tbl_id[q]], x, y, z))
+                    {
+                        dist = 0.;
+                        best = g.tbl_id[q];
+                    }
+            }
+            for (int o = 32; o > 0; o >>= 1)
+            {
+                const double d = __shfl_xor(dist, o);
+                const int c = __shfl_xor(best, o);
+                if (d < dist)
+                {
+                    dist = d;
+                    best = c;
+                }
+            }
+        }
+        if (threadIdx.x == 0) *out = best;
+    }
 }
 
 // ==================================================================== host side
@@ -417,7 +463,7 @@ struct skg_engine
     // source / options
     double src[3] = {0, 0, 0};
     bool haveSource = false;
-    int srcHint = -1;           // octree: the leaf holding src (start hint of new packets)
+    int srcHint = -1;           // the cell (octree: leaf node) holding src (start hint of new packets)
     bool srcHintValid = false;  // srcHint belongs to the current grid and source
     double xi = 0.5, mwr = 1e4;
     int minScatt = 0;
@@ -934,9 +980,16 @@ int skg_grid_cartesian(skg_engine* e, const double* xb, int32_t nx, const double
     freeGrid(e);
     GridView g{};
     int st;
-    if ((st = gridUpload(e, xb, nx + 1, &g.xb)) || (st = gridUpload(e, yb, ny + 1, &g.yb))
-        || (st = gridUpload(e, zb, nz + 1, &g.zb)))
-        return st;
+    // the borders of the three axes in one table
+    std::vector<double> planes(xb, xb + nx + 1);
+    planes.insert(planes.end(), yb, yb + ny + 1);
+    planes.insert(planes.end(), zb, zb + nz + 1);
+    if ((st = gridUpload(e, planes.data(), planes.size(), &g.planes))) return st;
+    g.nplanes = static_cast<int>(planes.size());
+    g.ldsPlanes = planes.size() <= static_cast<size_t>(kLdsPlanes);
+    g.xb = g.planes;
+    g.yb = g.xb + nx + 1;
+    g.zb = g.yb + ny + 1;
     g.nx = nx;
     g.ny = ny;
     g.nz = nz;
@@ -1891,14 +1944,21 @@ static int runPersistent(skg_engine* e, uint64_t first_history, uint64_t count)
     p.gframe = e->gframe;
     p.guideMix = e->guideMix;
     p.contKey = e->contKey;
-    // the leaf of the point source, the start hint of every new packet (octree): found once
-    // per grid and source by the top-down search, which the hint check then reproduces
-    if (e->gridType == SKG_GRID_OCTREE && !e->srcHintValid)
+    // the cell of the point source, the start hint of every new packet: found once per grid and
+    // source.  (On a mesh grid a packet without a hint scans its block's candidates, hundreds of them
+    // around a dense centre: 43 % of the batched tetra launch went into that scan.)
+    if (e->gridType != SKG_GRID_CARTESIAN && !e->srcHintValid)
     {
         int* d = nullptr;
         HIPCHK(e, hipMalloc(&d, sizeof(int)));
         (void)hipGetLastError();  // a launch error below is then this launch's own
-        hipLaunchKernelGGL(octree_locate, dim3(1), dim3(1), 0, e->stream, e->grid, e->src[0], e->src[1], e->src[2], d);
+        const auto& r = e->src;
+        if (e->gridType == SKG_GRID_OCTREE)
+            hipLaunchKernelGGL(locate_cell<kOctree>, dim3(1), dim3(64), 0, e->stream, e->grid, r[0], r[1], r[2], d);
+        else if (e->gridType == SKG_GRID_VORONOI)
+            hipLaunchKernelGGL(locate_cell<kVoronoi>, dim3(1), dim3(64), 0, e->stream, e->grid, r[0], r[1], r[2], d);
+        else
+            hipLaunchKernelGGL(locate_cell<kTetra>, dim3(1), dim3(64), 0, e->stream, e->grid, r[0], r[1], r[2], d);
         hipError_t st = hipGetLastError();
         if (st == hipSuccess) st = hipMemcpyAsync(&e->srcHint, d, sizeof(int), hipMemcpyDeviceToHost, e->stream);
         if (st == hipSuccess) st = hipStreamSynchronize(e->stream);
@@ -1906,7 +1966,7 @@ static int runPersistent(skg_engine* e, uint64_t first_history, uint64_t count)
         if (st != hipSuccess) return fail(e, SKG_ERR_DEVICE, std::string("source cell: ") + hipGetErrorString(st));
         e->srcHintValid = true;
     }
-    p.srcHint = e->gridType == SKG_GRID_OCTREE ? e->srcHint : -1;
+    p.srcHint = e->gridType == SKG_GRID_CARTESIAN ? -1 : e->srcHint;
     p.rf = e->rf;
     p.persp = 0;
     for (const auto& f : e->frames) p.persp |= f.persp;

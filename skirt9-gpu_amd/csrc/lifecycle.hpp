@@ -30,10 +30,11 @@ namespace skg
         }
         else
         {
-            double st = sin(theta);
-            kx = st * cos(phi);
-            ky = st * sin(phi);
-            kz = cos(theta);
+            double st, sp, cp;
+            sincos(theta, &st, &kz);
+            sincos(phi, &sp, &cp);
+            kx = st * cp;
+            ky = st * sp;
         }
     }
 
@@ -49,8 +50,8 @@ namespace skg
     __device__ __forceinline__ void rotate(Philox& rng, double& kx, double& ky, double& kz, double costheta)
     {
         double phi = 2.0 * M_PI * rng.uniform();
-        double cosphi = cos(phi);
-        double sinphi = sin(phi);
+        double cosphi, sinphi;
+        sincos(phi, &sinphi, &cosphi);
         double sintheta = sqrt(fabs((1.0 - costheta) * (1.0 + costheta)));
         double x = kx, y = ky, z = kz;
         if (z > 0.99999)

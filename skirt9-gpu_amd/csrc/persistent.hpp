@@ -54,7 +54,7 @@ namespace skg
         uint32_t contKey;         // nonzero: histories continue on Philox tag contKey from their first
                                   // scattering on (same emission and first interaction, independent
                                   // continuations)
-        int32_t srcHint;          // octree: the leaf node of the point source (the start hint of new packets), -1: none
+        int32_t srcHint;          // the cell (octree: leaf node) of the point source (the start hint of new packets), -1: none
         double* rf;               // radiation-field variant: ncells x nlambda table
         int persp;                // some instruments are perspective instruments
         int nent;                 // particle-source variant: number of entities (0: the point source)
@@ -296,9 +296,8 @@ namespace skg
             double entry;
             bool fin = !gen.begin(grid, entry);
             // every traversal starts at the packet's position: its start cell is the hint for the
-            // next traversal from there (octree, Voronoi and tetrahedral grids)
-            if constexpr (GT != kCartesian)
-                if (gen.hint >= 0) cu[cHint * kLcThreads + t] = static_cast<uint32_t>(gen.hint);
+            // next traversal from there
+            if (gen.hint >= 0) cu[cHint * kLcThreads + t] = static_cast<uint32_t>(gen.hint);
             if (!fin && entry > 0.)
             {
                 steps = 1;
@@ -771,8 +770,7 @@ namespace skg
             double kext = n > 0. ? n * se : 0.;
             double albedo = kext > 0. ? ksca / kext : 0.;
             pk.W *= -expm1(-pk.taupath) * albedo;
-            if constexpr (GT != kCartesian)
-                pk.hint = m;  // the interaction point lies in the cell of its segment
+            pk.hint = GT == kCartesian ? -1 : m;  // the interaction point lies in the cell of its segment
             pk.rx += s * pk.kx;
             pk.ry += s * pk.ky;
             pk.rz += s * pk.kz;
@@ -845,17 +843,18 @@ namespace skg
     __device__ __forceinline__ int lane_id() { return __lane_id(); }
 
     // Minimum waves per SIMD, with the measured alternatives (ms at 2 / 3 / 4 waves):
-    //   Cartesian 64^3, 2^21 packets               25.1 / 23.0 / 22.4
+    //   Cartesian 64^3, 2^21 packets               23.2 / 22.5 / 21.8
+    //   Cartesian 44^3, 2e5 packets                 3.3 /  3.3 /  3.6 (one packet per lane)
     //   octree disk, ten levels, tau_V 50, 2^21    50.1 / 43.3 / 46.0 (at four, spills around the
     //   octree, nine levels, 40 wavelengths, 3e5    8.4 /  8.4 /  8.1  events double the writes)
     //   octree with the radiation field, 2e5        7.8 / 11.6 / 13.2 (bound by its atomics, whose
-    //                                                  targets collide more with more waves)
+    //   Cartesian with the field, 7e5              targets collide more with more waves)
     // Voronoi and tetra as measured before the events became calls: 1152 / 1086 / 1061 ms and
     // 6.72 / 5.80 / 5.27 s.  The guided variant's network call holds whole layers' weights in
     // registers, and its four-wave build does not compile for the mesh grids.
     template<int GT, int V> constexpr int lifecycle_waves()
     {
-        return V == kGuided || V == kStoreRF ? 2 : GT == kOctree ? 3 : 4;
+        return V == kGuided || V == kStoreRF ? 2 : GT == kOctree ? 3 : GT == kCartesian ? 3 : 4;
     }
 
     // The kernel's parameter block where it lies in the kernarg segment, behind a pointer the
@@ -890,6 +889,10 @@ namespace skg
         // waits in kFetch
         T.phase = lane < p.lanes ? kFetch : kDone;
         T.ended = false;
+        T.last = -1;
+        T.tau = T.s = T.lim = 0.;
+        T.tau32.reset();
+        T.s32.reset();
         bool busy = false;  // the lane's traversal is under way
         while (true)
         {

@@ -119,7 +119,8 @@ namespace skg
         int nx, ny, nz;
         const double* dens;  // Cartesian: number density per cell
         const OctNode* node;
-        const double* planes;   // the distinct coordinates of the tree's bounds
+        const double* planes;   // octree: the distinct coordinates of the tree's bounds; Cartesian: the
+                                // borders of the three axes, one after the other
         int nplanes;
         int ldsPlanes;          // nonzero: the kernel staged them in LDS (stage_planes)
         const int32_t* nbOff;   // start of each node's and wall's neighbour list (6 per node, and the end)
@@ -256,11 +257,14 @@ namespace skg
     // reference's search lists hold, in increasing index order, every tetra whose bounding
     // box meets the point's block, so its first hit is the lowest index; the block lists here
     // have the same property)
-    __device__ __forceinline__ int tet_cell_index(const GridView& g, double x, double y, double z)
+    __device__ __forceinline__ int tet_block(const GridView& g, double x, double y, double z)
     {
         const int n = g.tbn;
-        int i = tet_axis_block(g.tbx, n, x), j = tet_axis_block(g.tby, n, y), k = tet_axis_block(g.tbz, n, z);
-        int b = (i * n + j) * n + k;
+        return (tet_axis_block(g.tbx, n, x) * n + tet_axis_block(g.tby, n, y)) * n + tet_axis_block(g.tbz, n, z);
+    }
+    __device__ __forceinline__ int tet_cell_index(const GridView& g, double x, double y, double z)
+    {
+        const int b = tet_block(g, x, y, z);
         for (int q = g.tbl_off[b], e = g.tbl_off[b + 1]; q < e; ++q)
         {
             const int id = g.tbl_id[q];
@@ -290,27 +294,6 @@ namespace skg
         kOutside = 2
     };
 
-    __device__ __forceinline__ int locate_clip(const double* xv, int n, double x)
-    {
-        // NR::locateClip over n borders (NR.hpp:130-144, :177-183)
-        if (x < xv[0]) return 0;
-        int jl = -1, ju = n - 1;
-        while (ju - jl > 1)
-        {
-            int jm = (ju + jl) >> 1;
-            if (x < xv[jm])
-                ju = jm;
-            else
-                jl = jm;
-        }
-        return jl;
-    }
-
-    __device__ __forceinline__ bool node_contains(const double* b, double x, double y, double z)
-    {
-        return x >= b[0] && x <= b[3] && y >= b[1] && y <= b[4] && z >= b[2] && z <= b[5];
-    }
-
     // a ? x : b ? y : z on values (selecting among members by reference would make the
     // compiler select their addresses and keep the generator in scratch memory)
     template<typename T> __device__ __forceinline__ T pick3(bool a, bool b, T x, T y, T z)
@@ -331,13 +314,14 @@ namespace skg
         return fma(fma(-b, q, a), y, q);
     }
 
-    // The octree's coordinate table in LDS (dynamic shared memory of nplanes doubles when
-    // GridView::ldsPlanes is set); every kernel that walks an octree calls stage_planes first.
+    // The coordinate table of a Cartesian grid or octree in LDS (dynamic shared memory of nplanes
+    // doubles when GridView::ldsPlanes is set); every kernel that walks a grid calls stage_planes
+    // first.
     extern __shared__ double skg_planes[];
 
     template<int GT> __device__ __forceinline__ void stage_planes(const GridView& g)
     {
-        if constexpr (GT == kOctree)
+        if constexpr (GT == kOctree || GT == kCartesian)
         {
             if (g.ldsPlanes)
                 for (int t = threadIdx.x; t < g.nplanes; t += blockDim.x) skg_planes[t] = g.planes[t];
@@ -457,18 +441,20 @@ namespace skg
     {
         double rx, ry, rz, kx, ky, kz;
         int state;
-        int i, j, k;  // Cartesian cell indices; octree: i = current leaf's node; Voronoi, tetra: i =
+        int i, j, k;  // Cartesian: entry of the border ahead on each axis in the planes table; octree: i = current leaf's node; Voronoi, tetra: i =
                       // current cell (tetra: j = entering face, -1 if unknown; Voronoi: j = the
                       // header slot of the cell's run in the entry table)
         double sx, sy, sz;      // Voronoi: the current cell's site
         double ikx, iky, ikz;   // Cartesian, octree: reciprocals of the direction
-        double b0, b1, b2, bn;  // octree: the current cell's wall ahead on each axis, its density
+        double b0, b1, b2, bn;  // Cartesian, octree: the current cell's wall ahead on each axis, its
+                                // density
         int f0, f1, f2;         // octree: the node across each of those walls
-        int cell;               // octree: the current leaf's cell index
+        int cell;               // Cartesian, octree: the current cell's index
         uint32_t pend;  // octree: a node to descend into next and the crossed wall (node << 3 | wall),
                         // or kNoPend
-        int hint;  // octree (a node), Voronoi, tetra: a cell that probably contains the start point
-                   // (-1: none); after the first step, the start cell
+        int hint;  // a cell that probably contains the start point (-1: none), after the first step
+                   // the start cell: octree a node, Voronoi and tetra a cell, Cartesian the cell's
+                   // indices i | j << 10 | k << 20 (no more than 1024 cells along an axis)
         static constexpr uint32_t kNoPend = 0xFFFFFFFFu;  // node ids stay below 2^29
 
         __device__ __forceinline__ void start(double r0, double r1, double r2, double k0, double k1, double k2,
@@ -691,9 +677,25 @@ namespace skg
             }
             if constexpr (GT == kCartesian)
             {
-                i = locate_clip(g.xb, g.nx + 1, rx);
-                j = locate_clip(g.yb, g.ny + 1, ry);
-                k = locate_clip(g.zb, g.nz + 1, rz);
+                const int oy = g.nx + 1, oz = oy + g.ny + 1;
+                int ci = hint & 1023, cj = (hint >> 10) & 1023, ck = hint >> 20;
+                const bool found = hint >= 0 && rx >= border(g, ci) && rx < border(g, ci + 1) && ry >= border(g, oy + cj)
+                                   && ry < border(g, oy + cj + 1) && rz >= border(g, oz + ck) && rz < border(g, oz + ck + 1);
+                if (!found)
+                {
+                    ci = locate(g, 0, g.nx, rx);
+                    cj = locate(g, oy, g.ny, ry);
+                    ck = locate(g, oz, g.nz, rz);
+                }
+                hint = max(max(g.nx, g.ny), g.nz) <= 1024 ? ci | (cj << 10) | (ck << 20) : -1;
+                cell = ck + g.nz * cj + g.nz * g.ny * ci;
+                i = ci + (kx < 0.0 ? 0 : 1);
+                j = g.nx + 1 + cj + (ky < 0.0 ? 0 : 1);
+                k = g.nx + g.ny + 2 + ck + (kz < 0.0 ? 0 : 1);
+                b0 = border(g, i);
+                b1 = border(g, j);
+                b2 = border(g, k);
+                bn = g.dens ? g.dens[cell] : 0.;
             }
             else if constexpr (GT == kOctree)
             {
@@ -771,45 +773,64 @@ namespace skg
             return r > 0;
         }
 
-        // CartesianSpatialGrid.cpp:77-153
+        __device__ __forceinline__ static double border(const GridView& g, int q)
+        {
+            return g.ldsPlanes ? skg_planes[q] : g.planes[q];
+        }
+
+        // NR::locateClip (NR.hpp:130-144, :177-183) over the n + 1 borders from entry `first` on: the
+        // cell that holds x
+        __device__ __forceinline__ static int locate(const GridView& g, int first, int n, double x)
+        {
+            if (x < border(g, first)) return 0;
+            int jl = -1, ju = n;
+            while (ju - jl > 1)
+            {
+                const int jm = (ju + jl) >> 1;
+                if (x < border(g, first + jm))
+                    ju = jm;
+                else
+                    jl = jm;
+            }
+            return jl;
+        }
+
+        // CartesianSpatialGrid.cpp:77-153.  The border ahead on each axis and the cell's density are
+        // kept from crossing to crossing: a crossing reads one border (of the axis it moved along,
+        // from LDS) and the next cell's density, which is needed only when that cell's segment is
+        // complete, so that its load is in flight during the next crossing's arithmetic.
         __device__ __forceinline__ bool next_cartesian(const GridView& g, int& m, double& ds, double& n)
         {
-            int mm = k + g.nz * j + g.nz * g.ny * i;
-            double xE = (kx < 0.0) ? g.xb[i] : g.xb[i + 1];
-            double yE = (ky < 0.0) ? g.yb[j] : g.yb[j + 1];
-            double zE = (kz < 0.0) ? g.zb[k] : g.zb[k + 1];
-            double dsx = (fabs(kx) > 1e-15) ? (xE - rx) / kx : DBL_MAX;
-            double dsy = (fabs(ky) > 1e-15) ? (yE - ry) / ky : DBL_MAX;
-            double dsz = (fabs(kz) > 1e-15) ? (zE - rz) / kz : DBL_MAX;
-            m = mm;
-            n = g.dens ? g.dens[mm] : 0.;
-            if (dsx <= dsy && dsx <= dsz)
+            const double dsx = (fabs(kx) > 1e-15) ? quotient(b0 - rx, kx, ikx) : DBL_MAX;
+            const double dsy = (fabs(ky) > 1e-15) ? quotient(b1 - ry, ky, iky) : DBL_MAX;
+            const double dsz = (fabs(kz) > 1e-15) ? quotient(b2 - rz, kz, ikz) : DBL_MAX;
+            m = cell;
+            n = bn;
+            const bool ax = dsx <= dsy && dsx <= dsz;
+            const bool ay = !ax && dsy < dsx && dsy <= dsz;
+            ds = pick3(ax, ay, dsx, dsy, dsz);
+            rx = ax ? b0 : rx + kx * ds;
+            ry = ay ? b1 : ry + ky * ds;
+            rz = (ax || ay) ? rz + kz * ds : b2;
+            const bool neg = pick3(ax, ay, kx, ky, kz) < 0.0;
+            const int first = pick3(ax, ay, 0, g.nx + 1, g.nx + g.ny + 2), count = pick3(ax, ay, g.nx, g.ny, g.nz);
+            const int at = pick3(ax, ay, i, j, k);
+            if (at == (neg ? first : first + count))
             {
-                ds = dsx;
-                rx = xE;
-                ry += ky * dsx;
-                rz += kz * dsx;
-                i += (kx < 0.0) ? -1 : 1;
-                if (i >= g.nx || i < 0) state = kOutside;
+                state = kOutside;  // the domain's border
+                return true;
             }
-            else if (dsy < dsx && dsy <= dsz)
-            {
-                ds = dsy;
-                ry = yE;
-                rx += kx * dsy;
-                rz += kz * dsy;
-                j += (ky < 0.0) ? -1 : 1;
-                if (j >= g.ny || j < 0) state = kOutside;
-            }
-            else
-            {
-                ds = dsz;
-                rz = zE;
-                rx += kx * dsz;
-                ry += ky * dsz;
-                k += (kz < 0.0) ? -1 : 1;
-                if (k >= g.nz || k < 0) state = kOutside;
-            }
+            const int to = at + (neg ? -1 : 1);
+            const int stride = pick3(ax, ay, g.nz * g.ny, g.nz, 1);
+            cell += neg ? -stride : stride;
+            bn = g.dens ? g.dens[cell] : 0.;
+            const double b = border(g, to);
+            i = ax ? to : i;
+            j = ay ? to : j;
+            k = (ax || ay) ? k : to;
+            b0 = ax ? b : b0;
+            b1 = ay ? b : b1;
+            b2 = (ax || ay) ? b2 : b;
             return true;
         }
 
