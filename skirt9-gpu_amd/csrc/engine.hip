@@ -33,13 +33,21 @@
 namespace skg
 {
     // ------------------------------------------------------------------ path service kernels
-    template<int GT> __global__ void trace_count(GridView g, const double* __restrict__ rays, int64_t n, int64_t* counts)
+    // the path of this thread, and whether the thread stores its results: L lanes walk each path
+    template<int L> __device__ __forceinline__ int64_t path_index()
     {
-        int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
+        return (blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x) / L;
+    }
+    template<int L> __device__ __forceinline__ bool path_lead() { return threadIdx.x % L == 0; }
+
+    template<int GT, int L> __global__ void __launch_bounds__(256) trace_count(GridView g, const double* __restrict__ rays, int64_t n, int64_t* counts)
+    {
+        const int64_t t = path_index<L>();
+        const bool lead = path_lead<L>();
         stage_planes<GT>(g);
         if (t >= n) return;
         const double* ray = rays + 6 * t;
-        Gen<GT> gen;
+        Gen<GT, L> gen;
         gen.start(ray[0], ray[1], ray[2], ray[3], ray[4], ray[5]);
         int m;
         double ds, nd;
@@ -51,19 +59,21 @@ namespace skg
             ++c;
             if (ds > 0.) ++cs;
         }
+        if (!lead) return;
         counts[2 * t] = c;
         counts[2 * t + 1] = cs;
     }
 
-    template<int GT>
-    __global__ void trace_write(GridView g, const double* __restrict__ rays, int64_t n, const int64_t* off, int32_t* mo,
+    template<int GT, int L>
+    __global__ void __launch_bounds__(256) trace_write(GridView g, const double* __restrict__ rays, int64_t n, const int64_t* off, int32_t* mo,
                                 double* dso)
     {
-        int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
+        const int64_t t = path_index<L>();
+        const bool lead = path_lead<L>();
         stage_planes<GT>(g);
         if (t >= n) return;
         const double* ray = rays + 6 * t;
-        Gen<GT> gen;
+        Gen<GT, L> gen;
         gen.start(ray[0], ray[1], ray[2], ray[3], ray[4], ray[5]);
         int m;
         double ds, nd;
@@ -72,8 +82,11 @@ namespace skg
         {
             r = gen.advance(g, m, ds, nd);
             if (r <= 0) continue;
-            mo[o] = m;
-            dso[o] = ds;
+            if (lead)
+            {
+                mo[o] = m;
+                dso[o] = ds;
+            }
             ++o;
         }
     }
@@ -86,14 +99,15 @@ namespace skg
     // the scan's block sums and, after the last one, the total; shared by every call on a device
     static __device__ __align__(256) int64_t scratch[kScanMaxBlocks + 1];
 
-    template<int GT> __global__ void trace_count_off(GridView g, const double* __restrict__ rays, int64_t n, int64_t* off)
+    template<int GT, int L> __global__ void __launch_bounds__(256) trace_count_off(GridView g, const double* __restrict__ rays, int64_t n, int64_t* off)
     {
-        int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
+        const int64_t t = path_index<L>();
+        const bool lead = path_lead<L>();
         stage_planes<GT>(g);
-        if (t == 0) off[0] = 0;
+        if (t == 0 && lead) off[0] = 0;
         if (t >= n) return;
         const double* ray = rays + 6 * t;
-        Gen<GT> gen;
+        Gen<GT, L> gen;
         gen.start(ray[0], ray[1], ray[2], ray[3], ray[4], ray[5]);
         int m;
         double ds, nd;
@@ -103,7 +117,7 @@ namespace skg
             r = gen.advance(g, m, ds, nd);
             if (r > 0) ++c;
         }
-        off[t + 1] = c;
+        if (lead) off[t + 1] = c;
     }
 
     // inclusive scan of off[1..n] within blocks of kScanItems; block b's sum into sums[b]
@@ -188,30 +202,31 @@ namespace skg
         if (c >= 0) node[i].dens = dens[c];
     }
 
-    // and into the cell records (Voronoi cells, tetrahedra)
-    template<typename Rec> __global__ void fill_record_density(Rec* rec, const double* dens, int64_t n)
+    // and into the tetrahedra's records
+    __global__ void fill_tet_density(TetCell* rec, const double* dens, int64_t n)
     {
         int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
         if (i < n) rec[i].dens = dens[i];
     }
 
-    // and into the header slot of each Voronoi cell's run in the entry table
-    __global__ void fill_vor_run_density(VorNb* nb, const VorCell* cells, const double* dens, int64_t n)
+    // and into the heads of the Voronoi cells' runs
+    __global__ void fill_vor_density(VorNb* nb, const VorCell* cell, const double* dens, int64_t n)
     {
         int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
-        if (i < n) nb[cells[i].begin].x = dens[i];
+        if (i < n) reinterpret_cast<VorHead*>(nb + cell[i].run)->dens = dens[i];
     }
 
-    template<int GT, int FP>
-    __global__ void trace_tau(GridView g, const double* __restrict__ dens, const float* __restrict__ dens32,
+    template<int GT, int FP, int L>
+    __global__ void __launch_bounds__(256) trace_tau(GridView g, const double* __restrict__ dens, const float* __restrict__ dens32,
                               double section, double taumax, const double* __restrict__ rays, int64_t n,
                               double* tau_path, double* tau_obs, const int64_t* toff, double* tau_cum)
     {
-        int64_t t = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
+        const int64_t t = path_index<L>();
+        const bool lead = path_lead<L>();
         stage_planes<GT>(g);
         if (t >= n) return;
         const double* ray = rays + 6 * t;
-        Gen<GT> gen;
+        Gen<GT, L> gen;
         int m;
         double ds, nd;
         // complete path, cumulative tau over stored (ds > 0) segments
@@ -234,10 +249,14 @@ namespace skg
                     else
                         k32.add(s32 * static_cast<float>(nd) * static_cast<float>(ds));
                 }
-                if (tau_cum && o < oend) tau_cum[o++] = (FP == SKG_FP64) ? tau : static_cast<double>(k32.sum);
+                if (tau_cum && o < oend)
+                {
+                    if (lead) tau_cum[o] = (FP == SKG_FP64) ? tau : static_cast<double>(k32.sum);
+                    ++o;
+                }
             }
         }
-        tau_path[t] = (FP == SKG_FP64) ? tau : static_cast<double>(k32.sum);
+        if (lead) tau_path[t] = (FP == SKG_FP64) ? tau : static_cast<double>(k32.sum);
         // observer optical depth with early-out (every segment from next() counts)
         gen.start(ray[0], ray[1], ray[2], ray[3], ray[4], ray[5]);
         tau = 0.;
@@ -270,7 +289,7 @@ namespace skg
             }
         }
         res = (FP == SKG_FP64) ? tau : static_cast<double>(k32.sum);
-        tau_obs[t] = inf ? INFINITY : res;
+        if (lead) tau_obs[t] = inf ? INFINITY : res;
     }
 
     // ------------------------------------------------------------------ cell densities
@@ -359,8 +378,8 @@ namespace skg
 
 namespace skg
 {
-    // The start hint of paths from (x, y, z): the cell (octree: the leaf's node) that holds the
-    // position, -1 if none is found.  One wavefront; the candidates of a mesh grid's block are
+    // The start hint of paths from (x, y, z): the cell (octree: the leaf's node, Voronoi: the cell's
+    // run) that holds the position, -1 if none is found.  One wavefront; the candidates of a mesh grid's block are
     // tested 64 at a time.
     template<int GT> __global__ void locate_cell(GridView g, double x, double y, double z, int* out)
     {
@@ -405,6 +424,8 @@ namespace skg
                 }
             }
         }
+        if constexpr (GT == kVoronoi)
+            if (best >= 0) best = g.vcell[best].run;
         if (threadIdx.x == 0) *out = best;
     }
 }
@@ -594,6 +615,35 @@ namespace
         e->ncells = 0;
     }
 
+    // The cell of the point source, the start hint of every new packet (Cartesian: none): found once
+    // per grid and source.  (On a mesh grid a packet without a hint scans its block's candidates, hundreds of them
+    // around a dense centre: 43 % of the batched tetra launch went into that scan.)
+    int sourceHint(skg_engine* e)
+    {
+        if (e->srcHintValid) return SKG_OK;
+        e->srcHint = -1;
+        if (e->gridType != SKG_GRID_CARTESIAN)
+        {
+            int* d = nullptr;
+            HIPCHK(e, hipMalloc(&d, sizeof(int)));
+            (void)hipGetLastError();  // a launch error below is then this launch's own
+            const auto& r = e->src;
+            if (e->gridType == SKG_GRID_OCTREE)
+                hipLaunchKernelGGL(locate_cell<kOctree>, dim3(1), dim3(64), 0, e->stream, e->grid, r[0], r[1], r[2], d);
+            else if (e->gridType == SKG_GRID_VORONOI)
+                hipLaunchKernelGGL(locate_cell<kVoronoi>, dim3(1), dim3(64), 0, e->stream, e->grid, r[0], r[1], r[2], d);
+            else
+                hipLaunchKernelGGL(locate_cell<kTetra>, dim3(1), dim3(64), 0, e->stream, e->grid, r[0], r[1], r[2], d);
+            hipError_t st = hipGetLastError();
+            if (st == hipSuccess) st = hipMemcpyAsync(&e->srcHint, d, sizeof(int), hipMemcpyDeviceToHost, e->stream);
+            if (st == hipSuccess) st = hipStreamSynchronize(e->stream);
+            hipFree(d);
+            if (st != hipSuccess) return fail(e, SKG_ERR_DEVICE, std::string("source cell: ") + hipGetErrorString(st));
+        }
+        e->srcHintValid = true;
+        return SKG_OK;
+    }
+
     int refreshLeafDensity(skg_engine* e)
     {
         if (e->gridType == SKG_GRID_CARTESIAN || e->gridType < 0 || !e->dens || e->densCells < e->ncells) return SKG_OK;
@@ -603,13 +653,10 @@ namespace
             hipLaunchKernelGGL(fill_node_density, dim3(static_cast<unsigned>((e->nnodes + 255) / 256)), block, 0, e->stream,
                                const_cast<OctNode*>(e->grid.node), e->dens, e->nnodes);
         else if (e->gridType == SKG_GRID_VORONOI)
-        {
-            hipLaunchKernelGGL(fill_record_density<VorCell>, grid, block, 0, e->stream, const_cast<VorCell*>(e->grid.vcell), e->dens, n);
-            hipLaunchKernelGGL(fill_vor_run_density, grid, block, 0, e->stream, const_cast<VorNb*>(e->grid.vnb), e->grid.vcell,
+            hipLaunchKernelGGL(fill_vor_density, grid, block, 0, e->stream, const_cast<VorNb*>(e->grid.vnb), e->grid.vcell,
                                e->dens, n);
-        }
         else
-            hipLaunchKernelGGL(fill_record_density<TetCell>, grid, block, 0, e->stream, const_cast<TetCell*>(e->grid.tcell), e->dens, n);
+            hipLaunchKernelGGL(fill_tet_density, grid, block, 0, e->stream, const_cast<TetCell*>(e->grid.tcell), e->dens, n);
         HIPCHK(e, hipGetLastError());
         HIPCHK(e, hipStreamSynchronize(e->stream));
         return SKG_OK;
@@ -714,24 +761,24 @@ namespace
     // dynamic LDS of the kernels that walk the grid: the octree's coordinate table
     size_t planeBytes(const GridView& g) { return g.ldsPlanes ? static_cast<size_t>(g.nplanes) * sizeof(double) : 0; }
 
-    template<int GT, int FP>
+    template<int GT, int FP, int L>
     hipError_t launchLifecycle(const SimParams& p, bool guided, int blocks, int threads, hipStream_t s)
     {
         const size_t lds = planeBytes(p.grid);
         // batched instances, guided sampling and radiation-field storage take their own
         // instantiations; the plain run carries none of them
         if (p.ninst)
-            hipLaunchKernelGGL((lifecycle<GT, FP, kBatched>), dim3(blocks), dim3(threads), lds, s, p);
+            hipLaunchKernelGGL((lifecycle<GT, FP, kBatched, L>), dim3(blocks), dim3(threads), lds, s, p);
         else if (p.rf)
-            hipLaunchKernelGGL((lifecycle<GT, FP, kStoreRF>), dim3(blocks), dim3(threads), lds, s, p);
+            hipLaunchKernelGGL((lifecycle<GT, FP, kStoreRF, L>), dim3(blocks), dim3(threads), lds, s, p);
         else if (p.persp)
-            hipLaunchKernelGGL((lifecycle<GT, FP, kPersp>), dim3(blocks), dim3(threads), lds, s, p);
+            hipLaunchKernelGGL((lifecycle<GT, FP, kPersp, L>), dim3(blocks), dim3(threads), lds, s, p);
         else if (p.nent)
-            hipLaunchKernelGGL((lifecycle<GT, FP, kParticles>), dim3(blocks), dim3(threads), lds, s, p);
+            hipLaunchKernelGGL((lifecycle<GT, FP, kParticles, L>), dim3(blocks), dim3(threads), lds, s, p);
         else if (guided)
-            hipLaunchKernelGGL((lifecycle<GT, FP, kGuided>), dim3(blocks), dim3(threads), lds, s, p);
+            hipLaunchKernelGGL((lifecycle<GT, FP, kGuided, L>), dim3(blocks), dim3(threads), lds, s, p);
         else
-            hipLaunchKernelGGL((lifecycle<GT, FP, kPlain>), dim3(blocks), dim3(threads), lds, s, p);
+            hipLaunchKernelGGL((lifecycle<GT, FP, kPlain, L>), dim3(blocks), dim3(threads), lds, s, p);
         return hipGetLastError();
     }
 }
@@ -753,6 +800,24 @@ namespace
             case SKG_GRID_VORONOI: return f(std::integral_constant<int, kVoronoi>());
             default: return f(std::integral_constant<int, kTetra>());
         }
+    }
+
+    // The lanes of a wavefront that walk each of n paths together.  On a Voronoi grid four lanes share
+    // a cell's neighbours where the paths do not fill the chip: a crossing's chain is then shorter and
+    // its loads coalesce, but the FP64 part runs four times.  ms with one / four lanes (60 000 sites):
+    //              2 000       30 000      120 000     250 000     1 000 000
+    //   packets    4.6 / 2.4   5.4 / 3.7   7.9 / 7.8   10.3 / 14.3  27.9 / 49.5
+    //   rays       1.3 / 0.6   1.4 / 0.8   1.9 / 1.6    2.9 / 3.2   10.9 / 13.1
+    int pathLanes(const skg_engine* e, int64_t n)
+    {
+        return e->gridType == SKG_GRID_VORONOI && n <= 512 * static_cast<int64_t>(e->cus) ? 4 : 1;
+    }
+
+    // f(grid type, lanes per path) with both as compile-time constants
+    template<typename F> int dispatchLanes(skg_engine* e, int64_t n, F&& f)
+    {
+        if (pathLanes(e, n) == 4) return f(std::integral_constant<int, kVoronoi>(), std::integral_constant<int, 4>());
+        return dispatchGrid(e, [&](auto gt) { return f(gt, std::integral_constant<int, 1>()); });
     }
 
     // The node a crossing of wall w (BACK..TOP) of leaf n enters (OctNode::first).  A neighbour
@@ -1138,45 +1203,45 @@ int skg_grid_voronoi(skg_engine* e, int64_t nsites, const double* sites, const i
         return fail(e, SKG_ERR_ARGUMENT, "skg_grid_voronoi: bad arguments");
     if (!(box[0] < box[3] && box[1] < box[4] && box[2] < box[5])) return fail(e, SKG_ERR_ARGUMENT, "skg_grid_voronoi: empty box");
     std::vector<VorCell> cells(nsites);
-    // one run per cell in the entry table: a header slot, then the neighbour entries
     int64_t slots = 0;
     for (int64_t m = 0; m < nsites; ++m)
     {
         if (nb_begin[m] < 0 || nb_count[m] < 0) return fail(e, SKG_ERR_ARGUMENT, "skg_grid_voronoi: bad neighbour range");
-        VorCell& c = cells[m];
-        std::memset(&c, 0, sizeof(c));
-        c.x = sites[3 * m];
-        c.y = sites[3 * m + 1];
-        c.z = sites[3 * m + 2];
-        c.begin = static_cast<int32_t>(std::min<int64_t>(slots, INT32_MAX));
-        c.count = nb_count[m];
-        slots += 1 + static_cast<int64_t>(nb_count[m]);
-        if (slots + 3 > static_cast<int64_t>(INT32_MAX)) return fail(e, SKG_ERR_ARGUMENT, "skg_grid_voronoi: too many neighbours");
+        cells[m] = VorCell{sites[3 * m], sites[3 * m + 1], sites[3 * m + 2], static_cast<int32_t>(slots), 0};
+        slots += (3 + std::max<int64_t>(nb_count[m], kVorPad) + 3) & ~int64_t(3);
+        if (slots > static_cast<int64_t>(INT32_MAX) - kVorSlack) return fail(e, SKG_ERR_ARGUMENT, "skg_grid_voronoi: too many neighbours");
     }
-    std::vector<VorNb> nbs(static_cast<size_t>(slots + 3));
-    std::memset(nbs.data(), 0, nbs.size() * sizeof(VorNb));
+    double size = std::max({box[3] - box[0], box[4] - box[1], box[5] - box[2]});
+    const double scale = 1. / size;
+    for (int q = 0; q < 6; ++q) size = std::max(size, std::abs(box[q]));
+    const double least = kVorMinOffset * size * scale;
+    std::vector<VorNb> nbs(static_cast<size_t>(slots + kVorSlack), VorNb{NAN, NAN, NAN, 0});
     for (int64_t m = 0; m < nsites; ++m)
     {
-        const VorCell& c = cells[m];
-        VorNb& H = nbs[c.begin];
-        H.id = kVorHeader;
-        H.run = c.count;  // the density (x) is filled with the medium
+        VorNb* run = nbs.data() + cells[m].run;
+        VorHead h{cells[m].x, cells[m].y, cells[m].z, 0., nb_count[m], static_cast<int32_t>(m), 0.f, 0.f};
         for (int32_t q = 0; q < nb_count[m]; ++q)
         {
-            int32_t id = nb_index[static_cast<int64_t>(nb_begin[m]) + q];
+            const int32_t id = nb_index[static_cast<int64_t>(nb_begin[m]) + q];
             if (id < -6 || id >= nsites) return fail(e, SKG_ERR_ARGUMENT, "skg_grid_voronoi: neighbour id out of range");
-            VorNb& E = nbs[static_cast<size_t>(c.begin) + 1 + q];
-            E.id = id;
-            E.run = id >= 0 ? cells[id].begin : -1;
+            double d[3] = {0., 0., 0.};
             if (id >= 0)
+                for (int a = 0; a < 3; ++a) d[a] = (sites[3 * static_cast<int64_t>(id) + a] - sites[3 * m + a]) * scale;
+            else
             {
-                E.x = sites[3 * static_cast<int64_t>(id)];
-                E.y = sites[3 * static_cast<int64_t>(id) + 1];
-                E.z = sites[3 * static_cast<int64_t>(id) + 2];
+                const int w = -1 - id, a = w >> 1;
+                d[a] = 2. * (box[(w & 1) ? 3 + a : a] - sites[3 * m + a]) * scale;
+                if ((d[a] > 0.) != ((w & 1) != 0)) d[a] = 0.;  // a site beyond the wall
             }
+            const double norm = std::abs(d[0]) + std::abs(d[1]) + std::abs(d[2]);
+            if (!(norm >= least)) d[0] = d[1] = d[2] = 0.;
+            run[3 + q] = VorNb{static_cast<float>(d[0]), static_cast<float>(d[1]), static_cast<float>(d[2]),
+                               id < 0 ? id : cells[id].run};
+            h.r1 = std::max(h.r1, static_cast<float>(norm) * 1.0001f);
+            h.r2 = std::max(h.r2, static_cast<float>(d[0] * d[0] + d[1] * d[1] + d[2] * d[2]) * 1.0001f);
         }
+        std::memcpy(run, &h, sizeof(h));
     }
-    for (int q = 0; q < 3; ++q) nbs[static_cast<size_t>(slots) + q].id = kVorHeader;  // padding
     const int64_t nb3 = static_cast<int64_t>(block_n) * block_n * block_n;
     std::vector<int32_t> boff(nb3 + 1, 0), bids;
     for (int64_t b = 0; b < nb3; ++b)
@@ -1199,6 +1264,7 @@ int skg_grid_voronoi(skg_engine* e, int64_t nsites, const double* sites, const i
         return st;
     if ((st = gridUpload(e, nbs.data(), nbs.size(), &g.vnb))) return st;
     if (!bids.empty() && (st = gridUpload(e, bids.data(), bids.size(), &g.vbl_id))) return st;
+    g.vscale = scale;
     g.vbn = block_n;
     for (int q = 0; q < 6; ++q) g.box[q] = box[q];
     double dx = box[3] - box[0], dy = box[4] - box[1], dz = box[5] - box[2];
@@ -1320,11 +1386,12 @@ int skg_trace_paths(skg_engine* e, const double* rays, int64_t n, int64_t cap, i
     HIPCHK(e, hipMalloc(&dRays, n * 6 * sizeof(double)));
     HIPCHK(e, hipMalloc(&dCnt, n * 2 * sizeof(int64_t)));
     HIPCHK(e, hipMemcpy(dRays, rays, n * 6 * sizeof(double), hipMemcpyHostToDevice));
-    int blocks = static_cast<int>((n + 255) / 256);
     GridView g = e->grid;
     g.dens = e->dens;
-    dispatchGrid(e, [&](auto gt) {
-        hipLaunchKernelGGL((trace_count<decltype(gt)::value>), dim3(blocks), dim3(256), planeBytes(g), e->stream, g, dRays, n, dCnt);
+    dispatchLanes(e, n, [&](auto gt, auto lanes) {
+        constexpr int GT = decltype(gt)::value, L = decltype(lanes)::value;
+        hipLaunchKernelGGL((trace_count<GT, L>), dim3(blocksFor(n * L)),
+                           dim3(256), planeBytes(g), e->stream, g, dRays, n, dCnt);
         return 0;
     });
     std::vector<int64_t> cnt(2 * n);
@@ -1352,9 +1419,10 @@ int skg_trace_paths(skg_engine* e, const double* rays, int64_t n, int64_t cap, i
     HIPCHK(e, hipMemcpy(dOff, hoff.data(), (n + 1) * sizeof(int64_t), hipMemcpyHostToDevice));
     if (t)
     {
-        dispatchGrid(e, [&](auto gt) {
-            hipLaunchKernelGGL((trace_write<decltype(gt)::value>), dim3(blocks), dim3(256), planeBytes(g), e->stream, g, dRays, n, dOff,
-                               dM, dDs);
+        dispatchLanes(e, n, [&](auto gt, auto lanes) {
+            constexpr int GT = decltype(gt)::value, L = decltype(lanes)::value;
+            hipLaunchKernelGGL((trace_write<GT, L>), dim3(blocksFor(n * L)),
+                               dim3(256), planeBytes(g), e->stream, g, dRays, n, dOff, dM, dDs);
             return 0;
         });
         HIPCHK(e, hipGetLastError());
@@ -1390,9 +1458,10 @@ int skg_trace_paths_noalloc(skg_engine* e, const double* rays, int64_t n, int64_
     if (n == 0) return SKG_OK;
     GridView g = e->grid;
     g.dens = e->dens;
-    const int blocks = static_cast<int>((n + 255) / 256);
-    dispatchGrid(e, [&](auto gt) {
-        hipLaunchKernelGGL((trace_count_off<decltype(gt)::value>), dim3(blocks), dim3(256), planeBytes(g), e->stream, g, rays, n, off);
+    dispatchLanes(e, n, [&](auto gt, auto lanes) {
+        constexpr int GT = decltype(gt)::value, L = decltype(lanes)::value;
+        hipLaunchKernelGGL((trace_count_off<GT, L>), dim3(blocksFor(n * L)),
+                           dim3(256), planeBytes(g), e->stream, g, rays, n, off);
         return 0;
     });
     hipLaunchKernelGGL(scan_block_sums, dim3(static_cast<unsigned>(nb)), dim3(256), 0, e->stream, off, n, e->scan);
@@ -1407,8 +1476,10 @@ int skg_trace_paths_noalloc(skg_engine* e, const double* rays, int64_t n, int64_
         return fail(e, SKG_ERR_CAPACITY, "skg_trace_paths_noalloc: capacity " + std::to_string(cap) + " < " + std::to_string(t));
     if (t)
     {
-        dispatchGrid(e, [&](auto gt) {
-            hipLaunchKernelGGL((trace_write<decltype(gt)::value>), dim3(blocks), dim3(256), planeBytes(g), e->stream, g, rays, n, off, m, ds);
+        dispatchLanes(e, n, [&](auto gt, auto lanes) {
+            constexpr int GT = decltype(gt)::value, L = decltype(lanes)::value;
+            hipLaunchKernelGGL((trace_write<GT, L>), dim3(blocksFor(n * L)),
+                               dim3(256), planeBytes(g), e->stream, g, rays, n, off, m, ds);
             return 0;
         });
         HIPCHK(e, hipGetLastError());
@@ -1444,16 +1515,16 @@ int skg_trace_tau(skg_engine* e, const double* rays, int64_t n, int32_t ell, dou
     }
     double section = e->hSext[ell];
     double taumax = L > 0 ? std::log(L) + 745 : -INFINITY;
-    int blocks = static_cast<int>((n + 255) / 256);
     GridView g = e->grid;
     g.dens = e->dens;
-    dispatchGrid(e, [&](auto gt) {
+    dispatchLanes(e, n, [&](auto gt, auto lanes) {
+        constexpr int GT = decltype(gt)::value, L = decltype(lanes)::value;
         if (fp_mode == SKG_FP64)
-            hipLaunchKernelGGL((trace_tau<decltype(gt)::value, SKG_FP64>), dim3(blocks), dim3(256), planeBytes(g), e->stream, g, e->dens,
-                               e->dens32, section, taumax, dRays, n, dTp, dTo, dToff, dCum);
+            hipLaunchKernelGGL((trace_tau<GT, SKG_FP64, L>), dim3(blocksFor(n * L)),
+                               dim3(256), planeBytes(g), e->stream, g, e->dens, e->dens32, section, taumax, dRays, n, dTp, dTo, dToff, dCum);
         else
-            hipLaunchKernelGGL((trace_tau<decltype(gt)::value, SKG_FP32_KAHAN>), dim3(blocks), dim3(256), planeBytes(g), e->stream, g,
-                               e->dens, e->dens32, section, taumax, dRays, n, dTp, dTo, dToff, dCum);
+            hipLaunchKernelGGL((trace_tau<GT, SKG_FP32_KAHAN, L>), dim3(blocksFor(n * L)),
+                               dim3(256), planeBytes(g), e->stream, g, e->dens, e->dens32, section, taumax, dRays, n, dTp, dTo, dToff, dCum);
         return 0;
     });
     HIPCHK(e, hipGetLastError());
@@ -1944,29 +2015,8 @@ static int runPersistent(skg_engine* e, uint64_t first_history, uint64_t count)
     p.gframe = e->gframe;
     p.guideMix = e->guideMix;
     p.contKey = e->contKey;
-    // the cell of the point source, the start hint of every new packet: found once per grid and
-    // source.  (On a mesh grid a packet without a hint scans its block's candidates, hundreds of them
-    // around a dense centre: 43 % of the batched tetra launch went into that scan.)
-    if (e->gridType != SKG_GRID_CARTESIAN && !e->srcHintValid)
-    {
-        int* d = nullptr;
-        HIPCHK(e, hipMalloc(&d, sizeof(int)));
-        (void)hipGetLastError();  // a launch error below is then this launch's own
-        const auto& r = e->src;
-        if (e->gridType == SKG_GRID_OCTREE)
-            hipLaunchKernelGGL(locate_cell<kOctree>, dim3(1), dim3(64), 0, e->stream, e->grid, r[0], r[1], r[2], d);
-        else if (e->gridType == SKG_GRID_VORONOI)
-            hipLaunchKernelGGL(locate_cell<kVoronoi>, dim3(1), dim3(64), 0, e->stream, e->grid, r[0], r[1], r[2], d);
-        else
-            hipLaunchKernelGGL(locate_cell<kTetra>, dim3(1), dim3(64), 0, e->stream, e->grid, r[0], r[1], r[2], d);
-        hipError_t st = hipGetLastError();
-        if (st == hipSuccess) st = hipMemcpyAsync(&e->srcHint, d, sizeof(int), hipMemcpyDeviceToHost, e->stream);
-        if (st == hipSuccess) st = hipStreamSynchronize(e->stream);
-        hipFree(d);
-        if (st != hipSuccess) return fail(e, SKG_ERR_DEVICE, std::string("source cell: ") + hipGetErrorString(st));
-        e->srcHintValid = true;
-    }
-    p.srcHint = e->gridType == SKG_GRID_CARTESIAN ? -1 : e->srcHint;
+    if (int st = sourceHint(e)) return st;
+    p.srcHint = e->srcHint;
     p.rf = e->rf;
     p.persp = 0;
     for (const auto& f : e->frames) p.persp |= f.persp;
@@ -1999,17 +2049,18 @@ static int runPersistent(skg_engine* e, uint64_t first_history, uint64_t count)
     // spread over that many, with fewer lanes of each: a wave waits for the longest of its lanes
     // at every step, and 4096 packets in full wavefronts would use 16 of the 256 CUs (Cartesian
     // 32^3, 4096 packets: 0.92 -> 0.64 ms).  Below four lanes the waves only add up.
+    const int lanes = pathLanes(e, count);
     p.lanes = static_cast<int>(
-        std::clamp<int64_t>((static_cast<int64_t>(count) + 8 * e->cus - 1) / (8 * e->cus), 4, 64));
+        std::clamp<int64_t>((static_cast<int64_t>(count) + 8 * e->cus - 1) / (8 * e->cus), 4, 64 / lanes));
     const int64_t perBlock = static_cast<int64_t>(p.lanes) * (threads / 64);
     int64_t needBlocks = (static_cast<int64_t>(count) + perBlock - 1) / perBlock;
     blocks = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(blocks, needBlocks)));
     HIPCHK(e, hipEventRecord(e->ev0, e->stream));
     hipError_t err;
-    dispatchGrid(e, [&](auto gt) {
-        constexpr int GT = decltype(gt)::value;
-        err = e->fpMode == SKG_FP64 ? launchLifecycle<GT, SKG_FP64>(p, guided, blocks, threads, e->stream)
-                                    : launchLifecycle<GT, SKG_FP32_KAHAN>(p, guided, blocks, threads, e->stream);
+    dispatchLanes(e, static_cast<int64_t>(count), [&](auto gt, auto nl) {
+        constexpr int GT = decltype(gt)::value, L = decltype(nl)::value;
+        err = e->fpMode == SKG_FP64 ? launchLifecycle<GT, SKG_FP64, L>(p, guided, blocks, threads, e->stream)
+                                    : launchLifecycle<GT, SKG_FP32_KAHAN, L>(p, guided, blocks, threads, e->stream);
         return 0;
     });
     if (err != hipSuccess) return fail(e, SKG_ERR_DEVICE, std::string("lifecycle launch: ") + hipGetErrorString(err));
@@ -2120,6 +2171,8 @@ namespace
         int st = ensurePool(e, slots, qcap);
         if (st) return st;
         PipeParams p{};
+        if ((st = sourceHint(e))) return st;
+        p.srcHint = e->srcHint;
         p.grid = e->grid;
         p.grid.dens = e->dens;
     p.grid.dens = e->dens;

@@ -38,7 +38,7 @@ namespace skg
         double xi, min_weight_reduction;
         int min_scatt;
         int threshold;
-        int lanes;  // lanes of each wavefront that take packets
+        int lanes;  // packets that each wavefront takes at a time (lanes per packet: L)
         uint64_t seed;
         uint64_t first, count;
         unsigned long long* queue;     // next history offset (work queue head)
@@ -219,12 +219,33 @@ namespace skg
         double section, lim, slim, rfL;
         int64_t off;
         double v;
+
+        // the traversal of the first of each group of L lanes to the whole group
+        template<int L, int V> __device__ __forceinline__ void share()
+        {
+            if constexpr (L > 1)
+            {
+                phase = group_first<L>(phase);
+                hint = group_first<L>(hint);
+                kx = group_first<L>(kx);
+                ky = group_first<L>(ky);
+                kz = group_first<L>(kz);
+                section = group_first<L>(section);
+                lim = group_first<L>(lim);
+                if constexpr (V == kPersp || V == kStoreRF) slim = group_first<L>(slim);
+                if constexpr (V == kStoreRF)
+                {
+                    ell = group_first<L>(ell);
+                    rfL = group_first<L>(rfL);
+                }
+            }
+        }
     };
 
-    // traversal state of one lane: the generator, the running sums and the phase
-    template<int GT, int FP> struct Trav
+    // traversal state of one lane: the generator, the running sums and the phase (L lanes per packet)
+    template<int GT, int FP, int L> struct Trav
     {
-        Gen<GT> gen;
+        Gen<GT, L> gen;
         int phase;
         bool ended;
         int steps;
@@ -261,9 +282,15 @@ namespace skg
                 s32.add(static_cast<float>(ds));
         }
 
+        // the lane that acts for its packet (events, counts, sums in memory); the packet's other lanes
+        // have the same traversal state
+        static __device__ __forceinline__ bool lead() { return L == 1 || threadIdx.x % L == 0; }
+
         __device__ __forceinline__ void finish(LdsU32* lds)
         {
             ended = true;
+            gen.idle();
+            if (!lead()) return;
             // the crossing counters are added once, where a traversal ends
             lds_count(lds + 4, static_cast<uint32_t>(steps));
             if (phase == kFwd2) lds_count(lds + 7, static_cast<uint32_t>(steps));
@@ -318,7 +345,7 @@ namespace skg
         template<bool RF, bool PERSP>
         __device__ __forceinline__ void step(const GridView& grid, LdsU32* lds, double* rf, int nl)
         {
-            const int at = gen.i;  // the octree's leaves are named by their node, other cells by m
+            const int at = gen.i;  // the octree's leaves are named by their node, Voronoi cells by their run, others by m
             int m;
             double ds, nd;
             const int r = gen.cross(grid, m, ds, nd);
@@ -341,7 +368,7 @@ namespace skg
                     if (!peel)
                     {
                         add_length(ds);
-                        last = GT == kOctree ? at : m;
+                        last = GT == kOctree || GT == kVoronoi ? at : m;
                         if constexpr (RF)
                         {
                             if (phase == kFwd1)
@@ -349,7 +376,7 @@ namespace skg
                                 const double lnEnd = -tau_value();
                                 const double extEnd = exp(lnEnd);
                                 const double em = ln_mean(extEnd, rfExt, lnEnd, -tprev);
-                                unsafeAtomicAdd(rf + static_cast<int64_t>(m) * nl + ell, rfL * em * ds);
+                                if (lead()) unsafeAtomicAdd(rf + static_cast<int64_t>(m) * nl + ell, rfL * em * ds);
                                 rfExt = extEnd;
                             }
                         }
@@ -763,7 +790,10 @@ namespace skg
             // the interaction's cell and distance, or beyond the last segment that segment's
             const int m = last;
             double n = 0.;
-            if (m >= 0) n = GT == kOctree ? p.grid.node[m].dens : p.dens[m];
+            if (m >= 0)
+                n = GT == kOctree    ? p.grid.node[m].dens
+                    : GT == kVoronoi ? reinterpret_cast<const VorHead*>(p.grid.vnb + m)->dens
+                                     : p.dens[m];
             double ss = INST ? p.ssca[pk.ell] * p.inst[pk.inst].scale : p.ssca[pk.ell];
             double se = INST ? p.sext[pk.ell] * p.inst[pk.inst].scale : p.sext[pk.ell];
             double ksca = n > 0. ? n * ss : 0.;
@@ -849,12 +879,12 @@ namespace skg
     //   octree, nine levels, 40 wavelengths, 3e5    8.4 /  8.4 /  8.1  events double the writes)
     //   octree with the radiation field, 2e5        7.8 / 11.6 / 13.2 (bound by its atomics, whose
     //   Cartesian with the field, 7e5              targets collide more with more waves)
-    // Voronoi and tetra as measured before the events became calls: 1152 / 1086 / 1061 ms and
-    // 6.72 / 5.80 / 5.27 s.  The guided variant's network call holds whole layers' weights in
-    // registers, and its four-wave build does not compile for the mesh grids.
+    //   Voronoi, 400 000 sites, 2^18 packets         - / 48.0 / 52.8
+    //   tetra, before the events became calls      6720 / 5800 / 5270
+    // The guided variant's network call holds whole layers' weights in registers, and its four-wave build does not compile for the mesh grids.
     template<int GT, int V> constexpr int lifecycle_waves()
     {
-        return V == kGuided || V == kStoreRF ? 2 : GT == kOctree ? 3 : GT == kCartesian ? 3 : 4;
+        return V == kGuided || V == kStoreRF ? 2 : GT == kOctree ? 3 : GT == kTetra ? 4 : 3;
     }
 
     // The kernel's parameter block where it lies in the kernarg segment, behind a pointer the
@@ -869,7 +899,7 @@ namespace skg
         return *(const SimParams*)q;
     }
 
-    template<int GT, int FP, int V>
+    template<int GT, int FP, int V, int L>
     __global__ void __launch_bounds__(kLcThreads, (lifecycle_waves<GT, V>())) lifecycle(SimParams p)
     {
         constexpr bool PERSP = V == kPersp || V == kStoreRF;
@@ -882,13 +912,15 @@ namespace skg
         if (threadIdx.x < kNumCounters) wgcnt[threadIdx.x] = 0;
         stage_planes<GT>(p.grid);
         __syncthreads();  // the counters are zero before any wave adds to them
-        const int t = threadIdx.x;
+        const int t = threadIdx.x / L;
         const int lane = lane_id();
-        Trav<GT, FP> T;
+        const bool lead = Trav<GT, FP, L>::lead();
+        Trav<GT, FP, L> T;
         // the lanes that take packets (all of them unless the run is small); a lane without one
         // waits in kFetch
-        T.phase = lane < p.lanes ? kFetch : kDone;
+        T.phase = lane / L < p.lanes ? kFetch : kDone;
         T.ended = false;
+        T.gen.idle();
         T.last = -1;
         T.tau = T.s = T.lim = 0.;
         T.tau32.reset();
@@ -906,7 +938,7 @@ namespace skg
                 uint64_t hist = 0;
                 bool event = T.ended, go = false;
                 // new histories for the lanes without one, with one atomic per wavefront
-                const unsigned long long need = __ballot(T.phase == kFetch);
+                const unsigned long long need = __ballot(T.phase == kFetch && lead);
                 if (need)
                 {
                     const int leader = __ffsll(static_cast<long long>(need)) - 1;
@@ -915,7 +947,7 @@ namespace skg
                     base = __shfl(base, leader);
                     if (T.phase == kFetch)
                     {
-                        const unsigned long long mine = base + __popcll(need & ((1ull << lane) - 1ull));
+                        const unsigned long long mine = base + __popcll(need & ((1ull << (lane & -L)) - 1ull));
                         hist = kp.first + mine;
                         event = mine < kp.count;
                         if (!event) T.phase = kDone;
@@ -923,10 +955,14 @@ namespace skg
                 }
                 if (event)
                 {
-                    life_event<GT, V>(&kp, T.phase, T.last, T.tau_value(), T.s_end(T.tau_value() > T.lim), hist, io, cd, cu,
-                                      cnt, t);
-                    off = io.off;
-                    v = io.v;
+                    if (lead)
+                    {
+                        life_event<GT, V>(&kp, T.phase, T.last, T.tau_value(), T.s_end(T.tau_value() > T.lim), hist, io, cd,
+                                          cu, cnt, t);
+                        off = io.off;
+                        v = io.v;
+                    }
+                    io.template share<L, V>();
                     T.phase = io.phase;
                     T.ended = false;
                     go = io.phase == kPeel || io.phase == kFwd1 || io.phase == kFwd2;
@@ -935,9 +971,9 @@ namespace skg
                 {
                     // one network evaluation for the lanes of the wave that wait to scatter, once
                     // there are kGuideLanes of them or no lane of the wave is still traversing
-                    const bool sc = T.phase == kScatter;
+                    const bool sc = T.phase == kScatter && lead;
                     const unsigned long long scm = __ballot(sc);
-                    if (scm && (__popcll(scm) >= kGuideLanes || __ballot(go || busy) == 0))
+                    if (scm && (__popcll(scm) >= kGuideLanes / L || __ballot(go || busy) == 0))
                     {
                         float feat[kGuideIn];
                         for (int q = 0; q < kGuideIn; ++q) feat[q] = 0.f;
@@ -947,15 +983,21 @@ namespace skg
                                            cd[cKz * kLcThreads + t], cd[cLam * kLcThreads + t], feat);
                         float o[kGuideOut];
                         guide_wave_infer_regs(kp.net, feat, sc, o);
-                        if (sc)
+                        if (T.phase == kScatter)
                         {
-                            life_guided<GT>(&kp, o, io, cd, cu, cnt, t);
+                            if (sc) life_guided<GT>(&kp, o, io, cd, cu, cnt, t);
+                            io.template share<L, V>();
                             T.phase = io.phase;
                             go = true;
                         }
                     }
                 }
                 flush_deposits(kp.frame, off, v, cnt);  // the wave is converged here
+                if (!go && T.gen.asks() && !T.ended)
+                {
+                    T.gen.resolve(kp.grid);
+                    busy = true;
+                }
                 if (go)
                 {
                     T.template start<PERSP>(kp.grid, io, cd, cu, cnt, t);
@@ -978,7 +1020,7 @@ namespace skg
                 if (busy)
                 {
                     T.template step<V == kStoreRF, PERSP>(kernel_params().grid, cnt, kernel_params().rf, kernel_params().nlambda);
-                    busy = !T.ended;
+                    busy = !T.ended && !T.gen.asks();
                 }
             }
         }

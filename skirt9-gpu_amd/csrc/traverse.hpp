@@ -26,34 +26,55 @@ namespace skg
         kTetra = 3
     };
 
-    // Voronoi cell record (64 bytes, indexed by cell): the site, the cell's number density and
-    // its run in the entry table (begin: the run's header slot; count: its neighbour entries).
-    // Read at a path's start; a crossing reads only the entry table.
-    struct alignas(64) VorCell
+    // Voronoi cell record (indexed by cell, for the search of a position's cell): the site and the
+    // cell's run in the entry table.
+    struct alignas(32) VorCell
     {
         double x, y, z;
-        double dens;
-        int32_t begin, count;
-        int32_t pad[6];
-    };
-    static_assert(sizeof(VorCell) == 64, "Voronoi cell record must be 64 bytes");
-
-    // The entry table holds one run per cell: a header slot (id kVorHeader, x = the cell's
-    // number density, run = the number of neighbour entries) followed by one entry (32 bytes)
-    // per neighbour: the neighbour's site, its id and the header slot of its own run.  A cell's
-    // exit search streams through its run, and the entry it leaves through gives the next
-    // cell's site and run, so a crossing makes one dependent read (the run) instead of two (the
-    // cell record, then its neighbours).  Domain walls have ids -1..-6 (xmin, xmax, ymin, ymax,
-    // zmin, zmax) and run -1.  The table ends with 3 slots of padding (a run is read from its
-    // header in groups of four slots).
-    struct alignas(32) VorNb
-    {
-        double x, y, z;
-        int32_t id;
         int32_t run;
+        int32_t pad;
     };
-    static_assert(sizeof(VorNb) == 32, "Voronoi neighbour entry must be 32 bytes");
-    constexpr int32_t kVorHeader = -100;
+    static_assert(sizeof(VorCell) == 32, "Voronoi cell record must be 32 bytes");
+
+    // The entry table holds one run of 16-byte slots per cell, at a multiple of four slots: the
+    // cell's head (three slots), then one entry per neighbour, padded with NaN (which the exit
+    // search rejects) to at least kVorPad.  A crossing reads the run of the
+    // cell that it enters and nothing else, all of it in flight at once.
+    struct alignas(16) VorHead
+    {
+        double x, y, z;   // the site
+        double dens;
+        int32_t count;    // neighbours
+        int32_t cell;
+        float r2, r1;     // the largest squared length and 1-norm of the neighbours' offsets
+    };
+    static_assert(sizeof(VorHead) == 48 && offsetof(VorHead, dens) == 24 && offsetof(VorHead, count) == 32,
+                  "head layout that VorRun reads");
+    // The neighbour's site relative to the cell's, in units of the domain's largest side and rounded
+    // to FP32, and the neighbour's run (its first slot).  Domain walls have ids -1..-6 (xmin, xmax,
+    // ymin, ymax, zmin, zmax) and the site's mirror image as their site.  The exit search bounds
+    // every neighbour's exit distance in FP32 and computes the FP64 distance of the only one that
+    // can be the smallest: 16 bytes instead of 32 per neighbour, and one FP64 division per crossing.
+    struct alignas(16) VorNb
+    {
+        float x, y, z;
+        int32_t id;
+    };
+    static_assert(sizeof(VorNb) == 16, "Voronoi neighbour entry must be 16 bytes");
+    constexpr int kVorPad = 12;  // entries every run has room for
+    // entries a lane has in flight where L lanes share a path (400 000 sites, 2^18 packets, L = 1 with
+    // 6 / 8 / 10 / 12: 47.7 / 48.5 / 49.6 / 49.6 ms)
+    template<int L> constexpr int kVorAhead = L == 4 ? 5 : 8;
+    constexpr int kVorSlack = 32;  // slots behind the last run that may be read (and are not used)
+    // relative error allowed to the FP32 bounds: the offsets, the position and five operations are
+    // each rounded to within 2^-24 of products that (n.n + w.w) or |n| |k| bound, in sum below 2^-21
+    constexpr float kVorEps = 0x1p-19f;
+    // offsets shorter than this (of the largest of the domain's side and its coordinates) are stored
+    // as zero: the FP64 distances themselves are less exact there than the FP32 bounds assume, and a
+    // zero offset always takes the exact search
+    constexpr double kVorMinOffset = 0x1p-28;
+    constexpr int kVorNone = -99;  // no exit
+    constexpr int kVorAsk = -98;   // not decided yet (Gen::resolve)
 
     // Tetrahedron record (256 bytes, two cache lines, indexed by cell): vertex coordinates,
     // density and face links in the first line, the outward unit face normals in the second.
@@ -129,6 +150,7 @@ namespace skg
         // blocks of cell ids, in the reference's order)
         const VorCell* vcell;
         const VorNb* vnb;
+        double vscale;  // 1 / the domain's largest side
         int vbn;
         const int32_t* vbl_off;
         const int32_t* vbl_id;
@@ -156,51 +178,46 @@ namespace skg
         return i * n * n + j * n + k;
     }
 
-    // VoronoiMeshSnapshot::cellIndex: nearest site among the block's candidates, squared
-    // distance (r - site).norm2(), strict '<' (the first of equal distances wins)
-    __device__ __forceinline__ int vor_cell_index(const GridView& g, double x, double y, double z)
+    // the candidates' nearest site to a position, squared distance (r - site).norm2(), strict '<' (the
+    // first of equal distances wins), four candidates in flight: its run, -1 if there is none
+    __device__ __attribute__((noinline)) int vor_nearest(const VorCell* cell, const int32_t* ids, int q, int e, double x,
+                                                         double y, double z)
+    {
+        int run = -1;
+        double best = DBL_MAX;
+        for (; q < e; q += 4)
+        {
+            int c[4];
+            double d[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) c[u] = ids[min(q + u, e - 1)];
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+            {
+                const VorCell C = cell[c[u]];
+                const double dx = x - C.x, dy = y - C.y, dz = z - C.z;
+                d[u] = dx * dx + dy * dy + dz * dz;
+                c[u] = C.run;
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u)  // (the last candidate again where fewer than four are left)
+                if (d[u] < best)
+                {
+                    best = d[u];
+                    run = c[u];
+                }
+        }
+        return run;
+    }
+
+    // VoronoiMeshSnapshot::cellIndex: the run of the cell with the nearest site among the block's
+    // candidates, -1 outside the domain
+    __device__ __forceinline__ int vor_find(const GridView& g, double x, double y, double z)
     {
         if (!(x >= g.box[0] && x <= g.box[3] && y >= g.box[1] && y <= g.box[4] && z >= g.box[2] && z <= g.box[5]))
             return -1;
         const int b = vor_block(g, x, y, z);
-        int m = -1;
-        double best = DBL_MAX;
-        for (int q = g.vbl_off[b], e = g.vbl_off[b + 1]; q < e; ++q)
-        {
-            const int id = g.vbl_id[q];
-            const VorCell& c = g.vcell[id];
-            double dx = x - c.x, dy = y - c.y, dz = z - c.z;
-            double d = dx * dx + dy * dy + dz * dz;
-            if (d < best)
-            {
-                best = d;
-                m = id;
-            }
-        }
-        return m;
-    }
-
-    // True when the point lies in the domain and is nearer to the site of cell h than to each
-    // of h's neighbouring sites by a relative margin far above the rounding of the squared
-    // distances.  Inside the domain, the cell is the set of points nearer to its site than to
-    // the sites across its faces, so h's site is then the unique nearest site: the cell that
-    // VoronoiMeshSnapshot::cellIndex (and vor_cell_index) returns.
-    __device__ __forceinline__ bool vor_nearest_strict(const GridView& g, int h, double x, double y, double z)
-    {
-        if (!(x >= g.box[0] && x <= g.box[3] && y >= g.box[1] && y <= g.box[4] && z >= g.box[2] && z <= g.box[5]))
-            return false;
-        const VorCell& C = g.vcell[h];
-        const double hx = x - C.x, hy = y - C.y, hz = z - C.z;
-        const double dh = hx * hx + hy * hy + hz * hz;
-        for (int q = C.begin + 1, e = C.begin + 1 + C.count; q < e; ++q)
-        {
-            const VorNb E = g.vnb[q];
-            if (E.id < 0) continue;
-            const double ex = x - E.x, ey = y - E.y, ez = z - E.z;
-            const double dj = ex * ex + ey * ey + ez * ez;
-            if (!(dj - dh > 1e-12 * (dj + dh))) return false;
-        }
-        return true;
+        return vor_nearest(g.vcell, g.vbl_id, g.vbl_off[b], g.vbl_off[b + 1], x, y, z);
     }
 
     // number of borders <= v, minus one, clipped to a block index
@@ -437,23 +454,166 @@ namespace skg
         return OctNext{c == i ? -1 : c, x, y, z};
     }
 
-    template<int GT> struct Gen
+    struct VorExit
+    {
+        int id;
+        double s;
+    };
+
+    // Exit distance through the bisector plane between the sites p and e (0 where the plane is
+    // not ahead), or through domain wall id (VoronoiMeshSnapshot.cpp:1119-1170)
+    __device__ __forceinline__ double vor_bisector(double px, double py, double pz, double ex, double ey, double ez,
+                                                   double rx, double ry, double rz, double kx, double ky, double kz)
+    {
+        const double nx = ex - px, ny = ey - py, nz = ez - pz;
+        const double ndotk = nx * kx + ny * ky + nz * kz;
+        if (!(ndotk > 0)) return 0.;
+        const double qx = 0.5 * (ex + px), qy = 0.5 * (ey + py), qz = 0.5 * (ez + pz);
+        return (nx * (qx - rx) + ny * (qy - ry) + nz * (qz - rz)) / ndotk;
+    }
+    __device__ __forceinline__ double vor_wall(const double* box, int id, double rx, double ry, double rz, double kx,
+                                               double ky, double kz)
+    {
+        const int w = -1 - id;  // 0..5: xmin, xmax, ymin, ymax, zmin, zmax
+        if (w >= 6) return 0.;
+        const double face = w == 0 ? box[0] : w == 1 ? box[3] : w == 2 ? box[1] : w == 3 ? box[4] : w == 4 ? box[2] : box[5];
+        const double r = pick3(w < 2, w < 4, rx, ry, rz), k = pick3(w < 2, w < 4, kx, ky, kz);
+        return (face - r) / k;
+    }
+
+    // The exit of the cell with the run at slot i from the exact distances of all its neighbours:
+    // the smallest positive one, the first of equal ones (kVorNone if none is positive).  Called
+    // where the FP32 bounds leave more than one neighbour, and kept out of the crossing's registers.
+    __device__ __attribute__((noinline)) int vor_exit_exact(const VorNb* nb, double b0, double b1, double b2, double b3,
+                                                            double b4, double b5, int i, double rx, double ry, double rz,
+                                                            double kx, double ky, double kz)
+    {
+        const double box[6] = {b0, b1, b2, b3, b4, b5};
+        const VorHead& C = *reinterpret_cast<const VorHead*>(nb + i);
+        int out = kVorNone;
+        double best = DBL_MAX;
+        for (int q = i + 3; q < i + 3 + C.count; ++q)
+        {
+            const int id = nb[q].id;
+            double s;
+            if (id >= 0)
+            {
+                const VorHead& N = *reinterpret_cast<const VorHead*>(nb + id);
+                s = vor_bisector(C.x, C.y, C.z, N.x, N.y, N.z, rx, ry, rz, kx, ky, kz);
+            }
+            else
+                s = vor_wall(box, id, rx, ry, rz, kx, ky, kz);
+            if (s > 0 && s < best)
+            {
+                best = s;
+                out = id;
+            }
+        }
+        return out;
+    }
+
+    // the value of the first of each group of L lanes (1 or 4), in every lane of the group
+    template<int L> __device__ __forceinline__ int group_first(int v)
+    {
+        if constexpr (L == 1) return v;
+        return __builtin_amdgcn_update_dpp(v, v, 0x00, 0xF, 0xF, true);  // quad_perm 0 0 0 0
+    }
+    template<int L> __device__ __forceinline__ double group_first(double v)
+    {
+        return __hiloint2double(group_first<L>(__double2hiint(v)), group_first<L>(__double2loint(v)));
+    }
+
+    // a cell's run: the head, and the lane's entries of the first L * kVorAhead<L>
+    template<int L> struct VorRun
+    {
+        double2 a, b;
+        float4 c;
+        float4 f[kVorAhead<L>];
+        __device__ __forceinline__ void load_entries(const VorNb* p)
+        {
+#pragma unroll
+            for (int u = 0; u < kVorAhead<L>; ++u) f[u] = *reinterpret_cast<const float4*>(p + u * L);
+        }
+        __device__ __forceinline__ void load(const GridView& g, int slot, int sub)
+        {
+            const VorNb* p = g.vnb + slot;
+            a = *reinterpret_cast<const double2*>(p);
+            b = *reinterpret_cast<const double2*>(p + 1);
+            c = *reinterpret_cast<const float4*>(p + 2);
+            load_entries(p + 3 + sub);
+        }
+        __device__ __forceinline__ int count() const { return __float_as_int(c.x); }
+        __device__ __forceinline__ int cell() const { return __float_as_int(c.y); }
+    };
+
+    // The exit search in FP32 (lengths in units of the domain's side).  With the offset n of a
+    // neighbour's site and w of the position from the cell's site, the bisector is at the distance
+    // a = n.(n / 2 - w) / n.k.  The numerator is off by at most En = eps (r2 + w.w) and the
+    // denominator by Ed = eps r1 |k|, with the cell's largest n.n (r2) and 1-norm (r1); where the
+    // denominator exceeds 4 Ed, a is then off by at most 2 (En + a Ed) / n.k.  A denominator within
+    // 4 Ed of zero makes the neighbour an exit at any distance, a smaller one makes it no exit.
+    struct VorSearch
+    {
+        float wx, wy, wz, fx, fy, fz, en2, ed2, ed4;
+        float l1, l2, a1, mn;  // the two smallest lower bounds, the first one's distance; the smallest numerator
+        int id;
+
+        // valid: the entry is one (false: read past the end of the run)
+        __device__ __forceinline__ void entry(const float4& v, bool valid)
+        {
+            const float num = fmaf(v.x, fmaf(0.5f, v.x, -wx), fmaf(v.y, fmaf(0.5f, v.y, -wy), v.z * fmaf(0.5f, v.z, -wz)));
+            const float den = fmaf(v.x, fx, fmaf(v.y, fy, v.z * fz));
+            const float r = __builtin_amdgcn_rcpf(den), a = num * r;
+            float lb = fmaf(-r, fmaf(a, ed2, en2), a);
+            lb = valid && den > ed4 ? lb : INFINITY;
+            lb = valid && fabsf(den) <= ed4 ? -1.f : lb;
+            const bool first = lb < l1;
+            l2 = __builtin_amdgcn_fmed3f(l1, lb, l2);
+            l1 = first ? lb : l1;
+            a1 = first ? a : a1;
+            id = first ? __float_as_int(v.w) : id;
+            mn = fminf(mn, valid ? num : INFINITY);
+        }
+
+        // with the search of the lane that quad_perm CTRL names
+        template<int CTRL> __device__ __forceinline__ void merge()
+        {
+            const float ol1 = other<CTRL>(l1), ol2 = other<CTRL>(l2), oa1 = other<CTRL>(a1);
+            const int oid = __builtin_amdgcn_update_dpp(id, id, CTRL, 0xF, 0xF, true);
+            mn = fminf(mn, other<CTRL>(mn));
+            l2 = fminf(fminf(l2, ol2), fmaxf(l1, ol1));
+            const bool first = ol1 < l1;
+            l1 = first ? ol1 : l1;
+            a1 = first ? oa1 : a1;
+            id = first ? oid : id;
+        }
+        template<int CTRL> static __device__ __forceinline__ float other(float v)
+        {
+            const int w = __float_as_int(v);
+            return __int_as_float(__builtin_amdgcn_update_dpp(w, w, CTRL, 0xF, 0xF, true));
+        }
+    };
+
+    // L: the lanes that walk a path together, all with the same state (Voronoi: each searches a share
+    // of the neighbours)
+    template<int GT, int L = 1> struct Gen
     {
         double rx, ry, rz, kx, ky, kz;
         int state;
-        int i, j, k;  // Cartesian: entry of the border ahead on each axis in the planes table; octree: i = current leaf's node; Voronoi, tetra: i =
-                      // current cell (tetra: j = entering face, -1 if unknown; Voronoi: j = the
-                      // header slot of the cell's run in the entry table)
+        int i, j, k;  // Cartesian: entry of the border ahead on each axis in the planes table; octree: i = current leaf's node; Voronoi: i = the
+                      // current cell's run, j = the run or wall behind its exit, k = the
+                      // steps without exit; tetra: i = current
+                      // cell, j = entering face, -1 if unknown
         double sx, sy, sz;      // Voronoi: the current cell's site
         double ikx, iky, ikz;   // Cartesian, octree: reciprocals of the direction
-        double b0, b1, b2, bn;  // Cartesian, octree: the current cell's wall ahead on each axis, its
-                                // density
+        double b0, b1, b2;      // Cartesian, octree: the current cell's wall ahead on each axis
+        double bn;              // Cartesian, octree, Voronoi: its density
         int f0, f1, f2;         // octree: the node across each of those walls
-        int cell;               // Cartesian, octree: the current cell's index
+        int cell;               // Cartesian, octree, Voronoi: the current cell's index
         uint32_t pend;  // octree: a node to descend into next and the crossed wall (node << 3 | wall),
                         // or kNoPend
         int hint;  // a cell that probably contains the start point (-1: none), after the first step
-                   // the start cell: octree a node, Voronoi and tetra a cell, Cartesian the cell's
+                   // the start cell: octree a node, Voronoi a run, tetra a cell, Cartesian the cell's
                    // indices i | j << 10 | k << 20 (no more than 1024 cells along an axis)
         static constexpr uint32_t kNoPend = 0xFFFFFFFFu;  // node ids stay below 2^29
 
@@ -708,19 +868,24 @@ namespace skg
             else
             {
                 if constexpr (GT == kVoronoi)
-                    i = hint >= 0 && vor_nearest_strict(g, hint, rx, ry, rz) ? hint : vor_cell_index(g, rx, ry, rz);
+                {
+                    // the first step enters the cell, and finds out whether the hint is right
+                    i = hint >= 0 ? kVorHinted : kVorEnter;
+                    if (hint < 0) hint = vor_find(g, rx, ry, rz);
+                    j = hint;
+                    k = 0;
+                }
                 else
+                {
                     i = hint >= 0 && tet_inside_strict(g.tcell[hint], rx, ry, rz) ? hint : tet_cell_index(g, rx, ry, rz);
-                hint = i;
-                if (i < 0)
+                    hint = i;
+                    j = -1;
+                }
+                if (hint < 0)
                 {
                     state = kOutside;
                     return false;
                 }
-                if constexpr (GT == kVoronoi)
-                    vor_enter(g, i);
-                else
-                    j = -1;
             }
             return true;
         }
@@ -732,13 +897,13 @@ namespace skg
         {
             if constexpr (GT == kOctree)
                 return cross_octree(g, m, ds, n);
+            else if constexpr (GT == kVoronoi)
+                return cross_voronoi(g, m, ds, n);
             else
             {
                 bool more;
                 if constexpr (GT == kCartesian)
                     more = next_cartesian(g, m, ds, n);
-                else if constexpr (GT == kVoronoi)
-                    more = next_voronoi(g, m, ds, n);
                 else
                     more = next_tetra(g, m, ds, n);
                 return !more ? -1 : state == kOutside ? 2 : 1;
@@ -748,6 +913,12 @@ namespace skg
         // One step of a path from its start on, as cross(); the first step begins the path and
         // returns its segment before the domain, if any (m = -1).
         __device__ __forceinline__ int advance(const GridView& g, int& m, double& ds, double& n)
+        {
+            if (state == kInside && asks()) resolve(g);
+            return step(g, m, ds, n);
+        }
+        // likewise, where the caller looks after asks()
+        __device__ __forceinline__ int step(const GridView& g, int& m, double& ds, double& n)
         {
             if (state == kOutside) return -1;
             if (state == kUnknown)
@@ -763,14 +934,6 @@ namespace skg
                 }
             }
             return cross(g, m, ds, n);
-        }
-
-        // The next segment of a path; false when it has no more.
-        __device__ __forceinline__ bool next(const GridView& g, int& m, double& ds, double& n)
-        {
-            int r;
-            while ((r = advance(g, m, ds, n)) == 0) {}
-            return r > 0;
         }
 
         __device__ __forceinline__ static double border(const GridView& g, int q)
@@ -834,117 +997,123 @@ namespace skg
             return true;
         }
 
-        // the cell c becomes the current cell, from its record: its site and its run
-        __device__ __forceinline__ void vor_enter(const GridView& g, int c)
+        // One step of the Voronoi generator (VoronoiMeshSnapshot.cpp:1119-1210): the crossing of the
+        // current cell through its exit, found by the step before, and the search of the exit of the
+        // cell behind it; the first step only does the latter.  Returns as cross() does.
+        //
+        // Bound by the vector memory path: the runs of the lanes lie apart, so each 16-byte load
+        // returns at about one lane a cycle (the return path was busy 80 % of the time with FP64
+        // sites), then by the latency of the run's lines, as the table does not fit the L2.  Hence
+        // 16-byte entries and one dependent read per step: the entries name their neighbours' runs,
+        // not their cells, and the exact exit distance takes the neighbour's site from the run that
+        // is read anyway.  400 000 sites, 2^18 packets, tau 5: 90 -> 48 ms; 1500 crossings in a row
+        // (2000 paths, 60 000 sites) with four lanes each: 1.3 -> 0.6 ms.
+        static constexpr int kVorHinted = -1, kVorEnter = -2;  // i before the first step
+        __device__ __forceinline__ int cross_voronoi(const GridView& g, int& m, double& ds, double& n)
         {
-            const VorCell& C = g.vcell[c];
-            j = C.begin;
-            sx = C.x;
-            sy = C.y;
-            sz = C.z;
-        }
-
-        // exit through the nearest bisector plane or domain wall (VoronoiMeshSnapshot.cpp:1119-1210)
-        __device__ __forceinline__ bool next_voronoi(const GridView& g, int& m, double& ds, double& n)
-        {
-            for (int tries = 0; tries < kMaxNoExit; ++tries)
+            if (__builtin_expect(j == kVorNone, 0))
             {
-                const double px0 = sx, py0 = sy, pz0 = sz;
-                double sq = DBL_MAX;
-                int mq = -99;
-                double nsx = 0., nsy = 0., nsz = 0.;  // the winning entry's site and run
-                int nrun = -1;
-                // exit distance through one neighbour entry; the smallest positive one wins,
-                // strict '<' (the first of equal distances wins)
-                auto consider = [&](const VorNb E) {
-                    const int mi = E.id;
-                    double si = 0;
-                    if (mi >= 0)
-                    {
-                        double nx = E.x - px0, ny = E.y - py0, nz = E.z - pz0;
-                        double ndotk = nx * kx + ny * ky + nz * kz;
-                        if (ndotk > 0)
-                        {
-                            double qx = 0.5 * (E.x + px0), qy = 0.5 * (E.y + py0), qz = 0.5 * (E.z + pz0);
-                            si = (nx * (qx - rx) + ny * (qy - ry) + nz * (qz - rz)) / ndotk;
-                        }
-                    }
-                    else
-                    {
-                        // walls -1..-6: (box face - r_axis) / k_axis
-                        const int w = -1 - mi;
-                        const int ax = w >> 1;
-                        const double face = g.box[(w & 1) ? 3 + ax : ax];
-                        // register copies, selected by axis: a select among the members
-                        // themselves becomes an indexed load from a scratch copy of them, which
-                        // is then stored at every crossing (1412 -> 1085 ms per 2^22-packet launch
-                        // on the 1e6-site clumpy medium without it)
-                        double tx = rx, ty = ry, tz = rz, ux = kx, uy = ky, uz = kz;
-                        asm volatile("" : "+v"(tx), "+v"(ty), "+v"(tz), "+v"(ux), "+v"(uy), "+v"(uz));
-                        const double ra = ax == 0 ? tx : (ax == 1 ? ty : tz);
-                        const double ka = ax == 0 ? ux : (ax == 1 ? uy : uz);
-                        if (w < 6) si = (face - ra) / ka;
-                    }
-                    if (si > 0 && si < sq)
-                    {
-                        sq = si;
-                        mq = mi;
-                        nsx = E.x;
-                        nsy = E.y;
-                        nsz = E.z;
-                        nrun = E.run;
-                    }
-                };
-                // the run: its header and first three entries in one group, then the entries
-                // four at a time so that their loads are in flight together
-                const int hb = j;
-                const VorNb H = g.vnb[hb], E1 = g.vnb[hb + 1], E2 = g.vnb[hb + 2], E3 = g.vnb[hb + 3];
-                const double dens = H.x;
-                const int e = hb + 1 + H.run;
-                if (hb + 1 < e) consider(E1);
-                if (hb + 2 < e) consider(E2);
-                if (hb + 3 < e) consider(E3);
-                int q = hb + 4;
-                for (; q + 4 <= e; q += 4)
-                {
-                    const VorNb F0 = g.vnb[q], F1 = g.vnb[q + 1], F2 = g.vnb[q + 2], F3 = g.vnb[q + 3];
-                    consider(F0);
-                    consider(F1);
-                    consider(F2);
-                    consider(F3);
-                }
-                for (; q < e; ++q) consider(g.vnb[q]);
-                if (mq == -99)
-                {
-                    rx += kx * g.eps;
-                    ry += ky * g.eps;
-                    rz += kz * g.eps;
-                    i = vor_cell_index(g, rx, ry, rz);
-                    if (i < 0)
-                    {
-                        state = kOutside;
-                        return false;
-                    }
-                    vor_enter(g, i);
-                    continue;
-                }
-                const double step = sq + g.eps;
+                state = kOutside;
+                return -1;
+            }
+            const int sub = L > 1 ? static_cast<int>(threadIdx.x) & (L - 1) : 0;
+            VorRun<L> R;
+            R.load(g, max(j, 0), sub);
+            const bool hinted = i == kVorHinted;
+            int out = 0;
+            if (i >= 0)
+            {
+                const double d = j >= 0 ? vor_bisector(sx, sy, sz, R.a.x, R.a.y, R.b.x, rx, ry, rz, kx, ky, kz)
+                                        : vor_wall(g.box, j, rx, ry, rz, kx, ky, kz);
+                const double step = d + g.eps;
                 rx += kx * step;
                 ry += ky * step;
                 rz += kz * step;
-                m = i;
-                ds = sq;
-                n = dens;
-                i = mq;
-                j = nrun;
-                sx = nsx;
-                sy = nsy;
-                sz = nsz;
-                if (mq < 0) state = kOutside;
-                return true;
+                m = cell;
+                ds = d;
+                n = bn;
+                out = 1;
+                k = 0;
+                if (j < 0)
+                {
+                    state = kOutside;
+                    return 2;
+                }
             }
-            state = kOutside;
-            return false;
+            const int run = j;
+            if (!hinted) i = run;
+            sx = R.a.x;
+            sy = R.a.y;
+            sz = R.b.x;
+            bn = R.b.y;
+            cell = R.cell();
+            VorSearch S;
+            S.wx = static_cast<float>((rx - sx) * g.vscale);
+            S.wy = static_cast<float>((ry - sy) * g.vscale);
+            S.wz = static_cast<float>((rz - sz) * g.vscale);
+            S.fx = static_cast<float>(kx);
+            S.fy = static_cast<float>(ky);
+            S.fz = static_cast<float>(kz);
+            const float kk = fabsf(S.fx) + fabsf(S.fy) + fabsf(S.fz);
+            S.en2 = 2.f * kVorEps * fmaf(S.wx, S.wx, fmaf(S.wy, S.wy, fmaf(S.wz, S.wz, R.c.z)));
+            S.ed2 = 2.f * kVorEps * kk * R.c.w;
+            S.ed4 = 2.f * S.ed2;
+            S.l1 = S.l2 = S.mn = INFINITY;
+            S.a1 = 0.f;
+            S.id = kVorNone;
+#pragma unroll
+            for (int u = 0; u < kVorAhead<L>; ++u) S.entry(R.f[u], (u + 1) * L <= kVorPad || u * L + sub < R.count());
+            for (int q = L * kVorAhead<L>; q < R.count(); q += L * kVorAhead<L>)
+            {
+                R.load_entries(g.vnb + run + 3 + q + sub);
+#pragma unroll
+                for (int u = 0; u < kVorAhead<L>; ++u) S.entry(R.f[u], q + u * L + sub < R.count());
+            }
+            if constexpr (L == 4)
+            {
+                S.template merge<0xB1>();  // quad_perm 1 0 3 2
+                S.template merge<0x4E>();  // quad_perm 2 3 0 1
+            }
+            // the hint holds where the position is clearly nearer to the site than to every
+            // neighbour's (half the difference of the squared distances is the numerator): inside
+            // the domain, the cell is the set of points nearer to its site than to the sites
+            // across its faces, so that site is then the nearest of all
+            const bool there = !hinted || S.mn > S.en2;
+            // one neighbour is nearer than all the others can be
+            const bool one = S.l1 > 0.f && 1.00001f * (2.f * S.a1 - S.l1) < S.l2 && kk > 1e-12f && kk < 1e12f;
+            j = kVorAsk;
+            if (there)
+            {
+                i = run;
+                if (one) j = S.id;
+            }
+            return out;
+        }
+
+        // Whether the step could not decide the exit, or the cell, in FP32: resolve() then does,
+        // before the next step.  Apart from the step, so that no call lies in the loop of the
+        // crossings (the registers saved around one were half of that loop's time).
+        __device__ __forceinline__ bool asks() const { return GT == kVoronoi && j == kVorAsk; }
+        // no path: nothing to resolve
+        __device__ __forceinline__ void idle()
+        {
+            if constexpr (GT == kVoronoi) j = kVorNone;
+        }
+        __device__ __forceinline__ void resolve(const GridView& g)
+        {
+            if (i >= 0)
+            {
+                j = vor_exit_exact(g.vnb, g.box[0], g.box[1], g.box[2], g.box[3], g.box[4], g.box[5], i, rx, ry, rz, kx, ky,
+                                   kz);
+                if (j != kVorNone) return;
+                rx += kx * g.eps;
+                ry += ky * g.eps;
+                rz += kz * g.eps;
+                if (++k >= kMaxNoExit) return;
+            }
+            i = kVorEnter;
+            j = vor_find(g, rx, ry, rz);
+            if (j < 0) j = kVorNone;
         }
 
         // Tetra::findEnteringFace: the first of the six edges with a nonzero Pluecker product

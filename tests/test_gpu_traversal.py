@@ -1,0 +1,171 @@
+"""The path generators where their short cuts do not apply, on the GPU and bit for bit against the
+oracle: Voronoi cells with ties, close and many neighbours, with one and with four lanes per path;
+octrees with fine neighbours, split planes hit exactly, and more planes than the LDS holds; Cartesian
+grids beyond the LDS and beyond the packed start hint.  Start hints: the counters and images of
+packets from sources on and off the cells' faces."""
+
+import numpy as np
+import pytest
+
+import oracle as O
+from helpers import frame60, load_pkg
+
+pytestmark = pytest.mark.gpu
+
+VOR_KEYS = ("sites", "nb_begin", "nb_count", "nb_index", "block_n", "block_begin", "block_count", "block_index", "box")
+
+
+@pytest.fixture(scope="module")
+def eng():
+    e = load_pkg().Engine(0)
+    yield e
+    e.close()
+
+
+def _rays(box, on, seed, n=2000):
+    """Random rays, axis-parallel and diagonal ones, from inside, outside and the points `on`."""
+    rng = np.random.default_rng(seed)
+    lo, hi = box[:3], box[3:]
+    r = lo + (hi - lo) * (rng.random((n, 3)) * 1.2 - 0.1)
+    r[::4] = on[rng.integers(0, len(on), len(r[::4]))]
+    k = rng.normal(size=(n, 3))
+    k[1::5] = np.eye(3)[rng.integers(0, 3, len(k[1::5]))] * rng.choice([-1.0, 1.0], (len(k[1::5]), 1))
+    k[2::5] = rng.choice([-1.0, 1.0], (len(k[2::5]), 3))
+    return np.hstack([r, k / np.linalg.norm(k, axis=1, keepdims=True)])
+
+
+def _compare(eng, grid, rays, repeat):
+    off, m, ds = eng.trace_paths(np.tile(rays, (repeat, 1)), cap=None if repeat == 1 else repeat * 40 * len(rays))
+    ooff, om, ods = O.trace(grid, rays)
+    cnt = np.diff(ooff)
+    np.testing.assert_array_equal(np.diff(off), np.tile(cnt, repeat))
+    np.testing.assert_array_equal(m, np.tile(om, repeat))
+    np.testing.assert_array_equal(ds, np.tile(ods, repeat))
+
+
+def _vor_points(name):
+    rng = np.random.default_rng(4)
+    if name == "lattice":  # every vertex is shared by eight cells, and rays run along faces
+        a = (np.arange(6) + 0.5) / 6
+        return np.stack(np.meshgrid(a, a, a, indexing="ij"), -1).reshape(-1, 3)
+    if name == "close":  # pairs of sites nearer than the FP32 bounds resolve, and a dense clump
+        p = rng.random((150, 3))
+        return np.clip(np.vstack([p, p[:40] + 3e-10, 0.5 + 1e-6 * rng.random((60, 3))]), 1e-9, 1 - 1e-9)
+    if name == "hub":  # one cell with hundreds of neighbours
+        k = rng.normal(size=(400, 3))
+        return np.vstack([[[0.5, 0.5, 0.5]], 0.5 + 0.4 * k / np.linalg.norm(k, axis=1, keepdims=True)])
+    return rng.random((dict(one=1, two=2, few=5).get(name, 700), 3))
+
+
+@pytest.mark.parametrize("repeat", [1, 70], ids=["four_lanes", "one_lane"])
+@pytest.mark.parametrize("name,shift", [("lattice", 0.0), ("close", 0.0), ("hub", 0.0), ("one", 0.0), ("two", 0.0),
+                                        ("few", 0.0), ("far", 1e7)])
+def test_voronoi_paths_bit_exact(eng, name, shift, repeat):
+    pkg = load_pkg()
+    box = np.array([0.0, 0.0, 0.0, 1.0, 1.0, 1.0]) + shift
+    b = pkg.Voronoi.build(_vor_points(name) + shift, box)
+    t = b.export()
+    b.upload(eng)
+    b.close()
+    print("case voronoi", name, repeat, flush=True)
+    s = np.asarray(t["sites"])
+    on = np.vstack([s, 0.5 * (s + np.roll(s, 1, axis=0))])
+    _compare(eng, O.Grid("voronoi", **{k: t[k] for k in VOR_KEYS}), _rays(box, on, 1), repeat)
+
+
+def _octree_flags(box, levels, refine):
+    """Level-order division flags: nodes that `refine` (lo, hi, level) selects, up to `levels`."""
+    flags, row = [], [(tuple(box[:3]), tuple(box[3:]))]
+    for level in range(levels + 1):
+        nxt = []
+        for lo, hi in row:
+            d = level < levels and refine(lo, hi, level)
+            flags.append(1 if d else 0)
+            if d:
+                c = [0.5 * (a + b) for a, b in zip(lo, hi)]
+                for q in range(8):
+                    nxt.append((tuple(c[a] if q >> a & 1 else lo[a] for a in range(3)),
+                                tuple(hi[a] if q >> a & 1 else c[a] for a in range(3))))
+        row = nxt
+    return np.array(flags, np.uint8)
+
+
+@pytest.mark.parametrize("name", ["root", "random", "lines"])
+def test_octree_paths_bit_exact(eng, name):
+    pkg = load_pkg()
+    box = np.array([-1.0, -1.0, -1.0, 1.0, 1.0, 1.0])
+    if name == "root":
+        flags = _octree_flags(box, 0, None)
+    elif name == "random":
+        rng = np.random.default_rng(8)
+        flags = _octree_flags(box, 6, lambda lo, hi, level: level < 2 or rng.random() < 0.25)
+    else:  # fine along lines parallel to the x and to the y axis: more planes than the LDS table holds
+        p = (0.3, 0.7, 0.123, 0.234)
+        flags = _octree_flags(box, 12, lambda lo, hi, level: (lo[1] <= p[0] <= hi[1] and lo[2] <= p[1] <= hi[2])
+                              or (lo[0] <= p[2] <= hi[0] and lo[2] <= p[3] <= hi[2]))
+    tree = pkg.Octree.from_flags(box, flags)
+    t = tree.export()
+    tree.upload(eng)
+    tree.close()
+    print("case octree", name, len(flags), flush=True)
+    corners = np.asarray(t["bounds"])[:, 3:]
+    rays = _rays(box, corners[np.random.default_rng(2).integers(0, len(corners), 500)], 3)
+    _compare(eng, O.Grid("octree", **{k: t[k] for k in ("bounds", "child_first", "cell_index", "nb_off", "nb_id")}), rays, 1)
+
+
+@pytest.mark.parametrize("n", [(1, 1, 1), (7, 5, 3), (1030, 3, 2), (2, 3300, 2)])
+def test_cartesian_paths_and_packets(eng, n):
+    rng = np.random.default_rng(5)
+    b = [np.concatenate([[-1.0], np.sort(rng.uniform(-1, 1, q - 1)), [1.0]]) for q in n]
+    eng.grid_cartesian(*b)
+    box = np.array([-1.0] * 3 + [1.0] * 3)
+    g = O.Grid("cartesian", xb=b[0], yb=b[1], zb=b[2])
+    print("case cartesian", n, flush=True)
+    _compare(eng, g, _rays(box, np.stack([rng.choice(q, 200) for q in b], 1), 6, 400), 1)
+    _packets(eng, g, np.ones(int(np.prod(n))) * 1e-3, (b[0][0 if n[0] == 1 else 1], 0.1, 0.2))
+
+
+def _packets(eng, grid, dens, src):
+    """Few packets (the lanes-per-wave rule) from a source on a face: the oracle's counts and image."""
+    eng.medium(dens)
+    eng.dust([0.55e-6], [500.0], [300.0], [0.6])
+    fr = frame60(npix=20)
+    fr["fovx"] = fr["fovy"] = 4.0
+    eng.frame_remove_all()
+    eng.frame_add(fr["inclination"], fr["azimuth"], fr["roll"], fr["nx"], fr["ny"], fr["fovx"], fr["fovy"])
+    for npk, mode in ((1, 1), (700, 1), (700, 0)):  # persistent, persistent, pipeline
+        eng.source_point(src, [1.0 / npk])
+        eng.options(0.5, 1e4, 0, 0, 13)
+        eng.tune_pipeline(mode, 1 << 14, 0, 8)
+        eng.frame_clear()
+        eng.run_packets(0, npk)
+        img, cnt = eng.frame_read(0)[0], eng.counters()
+        ofr, ocnt = O.simulate(grid, dens, [0.55e-6], [500.0], [300.0], [0.6], [1.0 / npk], [fr], 0, npk, threads=4, seed=13,
+                               src=src)
+        # the transcendental functions differ in the last bits: a packet near a threshold may take
+        # another turn, one in a thousand at most
+        assert cnt[0] == ocnt[0] == npk
+        assert abs(int(cnt[2]) - int(ocnt[2])) <= max(1e-3 * ocnt[2], 1)
+        assert abs(img.sum() / ofr[0][0].sum() - 1) < 1e-6
+
+
+@pytest.mark.parametrize("kind", ["octree", "voronoi", "tetra"])
+def test_start_hints(eng, kind):
+    """Sources on a site, a vertex or a face, and moved from one cell to another without a new grid."""
+    pkg = load_pkg()
+    box = np.array([-1.0, -1.0, -1.0, 1.0, 1.0, 1.0])
+    rng = np.random.default_rng(9)
+    if kind == "octree":
+        b = pkg.Octree.from_flags(box, _octree_flags(box, 4, lambda lo, hi, level: level < 2 or rng.random() < 0.4))
+        keys, srcs = ("bounds", "child_first", "cell_index", "nb_off", "nb_id"), [(0.0, 0.0, 0.0), (0.5, 0.25, -0.1)]
+    else:
+        pts = rng.uniform(-1, 1, (900, 3))
+        b = pkg.Voronoi.build(pts, box) if kind == "voronoi" else pkg.Tetra.build(pts, box)
+        keys, srcs = VOR_KEYS if kind == "voronoi" else None, [(0.0, 0.0, 0.0), tuple(pts[17]), tuple(0.5 * (pts[3] + pts[4]))]
+    t = b.export()
+    b.upload(eng)
+    b.close()
+    g = O.Grid(kind, **({k: t[k] for k in keys} if keys else t))
+    for src in srcs:
+        print("case start hint", kind, src, flush=True)
+        _packets(eng, g, np.full(eng.num_cells(), 1e-3), src)
