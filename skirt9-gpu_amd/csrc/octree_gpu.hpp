@@ -65,16 +65,11 @@ namespace skg
             // DensityTreePolicy::needsSubdivide, maxDustFraction criterion: the mean normalised
             // density over `samples` uniform points of the box (stream id = node id) x volume
             const double* b = B + 6 * (lbeg + i);
-            Philox rng;
-            rng.init(seed, static_cast<uint64_t>(lbeg + i), kTagTree);
-            double sum = 0.;
-            for (int q = 0; q < samples; ++q)
-            {
-                const double x = b[0] + rng.uniform() * (b[3] - b[0]);
-                const double y = b[1] + rng.uniform() * (b[4] - b[1]);
-                const double z = b[2] + rng.uniform() * (b[5] - b[2]);
-                sum += md.geom(x, y, z);
-            }
+            const double x0 = b[0], y0 = b[1], z0 = b[2], dx = b[3] - x0, dy = b[4] - y0, dz = b[5] - z0;
+            const double sum = sample_sum(samples, 0, 1, seed, static_cast<uint64_t>(lbeg + i), kTagTree,
+                                          [&](double u, double v, double w) {
+                                              return md.geom_device(x0 + u * dx, y0 + v * dy, z0 + w * dz);
+                                          });
             const double rho = sum / samples;
             const double vol = (b[3] - b[0]) * (b[4] - b[1]) * (b[5] - b[2]);
             f = rho * vol > frac ? 1 : 0;

@@ -73,9 +73,15 @@ namespace skg
         {
             uint32_t b = draw >> 1;
             if (b != block) gen(b);
-            uint32_t hi = (draw & 1) ? c[2] : c[0];
-            uint32_t lo = (draw & 1) ? c[3] : c[1];
             ++draw;
+            return (draw & 1) ? first() : second();
+        }
+
+        // the two deviates of the current block
+        __host__ __device__ __forceinline__ double first() const { return deviate(c[0], c[1]); }
+        __host__ __device__ __forceinline__ double second() const { return deviate(c[2], c[3]); }
+        static __host__ __device__ __forceinline__ double deviate(uint32_t hi, uint32_t lo)
+        {
             uint64_t a = (static_cast<uint64_t>(hi) << 20) ^ (lo >> 12);
             return (static_cast<double>(a) + 0.5) * (1.0 / 4503599627370496.0);
         }

@@ -612,7 +612,9 @@ namespace skg
                             hint = p.srcHint;
                         else if constexpr (GT == kVoronoi)
                             hint = p.grid.vcell[hint].run;
-                        else if constexpr (GT != kTetra)
+                        else if constexpr (GT == kOctree)
+                            hint = p.grid.leaf[hint];
+                        else if constexpr (GT == kCartesian)
                             hint = -1;
                         gen.start(P.rx[slot], P.ry[slot], P.rz[slot], dx, dy, dz, hint);
                         gen.idle();

@@ -140,6 +140,7 @@ namespace skg
         int nx, ny, nz;
         const double* dens;  // Cartesian: number density per cell
         const OctNode* node;
+        const int32_t* leaf;  // cell -> node
         const double* planes;   // octree: the distinct coordinates of the tree's bounds; Cartesian: the
                                 // borders of the three axes, one after the other
         int nplanes;
