@@ -18,6 +18,8 @@
 #include <memory>
 #include <mutex>
 #include <string>
+#include <system_error>
+#include <thread>
 #include <unordered_map>
 #include <vector>
 
@@ -203,10 +205,16 @@ namespace skg
     }
 
     // and into the tetrahedra's records
-    __global__ void fill_tet_density(TetCell* rec, const double* dens, int64_t n)
+    __global__ void fill_tet_density(TetCell* rec, TetFace* face, const double* dens, int64_t n)
     {
         int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
-        if (i < n) rec[i].dens = dens[i];
+        if (i >= n) return;
+        rec[i].dens = dens[i];
+        for (int f = 0; f < 4; ++f)
+        {
+            const int nb = face[4 * i + f].cell;
+            face[4 * i + f].dens = nb >= 0 ? dens[nb] : 0.;
+        }
     }
 
     // and into the heads of the Voronoi cells' runs
@@ -640,7 +648,8 @@ namespace
             hipLaunchKernelGGL(fill_vor_density, grid, block, 0, e->stream, const_cast<VorNb*>(e->grid.vnb), e->grid.vcell,
                                e->dens, n);
         else
-            hipLaunchKernelGGL(fill_tet_density, grid, block, 0, e->stream, const_cast<TetCell*>(e->grid.tcell), e->dens, n);
+            hipLaunchKernelGGL(fill_tet_density, grid, block, 0, e->stream, const_cast<TetCell*>(e->grid.tcell),
+                               const_cast<TetFace*>(e->grid.tface), e->dens, n);
         HIPCHK(e, hipGetLastError());
         HIPCHK(e, hipStreamSynchronize(e->stream));
         return SKG_OK;
@@ -1263,6 +1272,33 @@ int skg_grid_voronoi(skg_engine* e, int64_t nsites, const double* sites, const i
     return refreshLeafDensity(e);
 }
 
+namespace
+{
+    // the link word of a TetFace: from the tetra with vertex ids a through its face f into the one with
+    // vertex ids b, whose face nf it is
+    uint32_t tetLink(const int32_t* a, int f, const int32_t* b, int nf)
+    {
+        uint32_t link = static_cast<uint32_t>(nf) << 16;
+        int d[3];
+        clockwise_vertices(nf, d[0], d[1], d[2]);
+        for (int e = 0; e < 4; ++e)
+        {
+            if (e == f) continue;
+            int c[3];
+            clockwise_vertices(e, c[0], c[1], c[2]);
+            const int q = static_cast<int>(std::find(c, c + 3, f) - c);
+            const int32_t list[3] = {a[e], a[c[(q + 1) % 3]], a[c[(q + 2) % 3]]};
+            int p[3];
+            for (int u = 0; u < 3; ++u) p[u] = static_cast<int>(std::find(list, list + 3, b[d[u]]) - list);
+            if (p[0] + p[1] + p[2] != 3 || p[0] == p[1] || p[0] == 3 || p[1] == 3)
+                link |= 1u << 18;
+            else
+                link |= static_cast<uint32_t>(p[0] | p[1] << 2) << (4 * e);
+        }
+        return link;
+    }
+}
+
 int skg_grid_tetra(skg_engine* e, int64_t nverts, const double* verts, int64_t ntets, const int32_t* tet_verts,
                    const int32_t* face_nb, const double* face_normal, const double* box)
 {
@@ -1270,34 +1306,58 @@ int skg_grid_tetra(skg_engine* e, int64_t nverts, const double* verts, int64_t n
         return fail(e, SKG_ERR_ARGUMENT, "skg_grid_tetra: bad arguments");
     if (!(box[0] < box[3] && box[1] < box[4] && box[2] < box[5])) return fail(e, SKG_ERR_ARGUMENT, "skg_grid_tetra: empty box");
     std::vector<TetCell> T(ntets);
-    for (int64_t m = 0; m < ntets; ++m)
-    {
-        TetCell& c = T[m];
-        std::memset(&c, 0, sizeof(c));
-        for (int t = 0; t < 4; ++t)
+    std::vector<TetFace> F(4 * static_cast<size_t>(ntets));
+    // the records of the cells [first, last); an error message where the tables are wrong
+    const auto records = [&](int64_t first, int64_t last) -> const char* {
+        for (int64_t m = first; m < last; ++m)
         {
-            int32_t vi = tet_verts[4 * m + t];
-            if (vi < 0 || vi >= nverts) return fail(e, SKG_ERR_ARGUMENT, "skg_grid_tetra: vertex id out of range");
-            for (int a = 0; a < 3; ++a)
+            TetCell& c = T[m];
+            for (int t = 0; t < 4; ++t)
             {
-                c.v[t][a] = verts[3 * static_cast<int64_t>(vi) + a];
-                c.n[t][a] = face_normal[12 * m + 3 * t + a];
+                const int32_t vi = tet_verts[4 * m + t];
+                if (vi < 0 || vi >= nverts) return "skg_grid_tetra: vertex id out of range";
+                TetFace& face = F[4 * static_cast<size_t>(m) + t];
+                for (int a = 0; a < 3; ++a)
+                {
+                    c.v[t][a] = verts[3 * static_cast<int64_t>(vi) + a];
+                    c.n[t][a] = face.n[a] = face_normal[12 * m + 3 * t + a];
+                }
+                const int32_t nt = face_nb[4 * m + t];
+                if (nt < -1 || nt >= ntets) return "skg_grid_tetra: neighbour id out of range";
+                face.cell = nt;
+                if (nt < 0) continue;
+                // the neighbour's face that points back (TetraMeshSpatialGrid.cpp:508-520)
+                const int32_t* back = face_nb + 4 * static_cast<int64_t>(nt);
+                const int nface = static_cast<int>(std::find(back, back + 4, static_cast<int32_t>(m)) - back);
+                if (nface == 4) return "skg_grid_tetra: neighbour relation not mutual";
+                face.link = tetLink(tet_verts + 4 * m, t, tet_verts + 4 * static_cast<int64_t>(nt), nface);
+                const int32_t apex = tet_verts[4 * static_cast<int64_t>(nt) + nface];
+                if (apex < 0 || apex >= nverts) return "skg_grid_tetra: vertex id out of range";
+                std::copy(verts + 3 * static_cast<int64_t>(apex), verts + 3 * static_cast<int64_t>(apex) + 3, face.v);
             }
-            int32_t nt = face_nb[4 * m + t];
-            if (nt < -1 || nt >= ntets) return fail(e, SKG_ERR_ARGUMENT, "skg_grid_tetra: neighbour id out of range");
-            c.nb[t] = nt;
-            c.nface[t] = -1;
-            // the neighbour's face that points back (TetraMeshSpatialGrid.cpp:508-520)
-            if (nt >= 0)
-                for (int fn = 0; fn < 4; ++fn)
-                    if (face_nb[4 * static_cast<int64_t>(nt) + fn] == m)
-                    {
-                        c.nface[t] = static_cast<int8_t>(fn);
-                        break;
-                    }
-            if (nt >= 0 && c.nface[t] < 0) return fail(e, SKG_ERR_ARGUMENT, "skg_grid_tetra: neighbour relation not mutual");
+        }
+        return nullptr;
+    };
+    // (a thread per 16 384 cells, eight at most)
+    const int nthr = static_cast<int>(std::clamp<int64_t>(ntets >> 14, 1, 8));
+    std::vector<const char*> bad(nthr, nullptr);
+    const auto share = [&](int q) { bad[q] = records(ntets * q / nthr, ntets * (q + 1) / nthr); };
+    std::vector<std::thread> team;
+    for (int q = 1; q < nthr; ++q)
+    {
+        try
+        {
+            team.emplace_back(share, q);
+        }
+        catch (const std::system_error&)
+        {
+            share(q);  // no more threads
         }
     }
+    share(0);
+    for (auto& th : team) th.join();
+    for (const char* b : bad)
+        if (b) return fail(e, SKG_ERR_ARGUMENT, b);
     int tbn = 0;
     std::vector<double> borders;
     std::vector<int32_t> off, ids;
@@ -1308,7 +1368,8 @@ int skg_grid_tetra(skg_engine* e, int64_t nverts, const double* verts, int64_t n
     GridView g{};
     int st;
     const double* dB = nullptr;
-    if ((st = gridUpload(e, T.data(), T.size(), &g.tcell)) || (st = gridUpload(e, borders.data(), borders.size(), &dB))
+    if ((st = gridUpload(e, T.data(), T.size(), &g.tcell)) || (st = gridUpload(e, F.data(), F.size(), &g.tface))
+        || (st = gridUpload(e, borders.data(), borders.size(), &dB))
         || (st = gridUpload(e, off.data(), off.size(), &g.tbl_off)) || (st = gridUpload(e, ids.data(), ids.size(), &g.tbl_id)))
         return st;
     g.tbn = tbn;

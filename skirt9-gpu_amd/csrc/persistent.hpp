@@ -880,7 +880,7 @@ namespace skg
     //   octree with the radiation field, 2e5        7.8 / 11.6 / 13.2 (bound by its atomics, whose
     //   Cartesian with the field, 7e5              targets collide more with more waves)
     //   Voronoi, 400 000 sites, 2^18 packets         - / 48.0 / 52.8
-    //   tetra, before the events became calls      6720 / 5800 / 5270
+    //   tetra, 150 000 vertices, 64 instances, 2^20   - / 61.2 / 57.8
     // The guided variant's network call holds whole layers' weights in registers, and its four-wave build does not compile for the mesh grids.
     template<int GT, int V> constexpr int lifecycle_waves()
     {

@@ -76,20 +76,35 @@ namespace skg
     constexpr int kVorNone = -99;  // no exit
     constexpr int kVorAsk = -98;   // not decided yet (Gen::resolve)
 
-    // Tetrahedron record (256 bytes, two cache lines, indexed by cell): vertex coordinates,
-    // density and face links in the first line, the outward unit face normals in the second.
+    // Tetrahedron record (indexed by cell, for the search of a position's cell and the start of a
+    // path): vertices and outward face normals (TetraMeshSpatialGrid), density
     struct alignas(128) TetCell
     {
-        double v[4][3];     // vertices in the reference's per-tetra order
-        double dens;        // number density
-        int32_t nb[4];      // neighbour tetra across face f (opposite vertex f), -1 on the hull
-        int8_t nface[4];    // the neighbour's index of the shared face
-        int32_t pad0;
-        double n[4][3];     // outward unit normal of face f
-        double pad1[4];
+        double v[4][3];
+        double dens;
+        double pad[3];
+        double n[4][3];
+        double pad2[4];
     };
     static_assert(sizeof(TetCell) == 256, "tetra record must be 256 bytes");
     static_assert(offsetof(TetCell, n) == 128, "tetra normals start the second line");
+
+    // One 64-byte record per face of a cell, at 4 * cell + face (the face opposite that vertex): its
+    // normal, the cell behind it (-1: none), that cell's vertex opposite the face and density.  link:
+    // bits 16-17 the face's number in that cell; bits 4e to 4e + 3, for a path that entered this cell
+    // by face e, the place of the next cell's first and second vertex clockwise around the face in the
+    // list (this cell's vertex e, then the two others of the face in this cell's clockwise order from
+    // the one left out); bit 18 where the cells' vertices do not match and have to be read instead.
+    struct alignas(64) TetFace
+    {
+        double n[3];
+        int32_t cell;
+        uint32_t link;
+        double v[3];
+        double dens;
+    };
+    static_assert(sizeof(TetFace) == 64, "tetra face record must be 64 bytes");
+
 
     // Consecutive "no exit found" steps after which a Voronoi or tetra path is ended.  The
     // reference steps by eps without limit; a path needs that many only when it has left the
@@ -158,6 +173,7 @@ namespace skg
         // tetra: records and a block search grid (tbn^3 blocks, borders per axis, CSR of tetra
         // ids in increasing order)
         const TetCell* tcell;
+        const TetFace* tface;
         int tbn;
         const double* tbx;
         const double* tby;
@@ -292,7 +308,7 @@ namespace skg
     }
 
     // TetraMeshSpatialGrid.cpp:44-50
-    __device__ __forceinline__ void clockwise_vertices(int face, int& c0, int& c1, int& c2)
+    __host__ __device__ __forceinline__ void clockwise_vertices(int face, int& c0, int& c1, int& c2)
     {
         c0 = (face + 3) & 3;
         c1 = (face + 2) & 3;
@@ -304,6 +320,32 @@ namespace skg
             c2 = t;
         }
     }
+
+    struct TetVert
+    {
+        double x, y, z;
+        __device__ __forceinline__ void load(const double* v)
+        {
+            x = v[0];
+            y = v[1];
+            z = v[2];
+        }
+    };
+    // a face record in registers
+    struct TetFaceRec
+    {
+        double2 a, b, c, d;
+        __device__ __forceinline__ void load(const TetFace* f)
+        {
+            const double2* p = reinterpret_cast<const double2*>(f);
+            a = p[0];
+            b = p[1];
+            c = p[2];
+            d = p[3];
+        }
+        __device__ __forceinline__ int cell() const { return __double2loint(b.y); }
+        __device__ __forceinline__ uint32_t link() const { return static_cast<uint32_t>(__double2hiint(b.y)); }
+    };
 
     enum GenState : int
     {
@@ -318,6 +360,11 @@ namespace skg
     {
         const T yz = b ? y : z;
         return a ? x : yz;
+    }
+    __device__ __forceinline__ TetVert pick_vert(bool first, bool second, const TetVert& a, const TetVert& b, const TetVert& c)
+    {
+        return TetVert{pick3(first, second, a.x, b.x, c.x), pick3(first, second, a.y, b.y, c.y),
+                       pick3(first, second, a.z, b.z, c.z)};
     }
 
     // a / b for a correctly rounded reciprocal y = RN(1 / b): the product with y, one Newton step
@@ -604,11 +651,13 @@ namespace skg
         int i, j, k;  // Cartesian: entry of the border ahead on each axis in the planes table; octree: i = current leaf's node; Voronoi: i = the
                       // current cell's run, j = the run or wall behind its exit, k = the
                       // steps without exit; tetra: i = current
-                      // cell, j = entering face, -1 if unknown
+                      // cell, j = entering face, -1 at the end, k = the steps without exit
         double sx, sy, sz;      // Voronoi: the current cell's site
         double ikx, iky, ikz;   // Cartesian, octree: reciprocals of the direction
         double b0, b1, b2;      // Cartesian, octree: the current cell's wall ahead on each axis
-        double bn;              // Cartesian, octree, Voronoi: its density
+        double bn;              // the current cell's density
+        TetVert V, C0, C1, C2;  // tetra: the vertex opposite the entering face, that face's clockwise
+        bool ask;               // tetra: something to resolve()
         int f0, f1, f2;         // octree: the node across each of those walls
         int cell;               // Cartesian, octree, Voronoi: the current cell's index
         uint32_t pend;  // octree: a node to descend into next and the crossed wall (node << 3 | wall),
@@ -880,7 +929,9 @@ namespace skg
                 {
                     i = hint >= 0 && tet_inside_strict(g.tcell[hint], rx, ry, rz) ? hint : tet_cell_index(g, rx, ry, rz);
                     hint = i;
-                    j = -1;
+                    k = 0;
+                    ask = false;
+                    if (i >= 0) tet_enter(g, -1);
                 }
                 if (hint < 0)
                 {
@@ -900,15 +951,10 @@ namespace skg
                 return cross_octree(g, m, ds, n);
             else if constexpr (GT == kVoronoi)
                 return cross_voronoi(g, m, ds, n);
+            else if constexpr (GT == kTetra)
+                return cross_tetra(g, m, ds, n);
             else
-            {
-                bool more;
-                if constexpr (GT == kCartesian)
-                    more = next_cartesian(g, m, ds, n);
-                else
-                    more = next_tetra(g, m, ds, n);
-                return !more ? -1 : state == kOutside ? 2 : 1;
-            }
+                return !next_cartesian(g, m, ds, n) ? -1 : state == kOutside ? 2 : 1;
         }
 
         // One step of a path from its start on, as cross(); the first step begins the path and
@@ -1091,30 +1137,57 @@ namespace skg
             return out;
         }
 
-        // Whether the step could not decide the exit, or the cell, in FP32: resolve() then does,
-        // before the next step.  Apart from the step, so that no call lies in the loop of the
-        // crossings (the registers saved around one were half of that loop's time).
-        __device__ __forceinline__ bool asks() const { return GT == kVoronoi && j == kVorAsk; }
+        // Whether the step left something to resolve() before the next step: an exit, or a start cell,
+        // that the Voronoi search could not decide in FP32; a tetra position without an exit, or vertices to read.  Apart
+        // from the step, so that no call and no cell search lies in the loop of the crossings (the
+        // registers saved around a call were half of the Voronoi loop's time).
+        __device__ __forceinline__ bool asks() const
+        {
+            return GT == kVoronoi ? j == kVorAsk : GT == kTetra ? ask : false;
+        }
         // no path: nothing to resolve
         __device__ __forceinline__ void idle()
         {
             if constexpr (GT == kVoronoi) j = kVorNone;
+            if constexpr (GT == kTetra) ask = false;
         }
         __device__ __forceinline__ void resolve(const GridView& g)
         {
-            if (i >= 0)
+            if constexpr (GT == kVoronoi)
             {
-                j = vor_exit_exact(g.vnb, g.box[0], g.box[1], g.box[2], g.box[3], g.box[4], g.box[5], i, rx, ry, rz, kx, ky,
-                                   kz);
-                if (j != kVorNone) return;
-                rx += kx * g.eps;
-                ry += ky * g.eps;
-                rz += kz * g.eps;
-                if (++k >= kMaxNoExit) return;
+                if (i >= 0)
+                {
+                    j = vor_exit_exact(g.vnb, g.box[0], g.box[1], g.box[2], g.box[3], g.box[4], g.box[5], i, rx, ry, rz,
+                                       kx, ky, kz);
+                    if (j != kVorNone) return;
+                    if (!nudge(g)) return;
+                }
+                i = kVorEnter;
+                j = vor_find(g, rx, ry, rz);
+                if (j < 0) j = kVorNone;
             }
-            i = kVorEnter;
-            j = vor_find(g, rx, ry, rz);
-            if (j < 0) j = kVorNone;
+            else if constexpr (GT == kTetra)
+            {
+                ask = false;
+                if (k == kTetReload)
+                {
+                    k = 0;
+                    tet_enter(g, j);
+                    return;
+                }
+                j = -1;
+                if (!nudge(g)) return;
+                i = tet_cell_index(g, rx, ry, rz);
+                if (i >= 0) tet_enter(g, -1);
+            }
+        }
+        // a step of eps along the path; false after too many without an exit
+        __device__ __forceinline__ bool nudge(const GridView& g)
+        {
+            rx += kx * g.eps;
+            ry += ky * g.eps;
+            rz += kz * g.eps;
+            return ++k < kMaxNoExit;
         }
 
         // Tetra::findEnteringFace: the first of the six edges with a nonzero Pluecker product
@@ -1140,88 +1213,118 @@ namespace skg
             return -1;
         }
 
-        // Pluecker exit-face decision with the plane-intersection fallback
-        // (TetraMeshSpatialGrid.cpp:719-819); the final segment before the hull is not returned.
-        // Ends the path where the reference would not terminate: no entering face (all six
-        // products zero) or a non-finite position.
-        __device__ __forceinline__ bool next_tetra(const GridView& g, int& m, double& ds, double& n)
+        // Enters the cell i through its face ef (-1: the face the path entered by, -1 again if there is
+        // none): its vertices, relative to that face, and its density.
+        __device__ __forceinline__ void tet_enter(const GridView& g, int ef)
         {
-            for (int tries = 0; tries < kMaxNoExit; ++tries)
+            const TetCell& T = g.tcell[i];
+            j = ef < 0 ? entering_face(T) : ef;
+            bn = T.dens;
+            if (j < 0) return;
+            int c0, c1, c2;
+            clockwise_vertices(j, c0, c1, c2);
+            V.load(T.v[j]);
+            C0.load(T.v[c0]);
+            C1.load(T.v[c1]);
+            C2.load(T.v[c2]);
+        }
+
+        // One step of the tetra generator: Pluecker exit-face decision with the plane-intersection
+        // fallback (TetraMeshSpatialGrid.cpp:719-819); the final segment before the hull is not
+        // returned.  Returns as cross() does.  Ends the path where the reference would not terminate:
+        // no entering face (all six products zero) or a non-finite position.
+        //
+        // Bound by the vector memory path: the lanes' cells lie apart, and the eleven loads of a
+        // crossing kept the return path busy 92 % of the time.  The vertices therefore stay in
+        // registers, ordered as seen from the entering face; the next cell shares three of them, and
+        // the record of the face between the two holds the fourth, with all else the crossing needs:
+        // four loads of one 64-byte line.  150 000 vertices, 64 instances, 2^20 packets: 79 -> 58 ms.
+        static constexpr int kTetReload = -1;  // k where the next cell's vertices do not match
+        __device__ __forceinline__ int cross_tetra(const GridView& g, int& m, double& ds, double& n)
+        {
+            if (j < 0 || !(isfinite(rx) && isfinite(ry) && isfinite(rz)))
             {
-                if (!(isfinite(rx) && isfinite(ry) && isfinite(rz))) break;
-                const TetCell& T = g.tcell[i];
-                if (j < 0) j = entering_face(T);
-                if (j < 0) break;
-                const int ef = j;
-                const double vx = T.v[ef][0], vy = T.v[ef][1], vz = T.v[ef][2];
-                double wx = rx - vx, wy = ry - vy, wz = rz - vz;
-                double mx = ky * wz - kz * wy, my = kz * wx - kx * wz, mz = kx * wy - ky * wx;
-                int c0, c1, c2;
-                clockwise_vertices(ef, c0, c1, c2);
-                double prod0 = mx * (vx - T.v[c0][0]) + my * (vy - T.v[c0][1]) + mz * (vz - T.v[c0][2]);
-                int clock0 = prod0 < 0;
-                int ci = clock0 ? c1 : c2;
-                double prodi = mx * (vx - T.v[ci][0]) + my * (vy - T.v[ci][1]) + mz * (vz - T.v[ci][2]);
-                int cclocki = prodi >= 0;
-                int leaving = -1;
-                double dsl = DBL_MAX;
-                if (prod0 == 0. || prodi == 0.)
+                state = kOutside;
+                return -1;
+            }
+            int c0, c1, c2;
+            clockwise_vertices(j, c0, c1, c2);
+            const double wx = rx - V.x, wy = ry - V.y, wz = rz - V.z;
+            const double mx = ky * wz - kz * wy, my = kz * wx - kx * wz, mz = kx * wy - ky * wx;
+            const double prod0 = mx * (V.x - C0.x) + my * (V.y - C0.y) + mz * (V.z - C0.z);
+            const bool clock0 = prod0 < 0;
+            const double qx = clock0 ? C1.x : C2.x, qy = clock0 ? C1.y : C2.y, qz = clock0 ? C1.z : C2.z;
+            const double prodi = mx * (V.x - qx) + my * (V.y - qy) + mz * (V.z - qz);
+            const bool cclocki = prodi >= 0;
+            // dtable {{1,0},{0,2}} indexes the clockwise vertices; which of them lies opposite the exit
+            int q = clock0 ? (cclocki ? 2 : 0) : (cclocki ? 0 : 1);
+            if (__builtin_expect(prod0 == 0. || prodi == 0., 0))
+            {
+                q = -1;
+                double least = DBL_MAX;
+                for (int u = 0; u < 3; ++u)
                 {
-                    const int cv[3] = {c0, c1, c2};
-                    for (int q = 0; q < 3; ++q)
+                    const TetFace& F = g.tface[4 * static_cast<int64_t>(i) + pick3(u == 0, u == 1, c0, c1, c2)];
+                    const double ndotk = F.n[0] * kx + F.n[1] * ky + F.n[2] * kz;
+                    if (ndotk > 0)
                     {
-                        const int f = cv[q];
-                        double ndotk = T.n[f][0] * kx + T.n[f][1] * ky + T.n[f][2] * kz;
-                        if (ndotk > 0)
+                        const double d = (F.n[0] * (V.x - rx) + F.n[1] * (V.y - ry) + F.n[2] * (V.z - rz)) / ndotk;
+                        if (d < least)
                         {
-                            double dq = (T.n[f][0] * (vx - rx) + T.n[f][1] * (vy - ry) + T.n[f][2] * (vz - rz)) / ndotk;
-                            if (dq < dsl)
-                            {
-                                dsl = dq;
-                                leaving = f;
-                            }
+                            least = d;
+                            q = u;
                         }
                     }
                 }
-                else
+                if (q < 0)
                 {
-                    // dtable {{1,0},{0,2}} indexes the clockwise vertices
-                    leaving = clock0 ? (cclocki ? c2 : c0) : (cclocki ? c0 : c1);
-                    double ndotk = T.n[leaving][0] * kx + T.n[leaving][1] * ky + T.n[leaving][2] * kz;
-                    dsl = (T.n[leaving][0] * (vx - rx) + T.n[leaving][1] * (vy - ry) + T.n[leaving][2] * (vz - rz)) / ndotk;
+                    ask = true;
+                    return 0;
                 }
-                if (leaving == -1 || dsl < g.eps)
-                {
-                    rx += kx * g.eps;
-                    ry += ky * g.eps;
-                    rz += kz * g.eps;
-                    i = tet_cell_index(g, rx, ry, rz);
-                    if (i < 0)
-                    {
-                        state = kOutside;
-                        return false;
-                    }
-                    j = -1;
-                    continue;
-                }
-                rx += kx * dsl;
-                ry += ky * dsl;
-                rz += kz * dsl;
-                const int nxt = T.nb[leaving];
-                if (nxt < 0)
-                {
-                    state = kOutside;
-                    return false;
-                }
-                m = i;
-                ds = dsl;
-                n = T.dens;
-                j = T.nface[leaving];
-                i = nxt;
-                return true;
             }
-            state = kOutside;
-            return false;
+            const bool q0 = q == 0, q1 = q == 1;
+            const int leaving = pick3(q0, q1, c0, c1, c2);
+            TetFaceRec F;
+            F.load(g.tface + 4 * static_cast<int64_t>(i) + leaving);
+            const double ndotk = F.a.x * kx + F.a.y * ky + F.b.x * kz;
+            const double d = (F.a.x * (V.x - rx) + F.a.y * (V.y - ry) + F.b.x * (V.z - rz)) / ndotk;
+            if (__builtin_expect(d < g.eps, 0))
+            {
+                ask = true;
+                return 0;
+            }
+            rx += kx * d;
+            ry += ky * d;
+            rz += kz * d;
+            const int nxt = F.cell();
+            if (nxt < 0)
+            {
+                state = kOutside;
+                return -1;
+            }
+            m = i;
+            ds = d;
+            n = bn;
+            k = 0;
+            // the exit face's vertices, then in the next cell's order
+            const uint32_t link = F.link();
+            const uint32_t p = link >> (4 * j);
+            const TetVert X1 = pick_vert(q0, q1, C1, C2, C0), X2 = pick_vert(q0, q1, C2, C0, C1);
+            const int p0 = p & 3, p1 = (p >> 2) & 3, p2 = 3 - p0 - p1;
+            i = nxt;
+            j = (link >> 16) & 3;
+            bn = F.d.y;
+            if (__builtin_expect((link >> 18) & 1, 0))
+            {
+                ask = true;
+                k = kTetReload;
+            }
+            const TetVert X0 = V;
+            C0 = pick_vert(p0 == 0, p0 == 1, X0, X1, X2);
+            C1 = pick_vert(p1 == 0, p1 == 1, X0, X1, X2);
+            C2 = pick_vert(p2 == 0, p2 == 1, X0, X1, X2);
+            V = TetVert{F.c.x, F.c.y, F.d.x};
+            return 1;
         }
     };
 }

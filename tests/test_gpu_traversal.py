@@ -73,6 +73,33 @@ def test_voronoi_paths_bit_exact(eng, name, shift, repeat):
     _compare(eng, O.Grid("voronoi", **{k: t[k] for k in VOR_KEYS}), _rays(box, on, 1), repeat)
 
 
+@pytest.mark.parametrize("name", ["shared", "split", "grid"])
+def test_tetra_paths_bit_exact(eng, name):
+    """Rays through vertices, along edges and in faces' planes; split: no two cells share vertex ids,
+    so that every crossing reads the next cell's vertices."""
+    pkg = load_pkg()
+    box = np.array([-1.0, -1.0, -1.0, 1.0, 1.0, 1.0])
+    rng = np.random.default_rng(7)
+    if name == "grid":  # nearly a lattice: flat tetrahedra and rays that graze them
+        a = np.linspace(-0.8, 0.8, 5)
+        pts = np.stack(np.meshgrid(a, a, a, indexing="ij"), -1).reshape(-1, 3) + rng.normal(0, 1e-7, (125, 3))
+    else:
+        pts = rng.uniform(-1, 1, (400, 3))
+    b = pkg.Tetra.build(pts, box)
+    t = b.export()
+    b.close()
+    v, tv = np.asarray(t["verts"]).reshape(-1, 3), np.asarray(t["tet_verts"]).reshape(-1, 4)
+    if name == "split":
+        t["verts"], t["tet_verts"] = v[tv.ravel()], np.arange(tv.size, dtype=np.int32).reshape(-1, 4)
+    eng.grid_tetra(t["verts"], t["tet_verts"], t["face_nb"], t["face_normal"], t["box"])
+    rays = _rays(box, np.vstack([pts, 0.5 * (v[tv[:, 0]] + v[tv[:, 1]])]), 5)
+    to = v[tv[rng.integers(0, len(tv), 300), 2]] - rays[:300, :3]  # exactly toward vertices
+    rays[:300, 3:] = to / np.maximum(np.linalg.norm(to, axis=1, keepdims=True), 1e-300)
+    rays = rays[np.linalg.norm(rays[:, 3:], axis=1) > 0.5]
+    print("case tetra", name, len(tv), flush=True)
+    _compare(eng, O.Grid("tetra", **t), rays, 1)
+
+
 def _octree_flags(box, levels, refine):
     """Level-order division flags: nodes that `refine` (lo, hi, level) selects, up to `levels`."""
     flags, row = [], [(tuple(box[:3]), tuple(box[3:]))]
