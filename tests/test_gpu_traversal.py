@@ -196,3 +196,33 @@ def test_start_hints(eng, kind):
     for src in srcs:
         print("case start hint", kind, src, flush=True)
         _packets(eng, g, np.full(eng.num_cells(), 1e-3), src)
+
+
+def test_service_calls_share_an_engines_buffer():
+    """Optical depths and densities of growing and shrinking calls in turn, one beyond the buffer that
+    the engine keeps, give what an engine of their own gives."""
+    pkg = load_pkg()
+    b = np.linspace(-1.0, 1.0, 9)
+    rng = np.random.default_rng(3)
+    md = pkg.disk_model(tau_v=1.0, scale_length=0.3, scale_height=0.1)
+
+    def engine():
+        e = pkg.Engine(0)
+        e.grid_cartesian(b, b, b)
+        e.medium(np.linspace(0.0, 2e-3, 512))
+        e.dust([0.55e-6], [500.0], [300.0], [0.6])
+        return e
+
+    shared = engine()
+    rays = np.hstack([rng.uniform(-1, 1, (3000, 3)), np.tile([0.6, 0.0, 0.8], (3000, 1))])
+    for n in (1, 3000, 7, 4_400_000, 100):
+        print("case shared buffer", n, flush=True)
+        r = np.resize(rays, (n, 6))
+        got = shared.trace_tau(r)
+        e = engine()
+        want = e.trace_tau(r[:3000])
+        for g, w in zip(got, want):
+            np.testing.assert_array_equal(g, np.resize(w, n))
+        np.testing.assert_array_equal(shared.sample_density(md, 5, n), e.sample_density(md, 5, n))
+        e.close()
+    shared.close()
