@@ -39,7 +39,7 @@ import numpy as np
 ROOT = os.path.dirname(os.path.abspath(__file__))
 HBM_PEAK_GBS = 8000.0
 CPU_PACKETS_DEFAULT = 1.5e6  # packets of the reference CPU sample on the octree disk (about 12 s on 16 cores)
-BYTES_PER_SEGMENT = 64.0  # octree: node bounds 48 B + leaf/cell 4 B + neighbour entry 4 B + density 8 B
+BYTES_PER_SEGMENT = 64.0  # octree: the 64-byte node record (bounds, six neighbours, density, cell)
 BYTES_PER_ATOMIC = 8.0
 BYTES_PER_REQUEST = 96.0  # per traversal: request 32 B + packet position/direction/bin 52 B + result 12 B
 
@@ -477,8 +477,8 @@ def main():
     elif a.workload == "tetra-batch":
         wl = workloads.tetra_batch(packet_scale=a.batch_scale, threads=threads)
         ncells = int(wl.tables["ntets"])
-        # tetra crossing: the 256-B record (4 vertices, 4 outward normals, 4 neighbours, density)
-        bytes_per_segment = 256.0
+        # tetra crossing: the exit face's 64-B record (normal, next cell, its far vertex and density)
+        bytes_per_segment = 64.0
         a.packets = wl.total_packets()
         wdesc = ("%d batched instances of the tau_V=1 disk (tau_V 0.1-50, inclination 0-90 deg, %.0f packets in "
                  "all) on a %d-tetra Delaunay mesh of 2e5 density-sampled points" %
@@ -489,9 +489,9 @@ def main():
     else:
         wl = workloads.voronoi_clumpy(num_sites=a.sites, threads=threads)
         ncells, nnb = wl.tables["mesh"].info()[:2]
-        # Voronoi crossing: the cell's run in the entry table, a 32 B header (density, entry
-        # count) + one 32 B entry per neighbour (site, id, the neighbour's run)
-        bytes_per_segment = 32.0 + 32.0 * nnb / ncells
+        # Voronoi crossing: the cell's run in the entry table, a 48 B head (site, density, entry
+        # count) + one 16 B entry per neighbour (FP32 site offset, the neighbour's run)
+        bytes_per_segment = 48.0 + 16.0 * nnb / ncells
         wdesc = "Voronoi %d sites, lognormal clumpy medium (P(k)~k^-3.7, sigma_ln 1), mean tauV=5, 3 frames" % ncells
         a.no_guide = True
         if a.cpu_packets == CPU_PACKETS_DEFAULT:
