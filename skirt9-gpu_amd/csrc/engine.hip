@@ -2860,9 +2860,9 @@ int skg_autotune(skg_engine* e, uint64_t first_history, uint64_t trial_packets, 
     };
     std::vector<Cand> cands;
     const int cus = e->cus;
-    // transition thresholds: the octree and Voronoi kernels are fastest around 16-24 waiting
-    // lanes, the Cartesian and tetra kernels with rounds only once every lane of the wave waits
-    // (64); the candidates cover both
+    // transition thresholds: the octree kernel is fastest around 32 waiting lanes (ten levels, 2^21
+    // packets: 42.9 ms at 16, 37.9 at 32), the Cartesian kernel with rounds only once every lane of
+    // the wave waits (22.1 ms at 64, 24.2 at 32); the candidates cover both
     if (engines & 1)
         for (int thr : {12, 16, 20, 24, 32, 48, 64})
             for (int wg : {4 * cus, 8 * cus}) cands.push_back({SKG_MODE_PERSISTENT, thr, wg, e->poolSlots, e->traceBlocks, e->graphIters});
