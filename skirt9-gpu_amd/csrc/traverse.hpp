@@ -1126,8 +1126,8 @@ namespace skg
             // the domain, the cell is the set of points nearer to its site than to the sites
             // across its faces, so that site is then the nearest of all
             const bool there = !hinted || S.mn > S.en2;
-            // one neighbour is nearer than all the others can be
-            const bool one = S.l1 > 0.f && 1.00001f * (2.f * S.a1 - S.l1) < S.l2 && kk > 1e-12f && kk < 1e12f;
+            // one neighbour is nearer than all the others can be (none at all: resolve() steps on)
+            const bool one = S.id != kVorNone && S.l1 > 0.f && 1.00001f * (2.f * S.a1 - S.l1) < S.l2 && kk > 1e-12f && kk < 1e12f;
             j = kVorAsk;
             if (there)
             {

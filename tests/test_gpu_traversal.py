@@ -226,3 +226,26 @@ def test_service_calls_share_an_engines_buffer():
         np.testing.assert_array_equal(shared.sample_density(md, 5, n), e.sample_density(md, 5, n))
         e.close()
     shared.close()
+
+
+@pytest.mark.parametrize("repeat", [1, 70], ids=["four_lanes", "one_lane"])
+def test_voronoi_cells_without_a_face_ahead(eng, repeat):
+    """Cells whose lists hold no neighbour ahead of the path, or none at all: the path steps on by eps
+    until the nearest site is another cell's, as with the oracle."""
+    sites = np.array([[-0.5, 0.0, 0.0], [0.5, 0.0, 0.0], [0.5, 0.0, 0.9]])
+    lists = [[-1], [-1, -2, -3, -4, -5, 2], []]
+    count = np.array([len(q) for q in lists], np.int32)
+    box = np.array([-1.0, -1.0, -1.0, 1.0, 1.0, 1.0])
+    t = dict(sites=sites, nb_begin=np.array([0, 1, 7], np.int32), nb_count=count,
+             nb_index=np.array(sum(lists, []), np.int32), block_n=1, block_begin=np.array([0], np.int32),
+             block_count=np.array([3], np.int32), block_index=np.arange(3, dtype=np.int32), box=box)
+    eng.grid_voronoi(*[t[k] for k in VOR_KEYS])
+    # from a few eps (3.5e-12) before the plane x = 0, and from above the third site's plane z = 0.45
+    rng = np.random.default_rng(11)
+    n = 2000
+    first = np.arange(n) % 2 == 0
+    r = np.stack([np.where(first, -4e-11 * rng.random(n), 0.3), 0.2 * rng.normal(size=n).clip(-3, 3),
+                  np.where(first, -0.3, 0.45 + 4e-11 * rng.random(n))], 1)
+    k = np.stack([np.where(first, 1.0, 0.3), 0.1 * rng.normal(size=n), np.where(first, 0.1, -1.0)], 1)
+    print("case voronoi without a face ahead", repeat, flush=True)
+    _compare(eng, O.Grid("voronoi", **t), np.hstack([r, k / np.linalg.norm(k, axis=1, keepdims=True)]), repeat)
