@@ -299,7 +299,8 @@ namespace skg
     __global__ void __launch_bounds__(256)
         sample_density_kernel(GridView g, DiskModel md, int n, uint64_t seed, int64_t count, double* out)
     {
-        const int64_t m = (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) / kSampleLanes;
+        const int64_t block = static_cast<int64_t>(blockIdx.y) * gridDim.x + blockIdx.x;
+        const int64_t m = (block * blockDim.x + threadIdx.x) / kSampleLanes;
         if (m >= count) return;
         const int sub = threadIdx.x % kSampleLanes;
         double sum;
@@ -1879,7 +1880,9 @@ int skg_sample_density(skg_engine* e, const skg_disk_model* model, int32_t num_s
     Scratch w(e);
     HIPCHK(e, w.reserve(static_cast<size_t>(e->ncells) * sizeof(double)));
     double* d = w.take<double>(e->ncells);
-    dim3 grid(blocksFor(e->ncells * kSampleLanes)), block(256);
+    // (a launch holds less than 2^32 threads along x: 2^30 cells and more take several rows of workgroups)
+    const unsigned blocks = blocksFor(e->ncells * kSampleLanes), row = 1u << 22;
+    dim3 grid(std::min(blocks, row), (blocks + row - 1) / row), block(256);
     if (e->gridType == SKG_GRID_CARTESIAN)
         hipLaunchKernelGGL(sample_density_kernel<kCartesian>, grid, block, 0, e->stream, e->grid, md, num_samples, seed, e->ncells, d);
     else if (e->gridType == SKG_GRID_OCTREE)
