@@ -2136,13 +2136,14 @@ static int runPersistent(skg_engine* e, uint64_t first_history, uint64_t count)
     (void)hipGetLastError();
     int threads = e->threads;
     int blocks = e->workgroups > 0 ? e->workgroups : e->cus * 8;
-    // Never more lanes than packets, and a run that does not fill two wavefronts per SIMD is
-    // spread over that many, with fewer lanes of each: a wave waits for the longest of its lanes
-    // at every step, and 4096 packets in full wavefronts would use 16 of the 256 CUs (Cartesian
-    // 32^3, 4096 packets: 0.92 -> 0.64 ms).  Below four lanes the waves only add up.
+    // Never more lanes than packets, and a run that does not fill two wavefronts per SIMD (or as many
+    // as the caller's workgroups have) is spread over that many, with fewer lanes of each: a wave
+    // waits for the longest of its lanes at every step, and 4096 packets in full wavefronts would use
+    // 16 of the 256 CUs (Cartesian 32^3, 4096 packets: 0.92 -> 0.64 ms).  Below four lanes the waves
+    // only add up.
     const int lanes = pathLanes(e, count);
-    p.lanes = static_cast<int>(
-        std::clamp<int64_t>((static_cast<int64_t>(count) + 8 * e->cus - 1) / (8 * e->cus), 4, 64 / lanes));
+    const int64_t waves = std::min<int64_t>(8 * e->cus, static_cast<int64_t>(blocks) * (threads / 64));
+    p.lanes = static_cast<int>(std::clamp<int64_t>((static_cast<int64_t>(count) + waves - 1) / waves, 4, 64 / lanes));
     const int64_t perBlock = static_cast<int64_t>(p.lanes) * (threads / 64);
     int64_t needBlocks = (static_cast<int64_t>(count) + perBlock - 1) / perBlock;
     blocks = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(blocks, needBlocks)));

@@ -249,3 +249,31 @@ def test_voronoi_cells_without_a_face_ahead(eng, repeat):
     k = np.stack([np.where(first, 1.0, 0.3), 0.1 * rng.normal(size=n), np.where(first, 0.1, -1.0)], 1)
     print("case voronoi without a face ahead", repeat, flush=True)
     _compare(eng, O.Grid("voronoi", **t), np.hstack([r, k / np.linalg.norm(k, axis=1, keepdims=True)]), repeat)
+
+
+def test_few_workgroups_use_all_their_lanes(eng):
+    """A small run held to one workgroup takes all its 256 lanes: 1000 packets are then four in a row per
+    lane instead of one, and full wavefronts take at most about three times as long per step as those of
+    four lanes.  (With four lanes of each wavefront they would be 63 in a row.)"""
+    b = np.linspace(-1.0, 1.0, 33)
+    eng.grid_cartesian(b, b, b)
+    eng.medium(np.full(32 ** 3, 1e-3))
+    eng.dust([0.55e-6], [5000.0], [3000.0], [0.6])
+    eng.frame_remove_all()
+    eng.frame_add(1.0, 0.0, 0.0, 20, 20, 4.0, 4.0)
+    eng.source_point((0.0, 0.0, 0.0), [1e-3])
+    eng.options(0.5, 1e4, 0, 0, 5)
+    eng.tune_pipeline(1)
+    print("case few workgroups", flush=True)
+    ms, flux = {}, {}
+    for wg in (0, 1):
+        eng.tune(wg, 256, 32)
+        runs = []
+        for _ in range(4):
+            eng.frame_clear()
+            eng.run_packets(0, 1000)
+            runs.append(eng.last_kernel_ms())
+        ms[wg], flux[wg] = min(runs), eng.frame_read(0).sum()
+    eng.tune(0, 256, 16)
+    assert flux[1] == pytest.approx(flux[0], rel=1e-12)
+    assert ms[1] < 12 * ms[0], ms
