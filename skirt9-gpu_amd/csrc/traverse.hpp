@@ -598,11 +598,15 @@ namespace skg
     // neighbour's site and w of the position from the cell's site, the bisector is at the distance
     // a = n.(n / 2 - w) / n.k.  The numerator is off by at most En = eps (r2 + w.w) and the
     // denominator by Ed = eps r1 |k|, with the cell's largest n.n (r2) and 1-norm (r1); where the
-    // denominator exceeds 4 Ed, a is then off by at most 2 (En + a Ed) / n.k.  A denominator within
-    // 4 Ed of zero makes the neighbour an exit at any distance, a smaller one makes it no exit.
+    // denominator exceeds 6 Ed, a is then off by at most 2 (En + a Ed) / n.k.  A denominator below
+    // -4 Ed makes the neighbour no exit.  One between the two (a face parallel to the path) makes it an
+    // exit at any distance from (num - En) / 7 Ed on, which the same formula with 6 Ed as the
+    // denominator stays below, or no exit at all.  (Without that bound, which the walls' cells of every
+    // mesh need, such crossings went to the exact search.  2^18 packets seen face-on and at 60 degrees,
+    // lattice of 36^3 sites: 26.6 -> 11.4 ms; and edge-on, 60 000 sites: 32.5 -> 23.6 ms.)
     struct VorSearch
     {
-        float wx, wy, wz, fx, fy, fz, en2, ed2, ed4;
+        float wx, wy, wz, fx, fy, fz, en2, ed2, ed4, ed6;
         float l1, l2, a1, mn;  // the two smallest lower bounds, the first one's distance; the smallest numerator
         int id;
 
@@ -611,10 +615,11 @@ namespace skg
         {
             const float num = fmaf(v.x, fmaf(0.5f, v.x, -wx), fmaf(v.y, fmaf(0.5f, v.y, -wy), v.z * fmaf(0.5f, v.z, -wz)));
             const float den = fmaf(v.x, fx, fmaf(v.y, fy, v.z * fz));
-            const float r = __builtin_amdgcn_rcpf(den), a = num * r;
+            const float r = __builtin_amdgcn_rcpf(fmaxf(den, ed6));
+            float a = num * r;
             float lb = fmaf(-r, fmaf(a, ed2, en2), a);
-            lb = valid && den > ed4 ? lb : INFINITY;
-            lb = valid && fabsf(den) <= ed4 ? -1.f : lb;
+            lb = valid && den >= -ed4 ? lb : INFINITY;
+            a = den > ed6 ? a : INFINITY;  // no upper bound
             const bool first = lb < l1;
             l2 = __builtin_amdgcn_fmed3f(l1, lb, l2);
             l1 = first ? lb : l1;
@@ -1105,6 +1110,7 @@ namespace skg
             S.en2 = 2.f * kVorEps * fmaf(S.wx, S.wx, fmaf(S.wy, S.wy, fmaf(S.wz, S.wz, R.c.z)));
             S.ed2 = 2.f * kVorEps * kk * R.c.w;
             S.ed4 = 2.f * S.ed2;
+            S.ed6 = 3.f * S.ed2;
             S.l1 = S.l2 = S.mn = INFINITY;
             S.a1 = 0.f;
             S.id = kVorNone;

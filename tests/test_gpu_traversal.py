@@ -277,3 +277,60 @@ def test_few_workgroups_use_all_their_lanes(eng):
     eng.tune(0, 256, 16)
     assert flux[1] == pytest.approx(flux[0], rel=1e-12)
     assert ms[1] < 12 * ms[0], ms
+
+
+def test_voronoi_paths_along_faces_are_no_slower(eng):
+    """A view in a plane of the lattice's faces against one that no face is parallel to, by time: the
+    peel-offs cross as many cells, and no crossing needs the search in FP64."""
+    pkg = load_pkg()
+    box = np.array([-1.0, -1.0, -1.0, 1.0, 1.0, 1.0])
+    a = (np.arange(24) + 0.5) / 12 - 1
+    b = pkg.Voronoi.build(np.stack(np.meshgrid(a, a, a, indexing="ij"), -1).reshape(-1, 3), box)
+    b.upload(eng)
+    b.close()
+    eng.medium(np.full(24 ** 3, 1e-3))
+    eng.dust([0.55e-6], [2000.0], [1200.0], [0.6])
+    eng.source_point((0.01, 0.02, 0.03), [1e-5])
+    eng.options(0.5, 1e4, 0, 0, 5)
+    eng.tune_pipeline(1)
+    ms = []
+    for azimuth in (0.3, 0.0):  # at 0, the view has no component along y
+        eng.frame_remove_all()
+        eng.frame_add(0.9, azimuth, 0.0, 20, 20, 4.0, 4.0)
+        print("case voronoi view", azimuth, flush=True)
+        runs = []
+        for _ in range(4):
+            eng.frame_clear()
+            eng.run_packets(0, 200_000)
+            runs.append(eng.last_kernel_ms())
+        ms.append(min(runs))
+    assert ms[1] < 1.25 * ms[0], ms
+
+
+@pytest.mark.parametrize("repeat", [1, 70], ids=["four_lanes", "one_lane"])
+@pytest.mark.parametrize("name", ["lattice", "few", "many"])
+def test_voronoi_paths_almost_along_faces_bit_exact(eng, name, repeat):
+    """Directions 1e-2 to 1e-12 away from a face's plane, around where the FP32 bounds take the face for
+    parallel, from inside cells and from close to their faces."""
+    pkg = load_pkg()
+    box = np.array([0.0, 0.0, 0.0, 1.0, 1.0, 1.0])
+    b = pkg.Voronoi.build(_vor_points(name), box)
+    t = b.export()
+    b.upload(eng)
+    b.close()
+    rng = np.random.default_rng(12)
+    n, s = 2000, np.asarray(t["sites"])
+    i, q = rng.integers(0, len(s), n), rng.integers(0, 3, n)
+    near = np.argsort(((s[:, None] - s[None]) ** 2).sum(-1), axis=1)[i, 1 % len(s)] if len(s) < 800 else i
+    normal = s[near] - s[i]
+    wall = (np.arange(n) % 3 == 0) | (np.linalg.norm(normal, axis=1) == 0)
+    normal[wall] = np.eye(3)[q[wall]]
+    normal /= np.linalg.norm(normal, axis=1, keepdims=True)
+    k = np.cross(normal, rng.normal(size=(n, 3)))
+    k /= np.linalg.norm(k, axis=1, keepdims=True)
+    k += normal * (10.0 ** rng.uniform(-12, -2, (n, 1)) * rng.choice([-1.0, 1.0], (n, 1)))
+    r = np.where((np.arange(n) % 2 == 0)[:, None], s[i], 0.5 * (s[i] + s[near]))
+    r = np.clip(r + normal * (10.0 ** rng.uniform(-12, -1, (n, 1)) * rng.choice([-1.0, 1.0], (n, 1))), 1e-9, 1 - 1e-9)
+    print("case voronoi almost along faces", name, repeat, flush=True)
+    _compare(eng, O.Grid("voronoi", **{k_: t[k_] for k_ in VOR_KEYS}),
+             np.hstack([r, k / np.linalg.norm(k, axis=1, keepdims=True)]), repeat)
