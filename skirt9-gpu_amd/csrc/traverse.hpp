@@ -524,7 +524,11 @@ namespace skg
     {
         const int w = -1 - id;  // 0..5: xmin, xmax, ymin, ymax, zmin, zmax
         if (w >= 6) return 0.;
-        const double face = w == 0 ? box[0] : w == 1 ? box[3] : w == 2 ? box[1] : w == 3 ? box[4] : w == 4 ? box[2] : box[5];
+        // (selected as values: a selection among the members' addresses made the pipeline's trace kernel
+        // keep its whole parameter block in scratch memory, 912 bytes per lane)
+        const bool up = w & 1;
+        const double x0 = box[0], y0 = box[1], z0 = box[2], x1 = box[3], y1 = box[4], z1 = box[5];
+        const double face = pick3(w < 2, w < 4, up ? x1 : x0, up ? y1 : y0, up ? z1 : z0);
         const double r = pick3(w < 2, w < 4, rx, ry, rz), k = pick3(w < 2, w < 4, kx, ky, kz);
         return (face - r) / k;
     }
