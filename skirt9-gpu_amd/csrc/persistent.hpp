@@ -606,7 +606,9 @@ namespace skg
                 pk.ry = p.src[1];
                 pk.rz = p.src[2];
             }
-            const int startHint = V == kParticles ? -1 : p.srcHint;
+            // (srcHint is the point source's cell: on a mesh, a particle far from it would first have that
+            // cell rejected, after a round's wait)
+            const int startHint = particles ? -1 : p.srcHint;
             isotropic(pk.rng, pk.kx, pk.ky, pk.kz);
             pk.nscatt = 0;
             pk.taupath = 0.;

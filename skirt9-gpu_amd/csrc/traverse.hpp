@@ -672,8 +672,10 @@ namespace skg
         uint32_t pend;  // octree: a node to descend into next and the crossed wall (node << 3 | wall),
                         // or kNoPend
         int hint;  // a cell that probably contains the start point (-1: none), after the first step
-                   // the start cell: octree a node, Voronoi a run, tetra a cell, Cartesian the cell's
-                   // indices i | j << 10 | k << 20 (no more than 1024 cells along an axis)
+                   // the start cell: octree a node, Voronoi a run (a hint that resolve() had to replace
+                   // stays: the position is then so near a face that its own cell would be rejected too),
+                   // tetra a cell, Cartesian the cell's indices i | j << 10 | k << 20 (no more than 1024
+                   // cells along an axis)
         static constexpr uint32_t kNoPend = 0xFFFFFFFFu;  // node ids stay below 2^29
 
         __device__ __forceinline__ void start(double r0, double r1, double r2, double k0, double k1, double k2,
