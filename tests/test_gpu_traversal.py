@@ -334,3 +334,56 @@ def test_voronoi_paths_almost_along_faces_bit_exact(eng, name, repeat):
     print("case voronoi almost along faces", name, repeat, flush=True)
     _compare(eng, O.Grid("voronoi", **{k_: t[k_] for k_ in VOR_KEYS}),
              np.hstack([r, k / np.linalg.norm(k, axis=1, keepdims=True)]), repeat)
+
+
+def _tetra_tables(points):
+    pkg = load_pkg()
+    b = pkg.Tetra.build(points, np.array([-1.0, -1.0, -1.0, 1.0, 1.0, 1.0]))
+    t = b.export()
+    b.close()
+    return t
+
+
+def test_tetra_records_of_a_large_mesh(eng):
+    """Copies of one mesh side by side, more cells than the records are built for at a time (2^20)."""
+    t = _tetra_tables(np.random.default_rng(7).uniform(-1, 1, (400, 3)))
+    v, tv = np.asarray(t["verts"]).reshape(-1, 3), np.asarray(t["tet_verts"]).reshape(-1, 4)
+    fn, nrm = np.asarray(t["face_nb"]).reshape(-1, 4), np.asarray(t["face_normal"]).reshape(-1, 4, 3)
+    n = (1 << 20) // len(tv) + 3
+    q = np.arange(n)
+    big = dict(verts=(v[None] + 2.25 * q[:, None, None] * np.array([1.0, 0.0, 0.0])).reshape(-1, 3),
+               tet_verts=(tv[None] + len(v) * q[:, None, None]).reshape(-1, 4).astype(np.int32),
+               face_nb=np.where(fn[None] < 0, -1, fn[None] + len(tv) * q[:, None, None]).reshape(-1, 4).astype(np.int32),
+               face_normal=np.tile(nrm, (n, 1, 1)), box=np.array([-1.0, -1.0, -1.0, 2.25 * n - 1.25, 1.0, 1.0]))
+    eng.grid_tetra(big["verts"], big["tet_verts"], big["face_nb"], big["face_normal"], big["box"])
+    copies = np.concatenate([[0, 1, n // 2], np.arange(n - 5, n)])
+    rays = np.concatenate([_rays(np.array([-0.9, -0.9, -0.9, 0.9, 0.9, 0.9]), v[8:], 20 + c, 25) + [2.25 * c, 0, 0, 0, 0, 0]
+                           for c in copies])
+    print("case tetra records of", n * len(tv), "cells", flush=True)
+    _compare(eng, O.Grid("tetra", **big), rays, 1)
+
+
+def test_tetra_tables_refused(eng):
+    """Wrong ids anywhere in the tables are refused, also in the last cell of a mesh that several threads
+    check, and the grid before stays."""
+    pkg = load_pkg()
+    t = _tetra_tables(np.random.default_rng(7).uniform(-1, 1, (6000, 3)))
+    v, tv, fn = (np.asarray(t[k]) for k in ("verts", "tet_verts", "face_nb"))
+    fn = fn.reshape(-1, 4)
+    assert len(fn) > 1 << 15
+    b = np.linspace(-1.0, 1.0, 5)
+    eng.grid_cartesian(b, b, b)
+    inner = int(np.flatnonzero((fn >= 0).all(1))[-1])
+    stranger = next(m for m in range(len(fn)) if m != inner and m not in fn[inner])
+    for cell in (0, inner, len(fn) - 1):
+        for name, value, text in (("tet_verts", -1, "vertex"), ("tet_verts", len(v.reshape(-1, 3)), "vertex"),
+                                  ("face_nb", -2, "neighbour"), ("face_nb", len(fn), "neighbour")):
+            bad = dict(t, **{name: np.array(t[name]).reshape(-1, 4)})
+            bad[name][cell, 3] = value
+            with pytest.raises(pkg.EngineError, match=text):
+                eng.grid_tetra(bad["verts"], bad["tet_verts"], bad["face_nb"], bad["face_normal"], bad["box"])
+    bad = np.array(fn)
+    bad[inner, 1] = stranger
+    with pytest.raises(pkg.EngineError, match="mutual"):
+        eng.grid_tetra(v, tv, bad, t["face_normal"], t["box"])
+    assert eng.num_cells() == 64
