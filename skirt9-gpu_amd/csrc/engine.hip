@@ -927,6 +927,32 @@ namespace
         return touches(t) && t[u] == b[u] && t[3 + u] == b[3 + u] && t[v] == b[v] && t[3 + v] == b[3 + v] ? top : kOctList;
     }
 
+    // f(first, last) over the shares of [0, n), on up to eight threads with `least` items each; the first
+    // share's message (nullptr: none)
+    template<typename F> const char* onThreads(int64_t n, int64_t least, F&& f)
+    {
+        const int count = static_cast<int>(std::clamp<int64_t>(n / least, 1, 8));
+        std::vector<const char*> said(count, nullptr);
+        const auto share = [&](int q) { said[q] = f(n * q / count, n * (q + 1) / count); };
+        std::vector<std::thread> team;
+        for (int q = 1; q < count; ++q)
+        {
+            try
+            {
+                team.emplace_back(share, q);
+            }
+            catch (const std::system_error&)
+            {
+                share(q);  // no more threads
+            }
+        }
+        share(0);
+        for (auto& th : team) th.join();
+        for (const char* text : said)
+            if (text) return text;
+        return nullptr;
+    }
+
     // block search lists for a tetrahedral grid: tbn^3 equal blocks over the domain; a tetra is
     // listed (in increasing index order) in every block its closed bounding box meets
     void buildTetraBlocks(const double* verts, int64_t nt, const int32_t* tet_verts, const double* box, int& tbn,
@@ -1203,10 +1229,7 @@ int skg_grid_octree(skg_engine* e, int64_t nnodes, const double* bounds, const i
     }
     if (ncells > INT32_MAX) return fail(e, SKG_ERR_ARGUMENT, "skg_grid_octree: too many cells");
     // one record per node; the leaves' neighbour lists keep their node ids
-    std::vector<OctNode> nodes(nnodes);
-    std::memset(nodes.data(), 0, nodes.size() * sizeof(OctNode));
-    std::vector<int32_t> nbc;
-    nbc.reserve(static_cast<size_t>(nb_off[6 * nnodes]));
+    std::vector<OctNode> nodes(nnodes, OctNode{});
     std::vector<char> seen(ncells, 0);
     std::vector<int32_t> parent(nnodes, -1);
     std::vector<int8_t> level(nnodes, 0);
@@ -1228,9 +1251,8 @@ int skg_grid_octree(skg_engine* e, int64_t nnodes, const double* bounds, const i
         if (fresh) planes.push_back(v);
         return it->second;
     };
-    std::vector<int32_t> nbOff;
-    nbOff.reserve(static_cast<size_t>(6 * nnodes + 1));
-    nbOff.push_back(0);
+    std::vector<int32_t> nbOff(static_cast<size_t>(6 * nnodes + 1), 0);
+    int64_t listed = 0;
     for (int64_t n = 0; n < nnodes; ++n)
     {
         OctNode& L = nodes[n];
@@ -1257,7 +1279,7 @@ int skg_grid_octree(skg_engine* e, int64_t nnodes, const double* bounds, const i
         {
             L.cell = ~child_first[n];
             for (int q = 0; q < 3; ++q) L.split[q] = plane(bounds[6 * static_cast<int64_t>(child_first[n]) + 3 + q]);
-            nbOff.insert(nbOff.end(), 6, static_cast<int32_t>(nbc.size()));
+            std::fill_n(nbOff.begin() + 6 * n + 1, 6, static_cast<int32_t>(listed));
             continue;
         }
         int32_t m = cell_index[n];
@@ -1266,19 +1288,34 @@ int skg_grid_octree(skg_engine* e, int64_t nnodes, const double* bounds, const i
         L.cell = m;
         for (int w = 0; w < 6; ++w)
         {
-            int64_t b0 = nb_off[6 * n + w], b1 = nb_off[6 * n + w + 1];
-            if (b1 < b0) return fail(e, SKG_ERR_ARGUMENT, "skg_grid_octree: offsets must not decrease");
-            for (int64_t q = b0; q < b1; ++q)
-            {
-                int32_t id = nb_id[q];
-                if (id < 0 || id >= nnodes || cell_index[id] < 0)
-                    return fail(e, SKG_ERR_ARGUMENT, "skg_grid_octree: a leaf's neighbour must be a leaf");
-                nbc.push_back(id);
-            }
-            nbOff.push_back(static_cast<int32_t>(nbc.size()));
-            L.first[w] = octAcross(bounds, parent.data(), level.data(), static_cast<int32_t>(n), w, nb_id + b0, b1 - b0);
+            const int64_t count = nb_off[6 * n + w + 1] - nb_off[6 * n + w];
+            if (count < 0) return fail(e, SKG_ERR_ARGUMENT, "skg_grid_octree: offsets must not decrease");
+            listed += count;
+            nbOff[6 * n + w + 1] = static_cast<int32_t>(listed);
         }
     }
+    // the lists, and the node across each wall (1.7e6 nodes: 206 -> 156 ms a call on eight threads)
+    std::vector<int32_t> nbc(static_cast<size_t>(listed));
+    const auto across = [&](int64_t first, int64_t last) -> const char* {
+        for (int64_t n = first; n < last; ++n)
+        {
+            if (child_first[n] >= 0) continue;
+            for (int w = 0; w < 6; ++w)
+            {
+                const int64_t b0 = nb_off[6 * n + w], count = nb_off[6 * n + w + 1] - b0;
+                for (int64_t q = 0; q < count; ++q)
+                {
+                    const int32_t id = nb_id[b0 + q];
+                    if (id < 0 || id >= nnodes || cell_index[id] < 0)
+                        return "skg_grid_octree: a leaf's neighbour must be a leaf";
+                    nbc[nbOff[6 * n + w] + q] = id;
+                }
+                nodes[n].first[w] = octAcross(bounds, parent.data(), level.data(), static_cast<int32_t>(n), w, nb_id + b0, count);
+            }
+        }
+        return nullptr;
+    };
+    if (const char* bad = onThreads(nnodes, 16384, across)) return fail(e, SKG_ERR_ARGUMENT, bad);
     for (int64_t m = 0; m < ncells; ++m)
         if (!seen[m]) return fail(e, SKG_ERR_ARGUMENT, "skg_grid_octree: cell indices must be 0..ncells-1");
     std::lock_guard<std::mutex> lk(e->mu);
@@ -1449,26 +1486,7 @@ int skg_grid_tetra(skg_engine* e, int64_t nverts, const double* verts, int64_t n
         }
         return nullptr;
     };
-    // (a thread per 16 384 cells, eight at most)
-    const int nthr = static_cast<int>(std::clamp<int64_t>(ntets >> 14, 1, 8));
-    std::vector<const char*> bad(nthr, nullptr);
-    const auto share = [&](int q) { bad[q] = check(ntets * q / nthr, ntets * (q + 1) / nthr); };
-    std::vector<std::thread> team;
-    for (int q = 1; q < nthr; ++q)
-    {
-        try
-        {
-            team.emplace_back(share, q);
-        }
-        catch (const std::system_error&)
-        {
-            share(q);  // no more threads
-        }
-    }
-    share(0);
-    for (auto& th : team) th.join();
-    for (const char* b : bad)
-        if (b) return fail(e, SKG_ERR_ARGUMENT, b);
+    if (const char* bad = onThreads(ntets, 16384, check)) return fail(e, SKG_ERR_ARGUMENT, bad);
     int tbn = 0;
     std::vector<double> borders;
     std::vector<int32_t> off, ids;

@@ -387,3 +387,31 @@ def test_tetra_tables_refused(eng):
     with pytest.raises(pkg.EngineError, match="mutual"):
         eng.grid_tetra(v, tv, bad, t["face_normal"], t["box"])
     assert eng.num_cells() == 64
+
+
+def test_octree_of_several_threads_shares(eng):
+    """A tree whose node records several threads prepare: paths bit for bit, and wrong lists in its first
+    and last leaf are refused."""
+    pkg = load_pkg()
+    box = np.array([-1.0, -1.0, -1.0, 1.0, 1.0, 1.0])
+    rng = np.random.default_rng(14)
+    tree = pkg.Octree.from_flags(box, _octree_flags(box, 6, lambda lo, hi, level: level < 4 or rng.random() < 0.5))
+    t = tree.export()
+    tree.upload(eng)
+    tree.close()
+    keys = ("bounds", "child_first", "cell_index", "nb_off", "nb_id")
+    print("case octree of", len(t["cell_index"]), "nodes", flush=True)
+    assert len(t["cell_index"]) > 50000
+    corners = np.asarray(t["bounds"]).reshape(-1, 6)[:, 3:]
+    rays = _rays(box, corners[rng.integers(0, len(corners), 500)], 15)
+    _compare(eng, O.Grid("octree", **{k: t[k] for k in keys}), rays, 1)
+    cells = eng.num_cells()
+    leaves = np.flatnonzero(np.asarray(t["cell_index"]) >= 0)
+    listed = [n for n in leaves if t["nb_off"][6 * n + 6] > t["nb_off"][6 * n]]
+    for n in (listed[0], listed[-1]):
+        for value in (-1, len(t["cell_index"]), 0):  # (node 0 is the root, no leaf)
+            bad = np.array(t["nb_id"])
+            bad[t["nb_off"][6 * n]] = value
+            with pytest.raises(pkg.EngineError, match="leaf"):
+                eng.grid_octree(t["bounds"], t["child_first"], t["cell_index"], t["nb_off"], bad)
+    assert eng.num_cells() == cells
