@@ -821,27 +821,42 @@ namespace
         return SKG_OK;
     }
 
-    // dynamic LDS of the kernels that walk the grid: the octree's coordinate table
+    // dynamic LDS of the kernels that walk the grid: the coordinate table of an octree or Cartesian grid
     size_t planeBytes(const GridView& g) { return g.ldsPlanes ? static_cast<size_t>(g.nplanes) * sizeof(double) : 0; }
 
+    // coordinates beside which three workgroups of the life cycle fit into a CU's 160 KB of LDS (allotted
+    // in units of 1280 bytes)
+    constexpr int kPlanesOfThree = (163840 / 3 / 1280 * 1280 - kColdBytes - 64) / static_cast<int>(sizeof(double));
+
     template<int GT, int FP, int L>
-    hipError_t launchLifecycle(const SimParams& p, bool guided, int blocks, int threads, hipStream_t s)
+    hipError_t launchLifecycle(const SimParams& params, bool guided, int blocks, int threads, int cus, hipStream_t s)
     {
-        const size_t lds = planeBytes(p.grid);
+        const auto launch = [&](auto variant) {
+            constexpr int V = decltype(variant)::value;
+            SimParams p = params;
+            // An octree whose table leaves room for two workgroups only is read from memory where the
+            // kernel is built for three and the run has more than two: 2^20 packets, 2852 coordinates
+            // 19.2 -> 18.0 ms (2785: 18.8 -> 17.3).  With fewer workgroups, or those variants that are
+            // built for two, the table in LDS is faster (5000 packets 2.6 -> 2.4, field 11.3 -> 10.8 ms),
+            // and so it is for Cartesian grids (2403 borders: 68.7 -> 64.6).
+            if (GT == kOctree && lifecycle_waves<GT, V>() == 3 && blocks > 2 * cus && p.grid.nplanes > kPlanesOfThree)
+                p.grid.ldsPlanes = 0;
+            hipLaunchKernelGGL((lifecycle<GT, FP, V, L>), dim3(blocks), dim3(threads), planeBytes(p.grid), s, p);
+        };
         // batched instances, guided sampling and radiation-field storage take their own
         // instantiations; the plain run carries none of them
-        if (p.ninst)
-            hipLaunchKernelGGL((lifecycle<GT, FP, kBatched, L>), dim3(blocks), dim3(threads), lds, s, p);
-        else if (p.rf)
-            hipLaunchKernelGGL((lifecycle<GT, FP, kStoreRF, L>), dim3(blocks), dim3(threads), lds, s, p);
-        else if (p.persp)
-            hipLaunchKernelGGL((lifecycle<GT, FP, kPersp, L>), dim3(blocks), dim3(threads), lds, s, p);
-        else if (p.nent)
-            hipLaunchKernelGGL((lifecycle<GT, FP, kParticles, L>), dim3(blocks), dim3(threads), lds, s, p);
+        if (params.ninst)
+            launch(std::integral_constant<int, kBatched>());
+        else if (params.rf)
+            launch(std::integral_constant<int, kStoreRF>());
+        else if (params.persp)
+            launch(std::integral_constant<int, kPersp>());
+        else if (params.nent)
+            launch(std::integral_constant<int, kParticles>());
         else if (guided)
-            hipLaunchKernelGGL((lifecycle<GT, FP, kGuided, L>), dim3(blocks), dim3(threads), lds, s, p);
+            launch(std::integral_constant<int, kGuided>());
         else
-            hipLaunchKernelGGL((lifecycle<GT, FP, kPlain, L>), dim3(blocks), dim3(threads), lds, s, p);
+            launch(std::integral_constant<int, kPlain>());
         return hipGetLastError();
     }
 }
@@ -2232,8 +2247,8 @@ static int runPersistent(skg_engine* e, uint64_t first_history, uint64_t count)
     hipError_t err;
     dispatchLanes(e, static_cast<int64_t>(count), [&](auto gt, auto nl) {
         constexpr int GT = decltype(gt)::value, L = decltype(nl)::value;
-        err = e->fpMode == SKG_FP64 ? launchLifecycle<GT, SKG_FP64, L>(p, guided, blocks, threads, e->stream)
-                                    : launchLifecycle<GT, SKG_FP32_KAHAN, L>(p, guided, blocks, threads, e->stream);
+        err = e->fpMode == SKG_FP64 ? launchLifecycle<GT, SKG_FP64, L>(p, guided, blocks, threads, e->cus, e->stream)
+                                    : launchLifecycle<GT, SKG_FP32_KAHAN, L>(p, guided, blocks, threads, e->cus, e->stream);
         return 0;
     });
     if (err != hipSuccess) return fail(e, SKG_ERR_DEVICE, std::string("lifecycle launch: ") + hipGetErrorString(err));

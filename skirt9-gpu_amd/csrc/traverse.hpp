@@ -115,8 +115,8 @@ namespace skg
     // crossing reads: its bounds, number density, cell index and, per wall, the node across it.  An
     // inner node holds its bounds, its first child and its split point (the upper corner of the first
     // child, TreeNode::leafChild's test point).  Bounds and split points are indices into the table
-    // of the tree's distinct coordinates (GridView::planes, 3075 FP64 values for ten levels), which
-    // the kernels keep in LDS: a crossing reads half a cache line instead of a whole one, two
+    // of the tree's distinct coordinates (GridView::planes: at most 3075 FP64 values for ten
+    // levels, 1025 in a cube around the origin), which the kernels keep in LDS: a crossing reads half a cache line instead of a whole one, two
     // siblings share a line, and the 3.4e6 nodes of the spiral disk take 215 MB, less than the
     // last-level cache, instead of 430 MB.
     //
@@ -141,7 +141,7 @@ namespace skg
     static_assert(offsetof(OctNode, first) == 24 && offsetof(OctNode, dens) == 48 && offsetof(OctNode, cell) == 56,
                   "node record layout that OctRec reads");
     constexpr int32_t kOctNoNb = -1, kOctList = -2;
-    constexpr int kLdsPlanes = 3200;  // coordinates kept in LDS at most (25.6 KB): ten levels have 3075
+    constexpr int kLdsPlanes = 3200;  // coordinates kept in LDS at most (25.6 KB): ten levels have up to 3075
 
     // Read-only grid tables resident in HBM.  Octree: the node records and the leaves' neighbour
     // lists (node ids, sorted by decreasing overlap as TreeNode::sortNeighbors).

@@ -415,3 +415,42 @@ def test_octree_of_several_threads_shares(eng):
             with pytest.raises(pkg.EngineError, match="leaf"):
                 eng.grid_octree(t["bounds"], t["child_first"], t["cell_index"], t["nb_off"], bad)
     assert eng.num_cells() == cells
+
+
+@pytest.mark.parametrize("npk", [3000, 150_000], ids=["table_in_lds", "table_in_memory"])
+def test_octree_of_many_coordinates(eng, npk):
+    """A tree whose coordinate table leaves room for two of the life cycle's workgroups per compute unit:
+    long runs read it from memory, short ones keep it in LDS.  Against the oracle."""
+    pkg = load_pkg()
+    box = np.array([-1.0, -0.9, -1.1, 1.3, 1.0, 0.8])
+    size = box[3:] - box[:3]
+
+    def diagonal(lo, hi, level):
+        return max((np.array(lo) - box[:3]) / size) <= min((np.array(hi) - box[:3]) / size)
+
+    tree = pkg.Octree.from_flags(box, _octree_flags(box, 10, diagonal))
+    t = tree.export()
+    tree.upload(eng)
+    tree.close()
+    assert 2360 < len(np.unique(t["bounds"])) <= 3200
+    dens = 1e-3 * np.random.default_rng(3).lognormal(0.0, 0.5, eng.num_cells())
+    eng.medium(dens)
+    eng.dust([0.55e-6], [900.0], [540.0], [0.6])
+    fr = frame60(npix=20)
+    fr["fovx"] = fr["fovy"] = 4.0
+    eng.frame_remove_all()
+    eng.frame_add(fr["inclination"], fr["azimuth"], fr["roll"], fr["nx"], fr["ny"], fr["fovx"], fr["fovy"])
+    src = (0.0, 0.1, -0.1)
+    eng.source_point(src, [1.0 / npk])
+    eng.options(0.5, 1e4, 0, 0, 13)
+    eng.tune_pipeline(1)
+    print("case octree of many coordinates", npk, flush=True)
+    eng.run_packets(0, npk)
+    img, cnt = eng.frame_read(0)[0], eng.counters()
+    ofr, ocnt = O.simulate(O.Grid("octree", **{k: t[k] for k in ("bounds", "child_first", "cell_index", "nb_off", "nb_id")}),
+                           dens, [0.55e-6], [900.0], [540.0], [0.6], [1.0 / npk], [fr], 0, npk, threads=8, seed=13, src=src)
+    assert cnt[0] == ocnt[0] == npk
+    assert abs(int(cnt[2]) - int(ocnt[2])) <= 1e-3 * ocnt[2]
+    assert abs(img.sum() / ofr[0][0].sum() - 1) < 1e-6
+    nz = ofr[0][0] > 0
+    assert np.median(np.abs(img[nz] / ofr[0][0][nz] - 1)) < 1e-9
