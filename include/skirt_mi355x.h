@@ -239,8 +239,11 @@ int skg_counters(skg_engine* e, int64_t* out8);
 int skg_counters_n(skg_engine* e, int64_t* out, int32_t n);
 
 /* Launch shape of the persistent life-cycle kernel: workgroups (0 = automatic), threads per
- * workgroup (64..1024, multiple of 64) and the number of lanes of a wavefront that must be
- * waiting before a wave-wide transition round runs (1..64).  Chosen by the autotuner. */
+ * workgroup (64..256, multiple of 64) and the share of a wavefront's lanes, in 64ths (1..64),
+ * that must be waiting before a wave-wide transition round runs: of a full wavefront that many
+ * lanes, of the lanes that still have packets (small runs, the end of every run) the same share,
+ * rounded up.  Lanes that wait for the guide's network are not counted among them.  Chosen by
+ * the autotuner. */
 int skg_tune(skg_engine* e, int32_t workgroups, int32_t threads, int32_t transition_threshold);
 
 /* Autotuner (no counterpart in the reference, which has no launch parameters): times a trial

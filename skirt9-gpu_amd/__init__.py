@@ -20,6 +20,10 @@ import numpy as np
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libskirt_mi355x.so")
 
+# what the launch parameters of a saved tuning mean (2: the transition threshold as a share of the
+# lanes that still take part); entries of another meaning are tuned again
+TUNING_RULE = 2
+
 SKG_OK = 0
 SKG_GRID_CARTESIAN = 0
 SKG_GRID_OCTREE = 1
@@ -407,7 +411,8 @@ class Engine:
         pool slots, trace workgroups, graph length) from timed trial runs of histories
         [first, ...) and keeps it; the detector contents are restored.  With `cache` (a JSON
         file) and `key`, a configuration stored under the key is applied without trials and
-        new results are stored.  Returns (config dict, trial packets/s or None)."""
+        new results are stored; an entry saved when the parameters meant something else
+        (TUNING_RULE) is replaced.  Returns (config dict, trial packets/s or None)."""
         import json
         names = ("mode", "threshold", "workgroups", "pool_slots", "trace_workgroups", "graph_iterations")
         if cache and key and os.path.exists(cache):
@@ -415,7 +420,7 @@ class Engine:
                 entry = json.load(open(cache)).get(key)
             except (OSError, ValueError):
                 entry = None
-            if entry:
+            if entry and entry.get("rule") == TUNING_RULE:
                 self.tune(int(entry["workgroups"]), 256, int(entry["threshold"]))
                 self.tune_pipeline(int(entry["mode"]), int(entry["pool_slots"]), int(entry["trace_workgroups"]),
                                    int(entry["graph_iterations"]))
@@ -432,7 +437,7 @@ class Engine:
                     data = json.load(open(cache))
                 except (OSError, ValueError):
                     data = {}
-            data[key] = dict(cfg, rate=rate.value)
+            data[key] = dict(cfg, rate=rate.value, rule=TUNING_RULE)
             with open(cache, "w") as f:
                 json.dump(data, f, indent=1)
         return cfg, rate.value
