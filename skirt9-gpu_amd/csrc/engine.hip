@@ -352,7 +352,7 @@ namespace skg
     // ------------------------------------------------------------------ cell densities
     constexpr uint32_t kTagDensity = 0x44454e53u;  // the host samplers' stream tag for cell densities
 
-    // Cell-averaged number density of the disk model in every cell of the resident grid (one thread
+    // Cell-averaged number density of the disk model in every cell of the resident grid (four threads
     // per cell) from n random points per cell, drawn from the same Philox stream (seed, cell, tag) and placed
     // the same way as the host samplers do (uniform in the Cartesian / octree cell box, x then
     // y then z; folded barycentric weights in a tetra), as MediumSystem's PropertySampler
@@ -882,10 +882,11 @@ namespace
 
     // The lanes of a wavefront that walk each of n paths together.  On a Voronoi grid four lanes share
     // a cell's neighbours where the paths do not fill the chip: a crossing's chain is then shorter and
-    // its loads coalesce, but the FP64 part runs four times.  ms with one / four lanes (60 000 sites):
-    //              2 000       30 000      120 000     250 000     1 000 000
-    //   packets    4.6 / 2.4   5.4 / 3.7   7.9 / 7.8   10.3 / 14.3  27.9 / 49.5
-    //   rays       1.3 / 0.6   1.4 / 0.8   1.9 / 1.6    2.9 / 3.2   10.9 / 13.1
+    // its loads coalesce, but the FP64 part runs four times.  ms with one / four lanes (60 000 sites; the
+    // rays' optical depths with the copies):
+    //              2 000         30 000        120 000       250 000       1 000 000
+    //   packets    5.9 / 2.9     7.8 / 4.5     8.8 / 8.1     12.6 / 13.4   31.1 / 46.1
+    //   rays       0.47 / 0.25   1.21 / 0.99   0.85 / 0.77   1.55 / 1.45   5.5 / 6.1
     int pathLanes(const skg_engine* e, int64_t n)
     {
         return e->gridType == SKG_GRID_VORONOI && n <= 512 * static_cast<int64_t>(e->cus) ? 4 : 1;

@@ -54,7 +54,7 @@ namespace skg
         uint32_t contKey;         // nonzero: histories continue on Philox tag contKey from their first
                                   // scattering on (same emission and first interaction, independent
                                   // continuations)
-        int32_t srcHint;          // the cell (octree: leaf node) of the point source (the start hint of new packets), -1: none
+        int32_t srcHint;          // the cell (octree: leaf node) of the point source (the start hint of its packets), -1: none
         double* rf;               // radiation-field variant: ncells x nlambda table
         int persp;                // some instruments are perspective instruments
         int nent;                 // particle-source variant: number of entities (0: the point source)
@@ -881,7 +881,7 @@ namespace skg
     //   octree, nine levels, 40 wavelengths, 3e5    8.4 /  8.4 /  8.1  events double the writes)
     //   octree with the radiation field, 2e5        7.8 / 11.6 / 13.2 (bound by its atomics, whose
     //   Cartesian with the field, 7e5              targets collide more with more waves)
-    //   Voronoi, 400 000 sites, 2^18 packets         - / 48.0 / 52.8
+    //   Voronoi, 400 000 sites, 2^18 packets       39.9 / 39.6 / 44.4
     //   tetra, 150 000 vertices, 64 instances, 2^20   - / 61.2 / 57.8
     // The guided variant's network call holds whole layers' weights in registers, and its four-wave build does not compile for the mesh grids.
     template<int GT, int V> constexpr int lifecycle_waves()

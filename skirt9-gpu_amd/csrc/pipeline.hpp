@@ -517,7 +517,8 @@ namespace skg
     constexpr unsigned kTraceChunk = 256;  // request indices a wavefront reserves at once
     constexpr int kTraceRefill = 8;        // idle lanes that trigger a refill round
 #ifndef SKG_TRACE_WAVES
-#define SKG_TRACE_WAVES (GT == kVoronoi ? 3 : 4)  // minimum waves per SIMD of the trace kernel
+// minimum waves per SIMD of the trace kernel (Voronoi, 60 000 sites, 300 000 packets at 3 / 4: 43.2 / 45.2 ms)
+#define SKG_TRACE_WAVES (GT == kVoronoi ? 3 : 4)
 #endif
     template<int GT, int FP> __global__ void __launch_bounds__(256, (SKG_TRACE_WAVES)) pipe_trace(PipeParams p, int in)
     {
@@ -604,9 +605,9 @@ namespace skg
                             dz = P.kz[slot];
                         }
                         // the packet stands in the cell of its last second pass's result, or at the
-                        // source.  (Without hints, the scans for the start cells took most of the
-                        // tetra and Voronoi runs: 30 000 vertices,
-                        // 200 000 packets 114 -> 28 ms, 60 000 sites, 300 000 packets 46 -> 40 ms.)
+                        // source.  (Without hints, the scans for the start cells took most of a
+                        // tetra run: 60 000 vertices, 200 000 packets 178 -> 47 ms; Voronoi, 60 000
+                        // sites, 300 000 packets 49.7 -> 43.2 ms.)
                         int hint = P.res_m[slot];
                         if (hint < 0)
                             hint = p.srcHint;

@@ -8,7 +8,7 @@
 //   Voronoi next()      VoronoiMeshSnapshot.cpp:1094-1213, cellIndex :1037-1071
 //   tetra next()        TetraMeshSpatialGrid.cpp:697-820, findEnteringFace :87-108, contains :110-133,
 //                       cellIndex :615-624
-// One lane owns one path; the generator state lives in registers.
+// One lane owns one path, or four lanes of a Voronoi path's; the generator state lives in registers.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -63,7 +63,7 @@ namespace skg
     static_assert(sizeof(VorNb) == 16, "Voronoi neighbour entry must be 16 bytes");
     constexpr int kVorPad = 12;  // entries every run has room for
     // entries a lane has in flight where L lanes share a path (400 000 sites, 2^18 packets, L = 1 with
-    // 6 / 8 / 10 / 12: 47.7 / 48.5 / 49.6 / 49.6 ms)
+    // 6 / 8 / 10 / 12: 40.8 / 39.6 / 40.1 / 43.0 ms)
     template<int L> constexpr int kVorAhead = L == 4 ? 5 : 8;
     constexpr int kVorSlack = 32;  // slots behind the last run that may be read (and are not used)
     // relative error allowed to the FP32 bounds: the offsets, the position and five operations are
@@ -1064,8 +1064,8 @@ namespace skg
         // sites), then by the latency of the run's lines, as the table does not fit the L2.  Hence
         // 16-byte entries and one dependent read per step: the entries name their neighbours' runs,
         // not their cells, and the exact exit distance takes the neighbour's site from the run that
-        // is read anyway.  400 000 sites, 2^18 packets, tau 5: 90 -> 48 ms; 1500 crossings in a row
-        // (2000 paths, 60 000 sites) with four lanes each: 1.3 -> 0.6 ms.
+        // is read anyway.  400 000 sites, 2^18 packets, tau 5: 90 -> 40 ms; 2000 optical
+        // depths through 60 000 sites with four lanes each: 0.47 -> 0.25 ms.
         static constexpr int kVorHinted = -1, kVorEnter = -2;  // i before the first step
         __device__ __forceinline__ int cross_voronoi(const GridView& g, int& m, double& ds, double& n)
         {
